@@ -695,6 +695,173 @@ __device__ __forceinline__ double wg_imtrace(int n, const double2* X, ldsd* red)
   return block_sum(s, red);
 }
 
+// --------------------------------------------------- Gauss-Jordan column steps
+// Maximum over the wave of an int, uniform result: DPP swaps within rows of 16 lanes,
+// then lane 15 of rows 0 / 2 into rows 1 / 3 and lane 31 into rows 2, 3; lane 63 holds
+// the maximum of all.
+__device__ __forceinline__ int wave_max_i32(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));  // row_mirror
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Row of the largest v >= 0 over the wave, the lowest row among equal values; -1 when
+// every v is negative or zero.  Each lane brings its own largest value and its row.
+// Non-negative doubles order like their bit patterns, so the high words decide unless
+// several lanes share the largest one (or it is zero), where the low words do.
+__device__ __forceinline__ int wave_pivot(double v, int row) {
+  const long long bits = __builtin_bit_cast(long long, v);
+  const int hi = (int)(bits >> 32);
+  const int mh = wave_max_i32(hi);
+  if (mh < 0) return -1;
+  unsigned long long hit = __ballot(hi == mh);
+  if (mh == 0 || __builtin_popcountll(hit) > 1) {
+    // unsigned order of the low words as signed ints
+    const int lo = (hi == mh) ? (int)((unsigned)bits ^ 0x80000000u) : (int)0x80000000;
+    const int ml = wave_max_i32(lo);
+    if (mh == 0 && ml == (int)0x80000000) return -1;
+    const bool top = hi == mh && lo == ml;
+    const int r = wave_max_i32(top ? -row : (int)0x80000000);
+    return -r;
+  }
+  return __builtin_amdgcn_readlane(row, __builtin_ctzll(hit));
+}
+
+// a row of registers read at a wave-uniform row index
+template <int R, int RT, int CT, typename F>
+__device__ __forceinline__ void with_row(double2 (&a)[RT][CT], int r, const F& f) {
+  if constexpr (R + 1 < RT) {
+    if (r != R) {
+      with_row<R + 1, RT, CT>(a, r, f);
+      return;
+    }
+  }
+  f(a[R]);
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) dvec2 ldsv;
+#else
+typedef dvec2 ldsv;
+#endif
+
+template <int RT, int HV>
+struct GjLds {
+  static constexpr int ROWS = (64 / HV) * RT;
+  static constexpr int DOUBLES = 2 * (2 * ROWS + 4);  // per parity: the column, its pivot, the pivot's row
+};
+
+// Gauss-Jordan sweep of 4 HV CT columns held in registers by 4 waves: lane l of wave w
+// holds rows (l mod 64/HV) + (64/HV) r, r < RT, of the CT columns of column block
+// cb = w HV + l / (64/HV).  Per column the wave that holds it chooses the pivot row (the
+// first maximum of |Re| + |Im| over the rows not yet used, as izamax in zgetrf), and
+// publishes the column through LDS with -1 in the pivot's place; after one barrier every
+// wave takes its own part of the pivot row from the lane that holds it (readlane, no
+// second exchange) and updates a_ij -= (a_ik / a_pk) a_pj.  The pivot row follows from
+// the -1 (a_pj = a_pj / a_pk) and column k from a one in the pivot row's place, so all
+// elements share one formula.  Column buffers alternate by column parity: a column's
+// reads are over before the barrier after which the next write to them starts.
+// A column step is a serial chain (pivot search, exchange, reciprocal, update), so its
+// length counts, not its operations; this split needs one barrier and no broadcast of
+// the pivot row.  Inverse of 256 blocks, one per CU, against one panel row per thread
+// (four candidate rows of 16 exchanged and scaled in every thread): n = 64 159 -> 83 us,
+// 96 300 -> 188, 128 449 -> 294, 192 966 -> 767, 256 1794 -> 1624 (there the passes over
+// W at HBM rate are the rest).
+// Returns 0 or the 1-based column without a nonzero pivot; piv[c] is the row of column c.
+template <int RT, int CT, int HV>
+__device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned& used, ldsi* piv, ldsd* xch) {
+  constexpr int RL = 64 / HV;
+  const int lane = threadIdx.x & 63, wave = uni((int)(threadIdx.x >> 6));
+  const int row = lane % RL, half = lane / RL;
+  for (int h = 0; h < 4 * HV; ++h) {  // column block
+#pragma unroll
+    for (int cc = 0; cc < CT; ++cc) {
+      ldsd* xc = xch + (cc & 1) * (GjLds<RT, HV>::DOUBLES / 2);
+      ldsv* col = (ldsv*)xc;
+      ldsv* pivot = (ldsv*)(xc + 2 * RL * RT);
+      ldsi* prow = (ldsi*)(xc + 2 * RL * RT + 2);
+      const bool holds = wave == h / HV;
+      const bool mine = holds && half == h % HV;
+      if (holds) {
+        double bv = -1.0;
+        int br = 0;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const double v = fabs(a[r][cc].x) + fabs(a[r][cc].y);
+          if (mine && row + RL * r < nrow && !((used >> r) & 1u) && v > bv) { bv = v; br = r; }
+        }
+        const int p = wave_pivot(bv, row + RL * br);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          dvec2 v;
+          const bool isp = row + RL * r == p;
+          v.x = a[r][cc].x;
+          v.y = a[r][cc].y;
+          if (mine && isp) *pivot = v;
+          v.x = isp ? -1.0 : v.x;
+          v.y = isp ? 0.0 : v.y;
+          if (mine) col[row + RL * r] = v;
+        }
+        if (lane == 0) {
+          *prow = p;
+          piv[h * CT + cc] = p;
+        }
+      }
+      __syncthreads();
+      const int p = uni((int)*prow);
+      if (p < 0) return h * CT + cc + 1;
+      const dvec2 pv = *pivot;
+      double2 f[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const dvec2 v = col[row + RL * r];
+        f[r] = make_double2(v.x, v.y);
+      }
+      // the pivot row's entries of this wave's columns; its registers restart from zero
+      const int pl = p % RL, pr = p / RL;
+      double2 rw[CT];
+      with_row<0, RT, CT>(a, pr, [&](double2 (&ar)[CT]) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          rw[c] = make_double2(lane_f64(ar[c].x, pl), lane_f64(ar[c].y, pl));
+          if constexpr (HV == 2) {
+            const double2 o = make_double2(lane_f64(ar[c].x, pl + RL), lane_f64(ar[c].y, pl + RL));
+            rw[c].x = half ? o.x : rw[c].x;
+            rw[c].y = half ? o.y : rw[c].y;
+          }
+          ar[c].x = row == pl ? 0.0 : ar[c].x;
+          ar[c].y = row == pl ? 0.0 : ar[c].y;
+        }
+        if (row == pl) used |= 1u << pr;
+      });
+      if (holds) {
+        rw[cc].x = mine ? 1.0 : rw[cc].x;
+        rw[cc].y = mine ? 0.0 : rw[cc].y;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          a[r][cc].x = mine ? 0.0 : a[r][cc].x;
+          a[r][cc].y = mine ? 0.0 : a[r][cc].y;
+        }
+      }
+      const double2 ainv = crecip(make_double2(pv.x, pv.y));
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const double2 g = cmul(f[r], ainv);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          a[r][c].x = fma(g.y, rw[c].y, fma(-g.x, rw[c].x, a[r][c].x));
+          a[r][c].y = fma(-g.y, rw[c].x, fma(-g.x, rw[c].y, a[r][c].y));
+        }
+      }
+    }
+  }
+  return 0;
+}
+
 // ------------------------------------------------------------------ inverse
 // In-place blocked Gauss-Jordan inverse with partial row pivoting (pivot =
 // first maximum of |Re|+|Im| among the rows not yet used, the izamax choice of
@@ -702,8 +869,8 @@ __device__ __forceinline__ double wg_imtrace(int n, const double2* X, ldsd* red)
 // the inverse is written column-major to out.  Returns 0, or k+1 when column k
 // has no nonzero pivot, in which case out is zeroed (src/green_rgf.f90:4429-4437).
 //
-// Panel step (16 columns K, pivot rows P): the panel is swept with one row per
-// thread in registers, giving F_P = A_PK^-1 and F_R = -A_RK A_PK^-1; the other
+// Panel step (16 or 32 columns K, pivot rows P): the panel is swept in registers
+// (gj_sweep), giving F_P = A_PK^-1 and F_R = -A_RK A_PK^-1; the other
 // columns J are updated by one MFMA GEMM W[:,J] += (F - E) W[P,J] with E the pivot
 // incidence (accumulating onto the loaded tiles of W), and columns K take F.
 // out (a separate n x n buffer) receives inv(i, q) = W[piv[i]][pinv[q]] after the
@@ -711,150 +878,69 @@ __device__ __forceinline__ double wg_imtrace(int n, const double2* X, ldsd* red)
 template <int T, int NMAX>
 struct InvSmallLds {
   static constexpr int LDI = NMAX + PAD;
-  static constexpr int DOUBLES = 4 * KP * LDI + 2 * NMAX + 16;
+  // columns per panel: 32 where the swept panel and the pivot rows fit in LDS (half the
+  // passes over W), else 16; 16 up to 64 rows, where two workgroups share a CU's LDS
+  static constexpr int KPI = NMAX > 64 && NMAX <= 128 ? 32 : 16;
+  static constexpr int DOUBLES = 4 * KPI * LDI + 2 * NMAX + 16;
 };
 
 template <int T, int NMAX>
 __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, ldsd* lds) {
   using C = Cfg<T>;
-  constexpr int LDI = NMAX + PAD;
+  constexpr int LDI = NMAX + PAD, KPI = InvSmallLds<T, NMAX>::KPI;
   constexpr int MR = C::MR, MC = C::MC, NTH = C::NTH, TA = C::TA, TB = C::TB;
+  constexpr int RT = (NMAX + 63) / 64, CT = KPI / 4;
   gd2* W = gw(W_);
   gd2* out = gw(out_);
   ldsd* Mr = lds;
-  ldsd* Mi = Mr + KP * LDI;
-  ldsd* Br = Mi + KP * LDI;
-  ldsd* Bi = Br + KP * LDI;
-  ldsi* piv = (ldsi*)(Bi + KP * LDI);
-  ldsi* used = piv + NMAX;
-  ldsd* redv = (ldsd*)(used + NMAX);
-  ldsi* redi = (ldsi*)(redv + 4);
+  ldsd* Mi = Mr + KPI * LDI;
+  ldsd* Br = Mi + KPI * LDI;
+  ldsd* Bi = Br + KPI * LDI;
+  ldsi* piv = (ldsi*)(Bi + KPI * LDI);
+  ldsi* pinv = piv + NMAX;
+  static_assert(NMAX <= NTH && NTH == 256, "four waves, one snapshot column per thread");
+  static_assert(GjLds<RT, 1>::DOUBLES <= KPI * LDI, "the column exchange fits the snapshot area");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int arow = (wave % C::WR) * 16 * TA, bcol = (wave / C::WR) * 16 * TB;
-  static_assert(NMAX <= NTH, "one panel row per thread");
-  for (int i = tid; i < n; i += NTH) used[i] = 0;
-  __syncthreads();
   int info = 0;
-  const bool own = tid < n;  // thread tid holds row tid of the current panel in registers
-  bool myused = false;
-  for (int k0 = 0; k0 < n && !info; k0 += KP) {
-    double2 rv[KP];
+  const bool own = tid < n;
+  unsigned used = 0;  // bit r: row lane + 64 r has been a pivot
+  for (int k0 = 0; k0 < n && !info; k0 += KPI) {
+    double2 a[RT][CT];
 #pragma unroll
-    for (int c2 = 0; c2 < KP; ++c2) rv[c2] = own ? W[(size_t)tid * n + k0 + c2] : make_double2(0, 0);
-    if (n <= 64) {
-      // all rows are in wave 0: the column steps run in that wave alone, the pivot
-      // row broadcast by readlane, no LDS exchange and no barrier per column
-      if (wave == 0) {
-        for (int c = 0; c < KP; ++c) {
-          double2 cand = make_double2(0, 0);
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-          for (int c2 = 0; c2 < KP; ++c2)
-            if (c2 == c) cand = rv[c2];
-          const bool valid = own && !myused;
-          const double myv = valid ? fabs(cand.x) + fabs(cand.y) : -1.0;
-          const double best = wave_max(myv);
-          if (!(best > 0.0)) { info = k0 + c + 1; break; }
-          const int p = uni(__builtin_ctzll(__ballot(valid && myv == best)));  // lowest row
-          double2 pr[KP];
-#pragma unroll
-          for (int c2 = 0; c2 < KP; ++c2) pr[c2] = make_double2(lane_f64(rv[c2].x, p), lane_f64(rv[c2].y, p));
-          double2 pc = pr[0];
-#pragma unroll
-          for (int c2 = 1; c2 < KP; ++c2)
-            if (c2 == c) pc = pr[c2];
-          const double2 ainv = crecip(pc);
-          double2 rp[KP];
-#pragma unroll
-          for (int c2 = 0; c2 < KP; ++c2) rp[c2] = (c2 == c) ? ainv : cmul(pr[c2], ainv);
-          if (tid == p) {
-            myused = true;
-            used[p] = 1;
-            piv[k0 + c] = p;
-#pragma unroll
-            for (int c2 = 0; c2 < KP; ++c2) rv[c2] = rp[c2];
-          } else if (own) {
-            const double2 f = cand;
-#pragma unroll
-            for (int c2 = 0; c2 < KP; ++c2) rv[c2] = csub((c2 == c) ? make_double2(0, 0) : rv[c2], cmul(f, rp[c2]));
-          }
-        }
-        if (tid == 0) redi[0] = info;
-      }
-      __syncthreads();
-      info = redi[0];
-    } else {
-      for (int c = 0; c < KP; ++c) {
-        // pivot: first maximum of |Re|+|Im| over unused rows (wave reduction, then one
-        // exchange of the 4 wave winners and their rows through LDS; Br/Bi hold the
-        // exchange area until the snapshot below, double-buffered by column parity)
-        double2 cand = make_double2(0, 0);
-  #pragma unroll
-        for (int c2 = 0; c2 < KP; ++c2)
-          if (c2 == c) cand = rv[c2];
-        const bool valid = own && !myused;
-        const double myv = valid ? fabs(cand.x) + fabs(cand.y) : -1.0;
-        double best = wave_max(myv);
-        const unsigned long long hit = __ballot(valid && myv == best);  // lowest lane = lowest row
-        int bi = hit ? wave * 64 + __builtin_ctzll(hit) : 0x7fffffff;
-        ldsd* xrow = Br + (c & 1) * (4 * 2 * KP);  // [wave][c2] re, im
-        ldsd* xval = Bi + (c & 1) * 8;               // [wave] value, [4 + wave] row index
-        if (tid == bi) {
-  #pragma unroll
-          for (int c2 = 0; c2 < KP; ++c2) {
-            xrow[wave * 2 * KP + 2 * c2] = rv[c2].x;
-            xrow[wave * 2 * KP + 2 * c2 + 1] = rv[c2].y;
-          }
-        }
-        if (lane == 0) { xval[wave] = best; xval[4 + wave] = (double)bi; }
-        __syncthreads();
-        best = xval[0];
-        bi = (int)xval[4];
-        for (int w = 1; w < NTH / 64; ++w) {
-          const double ov = xval[w];
-          const int oi = (int)xval[4 + w];
-          if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
-        }
-        if (!(best > 0.0)) { info = k0 + c + 1; break; }
-        const int p = bi;
-        const ldsd* prow = xrow + (p >> 6) * 2 * KP;
-        const double2 ainv = crecip(make_double2(prow[2 * c], prow[2 * c + 1]));
-        double2 rp[KP];
-  #pragma unroll
-        for (int c2 = 0; c2 < KP; ++c2)
-          rp[c2] = (c2 == c) ? ainv : cmul(make_double2(prow[2 * c2], prow[2 * c2 + 1]), ainv);
-        if (tid == p) {
-          myused = true;
-          used[p] = 1;
-          piv[k0 + c] = p;
-  #pragma unroll
-          for (int c2 = 0; c2 < KP; ++c2) rv[c2] = rp[c2];
-        } else if (own) {
-          const double2 f = cand;
-  #pragma unroll
-          for (int c2 = 0; c2 < KP; ++c2) rv[c2] = csub((c2 == c) ? make_double2(0, 0) : rv[c2], cmul(f, rp[c2]));
-        }
-      }
+      for (int c = 0; c < CT; ++c)
+        a[r][c] = lane + 64 * r < n ? W[(size_t)(lane + 64 * r) * n + k0 + wave * CT + c] : make_double2(0, 0);
+    // the exchange uses Br, free until the snapshot below
+    info = gj_sweep<RT, CT, 1>(a, n, used, piv + k0, Br);
+    if (info) {
+      info += k0;
+      break;
     }
-    if (!info && own) {
 #pragma unroll
-      for (int c2 = 0; c2 < KP; ++c2) { Mr[c2 * LDI + tid] = rv[c2].x; Mi[c2 * LDI + tid] = rv[c2].y; }
-    }
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        if (lane + 64 * r < n) {
+          Mr[(wave * CT + c) * LDI + lane + 64 * r] = a[r][c].x;
+          Mi[(wave * CT + c) * LDI + lane + 64 * r] = a[r][c].y;
+        }
     __syncthreads();
-    if (info) break;
     // snapshot of the pivot rows before they are updated: thread j copies column j
-    // of the KP rows, all its loads in flight at once
+    // of the KPI rows, all its loads in flight at once
     if (own) {
-      double2 v[KP];
+      double2 v[KPI];
 #pragma unroll
-      for (int c = 0; c < KP; ++c) v[c] = W[(size_t)piv[k0 + c] * n + tid];
+      for (int c = 0; c < KPI; ++c) v[c] = W[(size_t)piv[k0 + c] * n + tid];
 #pragma unroll
-      for (int c = 0; c < KP; ++c) {
+      for (int c = 0; c < KPI; ++c) {
         Br[c * LDI + tid] = v[c].x;
         Bi[c * LDI + tid] = v[c].y;
       }
     }
     __syncthreads();
-    if (tid < KP) Mr[tid * LDI + piv[k0 + tid]] -= 1.0;  // M = F - E
+    if (tid < KPI) Mr[tid * LDI + piv[k0 + tid]] -= 1.0;  // M = F - E
     __syncthreads();
     const int ntr = n / MR, ntc = n / MC;
     const int m = lane & 15, kq = lane >> 4;
@@ -875,7 +961,7 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
             cr[ti][tj][r] = o.x;
             ci[ti][tj][r] = o.y;
           }
-      mma_steps<TA, TB, 1, KP / 4>(cr, ci, Mr, Mi, LDI, row0 + arow, Br, Bi, LDI, col0 + bcol);
+      mma_steps<TA, TB, 1, KPI / 4>(cr, ci, Mr, Mi, LDI, row0 + arow, Br, Bi, LDI, col0 + bcol);
       const bool panel = col0 <= k0 && k0 < col0 + MC;  // the panel's columns take F
       if (!panel) {
 #pragma unroll
@@ -895,7 +981,7 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
             for (int r = 0; r < 4; ++r) {
               const int i = row0 + arow + ti * 16 + 4 * r + kq;
               const int j = col0 + bcol + tj * 16 + m;
-              const bool inp = j >= k0 && j < k0 + KP;
+              const bool inp = j >= k0 && j < k0 + KPI;
               const int c = inp ? j - k0 : 0;
               double2 f = make_double2(Mr[c * LDI + i], Mi[c * LDI + i]);
               f.x += (piv[k0 + c] == i) ? 1.0 : 0.0;
@@ -911,13 +997,12 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
     __syncthreads();
     return info;
   }
-  // inverse permutation into `used`
-  for (int q = tid; q < n; q += NTH) used[piv[q]] = q;
+  for (int q = tid; q < n; q += NTH) pinv[piv[q]] = q;  // inverse permutation
   __syncthreads();
-  // out(i, q) = W[piv[i]][used[q]], RB rows of out at a time: the source rows are
+  // out(i, q) = W[piv[i]][pinv[q]], RB rows of out at a time: the source rows are
   // read whole into LDS and out is written in column segments of RB elements
   constexpr int RB = 16;
-  static_assert(2 * RB * (NMAX + 1) <= 4 * KP * LDI, "row block fits the panel area");
+  static_assert(2 * RB * (NMAX + 1) <= 4 * KPI * LDI, "row block fits the panel area");
   const int ldr = n + 1;  // odd stride: the RB rows of one column sit in distinct banks
   ldsd* Lr = Mr;
   ldsd* Li = Mr + RB * ldr;
@@ -935,7 +1020,7 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
     __syncthreads();
     for (int idx = tid; idx < RB * n; idx += NTH) {
       const int rr = idx % RB, q = idx / RB;
-      const int c = used[q];
+      const int c = pinv[q];
       out[(size_t)(i0 + rr) + (size_t)q * n] = make_double2(Lr[rr * ldr + c], Li[rr * ldr + c]);
     }
     __syncthreads();
@@ -1194,24 +1279,17 @@ __device__ __noinline__ int wg_inverse_big(int n, double2* W_, double2* out_, ld
 }
 
 // ------------------------------------------------ inverse, n = 32 or 64
-// The whole matrix held in registers: thread t owns row i = t % N and the C = N*N / NTH
-// columns cb*C .. cb*C + C - 1, cb = t / N (16 columns at N = 64, 4 at N = 32).  The
-// same Gauss-Jordan sweep with the same pivot rule and logical row exchanges as the
-// blocked inverse, unblocked: per column k the threads holding column k (one wave at
-// N = 64, half a wave at N = 32) find the pivot row p and publish column k, the
-// threads of row p publish row p, and every thread updates its elements in registers.
-// Two barriers per column and no global memory between the load of W and the store
-// of the inverse, where the blocked inverse at these sizes spends most of its time
-// waiting on the loads and stores of each panel update.  Column and row exchange
-// buffers alternate by column parity, so a column's reads never meet the next
-// column's writes.
+// The whole matrix held in registers and swept by gj_sweep: at N = 64 lane l of wave w
+// holds row l of columns 16 w .. 16 w + 15, at N = 32 each half wave holds the 32 rows
+// of 4 columns.  No global memory between the load of W and the store of the inverse.
 template <int T, int N>
 struct InvRegLds {
+  static constexpr int HV = N == 32 ? 2 : 1;
   static constexpr int LDO = N + 1;           // odd row stride of the output staging tile
-  static constexpr int XCH = 2 * 4 * N;       // [parity][col re, col im, row re, row im][N]
+  static constexpr int XCH = GjLds<1, HV>::DOUBLES;
   static constexpr int OUT = 2 * N * LDO;     // re / im planes of the matrix for the final copy
   static constexpr int AREA = XCH > OUT ? XCH : OUT;
-  static constexpr int DOUBLES = AREA + N + 8;  // + piv, pinv (2 N ints) + pivot slots
+  static constexpr int DOUBLES = AREA + N + 8;  // + piv, pinv (2 N ints)
 };
 
 template <int T, int N>
@@ -1223,72 +1301,14 @@ __device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds
   gd2* out = gw(out_);
   ldsi* piv = (ldsi*)(lds + L::AREA);
   ldsi* pinv = piv + N;
-  ldsi* pvs = pinv + N;  // [parity] pivot row of the current column (-1: none)
   const int tid = threadIdx.x;
   const int i = tid % N, cb = tid / N;
-  double2 a[C];
+  double2 m[1][C];
+  double2(&a)[C] = m[0];
 #pragma unroll
   for (int c = 0; c < C; ++c) a[c] = W[(size_t)i * N + cb * C + c];
-  bool myused = false;
-  int info = 0;
-  const int wave = tid >> 6;
-  for (int k = 0; k < N; ++k) {
-    ldsd* X = lds + (k & 1) * (4 * N);
-    const int kb = k / C, kc = k % C;
-    const bool mine = (cb == kb);
-    // (a) the wave holding column k finds the pivot row and publishes the column
-    if (wave == (kb * N) / 64) {
-      double2 v = a[0];
-#pragma unroll
-      for (int c = 1; c < C; ++c)
-        if (c == kc) v = a[c];
-      const double m = (mine && !myused) ? fabs(v.x) + fabs(v.y) : -1.0;
-      const double best = wave_max(m);
-      const unsigned long long hit = __ballot(mine && !myused && m == best);
-      if (mine) {
-        X[i] = v.x;
-        X[N + i] = v.y;
-        if (i == 0) {
-          const int p = hit ? (int)(__builtin_ctzll(hit) % N) : -1;  // lowest row among equal maxima
-          pvs[k & 1] = (best > 0.0 && hit) ? p : -1;
-          piv[k] = p;
-        }
-      }
-    }
-    __syncthreads();
-    const int p = pvs[k & 1];
-    if (p < 0) {
-      info = k + 1;
-      break;
-    }
-    // (b) the threads of row p normalise their part of the pivot row and publish it
-    if (i == p) {
-      const double2 ainv = crecip(make_double2(X[p], X[N + p]));
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        const double2 r = (cb * C + c == k) ? ainv : cmul(a[c], ainv);
-        a[c] = r;
-        X[2 * N + cb * C + c] = r.x;
-        X[3 * N + cb * C + c] = r.y;
-      }
-      myused = true;
-    }
-    __syncthreads();
-    // (c) every other row: a -= a_ik * (pivot row), column k starting from zero
-    if (i != p) {
-      const double2 f = make_double2(X[i], X[N + i]);
-      double2 rp[C];
-#pragma unroll
-      for (int c = 0; c < C; ++c) rp[c] = make_double2(X[2 * N + cb * C + c], X[3 * N + cb * C + c]);
-      if (mine) {
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-          if (c == kc) a[c] = make_double2(0, 0);
-      }
-#pragma unroll
-      for (int c = 0; c < C; ++c) a[c] = csub(a[c], cmul(f, rp[c]));
-    }
-  }
+  unsigned used = 0;
+  const int info = gj_sweep<1, C, L::HV>(m, N, used, piv, lds);
   if (info) {
     for (int idx = tid; idx < N * N; idx += NTH) out[idx] = make_double2(0, 0);
     __syncthreads();

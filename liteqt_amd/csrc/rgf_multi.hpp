@@ -44,7 +44,7 @@ struct MultiLds {
 };
 
 __global__ __launch_bounds__(256, 1) void rgf_sweep_multi(MultiArgs m) {
-  __shared__ double lds[MultiLds::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[MultiLds::DOUBLES];
   __shared__ int next;
   static_assert(Cfg<1>::NTH == 256 && Cfg<2>::NTH == 256 && Cfg<3>::NTH == 256 && Cfg<4>::NTH == 256,
                 "all variants run 256 threads");

@@ -427,7 +427,7 @@ struct SweepLds {
 
 template <int T, int NMAX>
 __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void rgf_sweep(SweepArgs a) {
-  __shared__ double lds[SweepLds<T, NMAX>::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[SweepLds<T, NMAX>::DOUBLES];
   double2* ws = a.ws + (size_t)blockIdx.x * (size_t)a.ws_slot;
   for (int e = blockIdx.x; e < a.nE; e += gridDim.x) solve_energy<T, NMAX>(a, e, ws, (ldsd*)lds, (ldsd*)lds);
 }
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void rgf_sweep(SweepArgs 
 // green_RGF_CMS: the same persistent loop with the overlap variant of the solve.
 template <int T, int NMAX>
 __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void rgf_sweep_cms(SweepArgs a) {
-  __shared__ double lds[SweepLds<T, NMAX>::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[SweepLds<T, NMAX>::DOUBLES];
   double2* ws = a.ws + (size_t)blockIdx.x * (size_t)a.ws_slot;
   for (int e = blockIdx.x; e < a.nE; e += gridDim.x)
     solve_energy<T, NMAX, true>(a, e, ws, (ldsd*)lds, (ldsd*)lds);
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void rgf_sweep_cms(SweepA
 template <int T>
 __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void k_gemm_batched(int n, int nb, int opA, const double2* A, int opB,
                                                         const double2* B, double2* C, int c_rowmajor) {
-  __shared__ double lds[GemmLds<T>::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[GemmLds<T>::DOUBLES];
   const size_t nn = (size_t)n * n;
   for (int b = blockIdx.x; b < nb; b += gridDim.x)
     wg_gemm<T>(n, opA, A + b * nn, opB, B + b * nn, C + b * nn, c_rowmajor, epi_store(), (ldsd*)lds);
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void k_gemm_batched(int n
 template <int T, int NMAX>
 __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void k_inv_batched(int n, int nb, const double2* A, double2* Ainv, double2* W,
                                                        int* info) {
-  __shared__ double lds[SweepLds<T, NMAX>::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[SweepLds<T, NMAX>::DOUBLES];
   const size_t nn = (size_t)n * n;
   const double2 one = make_double2(1, 0), zero = make_double2(0, 0);
   for (int b = blockIdx.x; b < nb; b += gridDim.x) {

@@ -135,7 +135,7 @@ __device__ void w_energy(const WArgs& a, int e, double2* ws, ldsd* lds) {
 
 template <int T, int NMAX>
 __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void rgf_wsweep(WArgs a) {
-  __shared__ double lds[SweepLds<T, NMAX>::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[SweepLds<T, NMAX>::DOUBLES];
   double2* ws = a.ws + (size_t)blockIdx.x * (size_t)a.ws_slot;
   for (int e = blockIdx.x; e < a.nE; e += gridDim.x) w_energy<T, NMAX>(a, e, ws, (ldsd*)lds);
 }
