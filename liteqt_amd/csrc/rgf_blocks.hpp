@@ -83,6 +83,12 @@ __device__ __forceinline__ void stgb(double2* base, uint32_t boff, double2 v) {
 }
 __device__ __forceinline__ void stgb_re(double* base, uint32_t boff, double v) { *(gd*)((gwb*)base + boff) = v; }
 
+// A block dimension of type int is a lone workgroup's: it has every tile, and its
+// operations end with the workgroup barrier (rgf_group.hpp has the other kind).
+__device__ __forceinline__ int group_rank(int) { return 0; }
+__device__ __forceinline__ int group_size(int) { return 1; }
+__device__ __forceinline__ void group_sync(int) { __syncthreads(); }
+
 // Uniform values arrive in VGPRs through the calling convention of a
 // non-inlined function; moving them to SGPRs frees those VGPRs.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -116,6 +122,25 @@ __device__ __forceinline__ double2 crecip(double2 b) {
     double t = b.x / b.y, d = b.x * t + b.y;
     return make_double2(t / d, -1.0 / d);
   }
+}
+
+// 1/b for a wave-uniform b: where |b| is far from the ends of the exponent range (high
+// words of the components below 2^500, the larger above 2^-500) b* / |b|^2 with the
+// hardware's reciprocal refined by two Newton steps, 8 dependent operations against the
+// two divisions in a row of the general form; else the general form.
+__device__ __forceinline__ double2 crecip_uniform(double2 b) {
+  const unsigned hx = (unsigned)(__builtin_bit_cast(unsigned long long, b.x) >> 32) & 0x7fffffffu;
+  const unsigned hy = (unsigned)(__builtin_bit_cast(unsigned long long, b.y) >> 32) & 0x7fffffffu;
+  const unsigned h = uni((int)(hx > hy ? hx : hy));
+  constexpr unsigned lo = (1023u - 500u) << 20, hi = (1023u + 500u) << 20;
+  if (h >= lo && h < hi) {
+    const double d = fma(b.x, b.x, b.y * b.y);
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.0), r);
+    r = fma(r, fma(-d, r, 1.0), r);
+    return make_double2(b.x * r, -b.y * r);
+  }
+  return crecip(b);
 }
 
 // out(i,j) = sacc*acc(i,j) + diag*[i==j] + s1*D1(i,j) + s2*D2(i,j) + s3*conj(D3(j,i))
@@ -254,8 +279,8 @@ struct Cfg {
 // complex tiles.  A values at Ar/Ai[k*lda + arow + m], B at Br/Bi[k*ldb + bcol + m].
 // ROWMAJ=0: lane holds C[arow + ti*16 + l%16][bcol + tj*16 + 4r + l/16];
 // ROWMAJ=1: lane holds C[arow + ti*16 + 4r + l/16][bcol + tj*16 + l%16].
-// AKC / BKC: the panel is stored k-contiguous (A at Ar[(arow + m) * LDK + k], B at
-// Br[(bcol + m) * LDK + k]) instead of row-contiguous (A at Ar[k * lda + arow + m]).
+// AKC / BKC: the panel is stored k-contiguous (A at Ar[(arow + m) * lda + k], B at
+// Br[(bcol + m) * ldb + k]) instead of row-contiguous (A at Ar[k * lda + arow + m]).
 struct NoMid {
   __device__ void operator()(int) const {}
 };
@@ -277,13 +302,13 @@ __device__ __forceinline__ void mma_steps(d4 (&cr)[TA][TB], d4 (&ci)[TA][TB],
     const int k = ks * 4 + kq;
 #pragma unroll
     for (int t = 0; t < TA; ++t) {
-      const int ia = AKC ? (arow + t * 16 + m) * LDK + k : k * lda + arow + t * 16 + m;
+      const int ia = AKC ? (arow + t * 16 + m) * lda + k : k * lda + arow + t * 16 + m;
       ar[s][t] = Ar[ia];
       ai[s][t] = Ai[ia];
     }
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
-      const int ib = BKC ? (bcol + t * 16 + m) * LDK + k : k * ldb + bcol + t * 16 + m;
+      const int ib = BKC ? (bcol + t * 16 + m) * ldb + k : k * ldb + bcol + t * 16 + m;
       br[s][t] = Br[ib];
       bi[s][t] = Bi[ib];
     }
@@ -427,9 +452,10 @@ struct EpiMode {
   static constexpr int value = M;
 };
 
+// The output tiles rank, rank + size, ...; returns this thread's part of sum |C_ij|.
 template <int T, int OPA, int OPB, int CRM>
-__device__ __noinline__ double wg_gemm_k(int n_, const double2* __restrict__ A_, const double2* __restrict__ B_,
-                                         void* Cout_, Epi ep_, ldsd* lds) {
+__device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__ A_, const double2* __restrict__ B_,
+                                             void* Cout_, Epi ep_, ldsd* lds, int rank, int size) {
   using C = Cfg<T>;
   constexpr int MR = C::MR, MC = C::MC, LDA = C::LDA, LDB = C::LDB, STAGE = C::STAGE, TA = C::TA, TB = C::TB;
   constexpr bool AKC = (OPA != OP_N), BKC = (OPB == OP_N);
@@ -444,8 +470,6 @@ __device__ __noinline__ double wg_gemm_k(int n_, const double2* __restrict__ A_,
   ep.D3 = uni(ep_.D3); ep.s3 = uni(ep_.s3);
   ep.real_out = uni(ep_.real_out); ep.abs_sum = uni(ep_.abs_sum);
   const int emode = (ep.D2 || ep.D3 || ep.real_out || ep.abs_sum) ? 2 : (ep.D1 ? 1 : 0);
-  // the abs-sum reduction runs after the last panel's barrier, when stage 0 is free
-  ldsd* red = lds;
   const ldsd* s0Ar = lds;
   const ldsd* s0Ai = s0Ar + KP * LDA;
   const ldsd* s0Br = s0Ai + KP * LDA;
@@ -469,13 +493,14 @@ __device__ __noinline__ double wg_gemm_k(int n_, const double2* __restrict__ A_,
   const uint32_t t_cm = (uint32_t)(it + jt * n), t_tr = (uint32_t)(jt + it * n);
   const uint32_t t_out = CRM ? t_tr : t_cm;
   double asum = 0.0;
+  if (rank >= ntiles) return 0.0;
   double2 ra[C::PERA], rb[C::PERB];
-  gemm_load_panel<T, OPA, OPB>(a_org(0, 0), b_org(0, 0), oa, ob, ra, rb);
+  gemm_load_panel<T, OPA, OPB>(a_org((rank % ntr) * MR, 0), b_org((rank / ntr) * MC, 0), oa, ob, ra, rb);
   gemm_store_panel<T, OPA, OPB>(lds, ra, rb);
   __syncthreads();
-  for (int tile = 0; tile < ntiles; ++tile) {
+  for (int tile = rank; tile < ntiles; tile += size) {
     const int row0 = (tile % ntr) * MR, col0 = (tile / ntr) * MC;
-    const int tn = tile + 1 < ntiles ? tile + 1 : tile;  // the last tile refetches its own panel 0
+    const int tn = tile + size < ntiles ? tile + size : tile;  // the last tile refetches its own panel 0
     const int nrow0 = (tn % ntr) * MR, ncol0 = (tn / ntr) * MC;
     d4 cr[TA][TB], ci[TA][TB];
 #pragma unroll
@@ -485,15 +510,15 @@ __device__ __noinline__ double wg_gemm_k(int n_, const double2* __restrict__ A_,
     for (int p = 0; p < npan; p += 2) {
       // stage 0 holds panel p; panel p + 1 goes to stage 1
       gemm_load_panel<T, OPA, OPB>(a_org(row0, (p + 1) * KP), b_org(col0, (p + 1) * KP), oa, ob, ra, rb);
-      mma_steps<TA, TB, CRM, KP / 4, AKC, BKC>(cr, ci, s0Ar, s0Ai, LDA, arow, s0Br, s0Bi, LDB, bcol,
+      mma_steps<TA, TB, CRM, KP / 4, AKC, BKC>(cr, ci, s0Ar, s0Ai, AKC ? LDK : LDA, arow, s0Br, s0Bi, BKC ? LDK : LDB, bcol,
                                               [&](int g) { gemm_store_panel<T, OPA, OPB>(lds + STAGE, ra, rb, g); });
       __syncthreads();
       // stage 1 holds panel p + 1; panel p + 2 (or panel 0 of the next tile) goes to stage 0
       const bool last = p + 2 == npan;
       gemm_load_panel<T, OPA, OPB>(last ? a_org(nrow0, 0) : a_org(row0, (p + 2) * KP),
                                    last ? b_org(ncol0, 0) : b_org(col0, (p + 2) * KP), oa, ob, ra, rb);
-      mma_steps<TA, TB, CRM, KP / 4, AKC, BKC>(cr, ci, s0Ar + STAGE, s0Ai + STAGE, LDA, arow, s0Br + STAGE,
-                                              s0Bi + STAGE, LDB, bcol,
+      mma_steps<TA, TB, CRM, KP / 4, AKC, BKC>(cr, ci, s0Ar + STAGE, s0Ai + STAGE, AKC ? LDK : LDA, arow, s0Br + STAGE,
+                                              s0Bi + STAGE, BKC ? LDK : LDB, bcol,
                                               [&](int g) { gemm_store_panel<T, OPA, OPB>(lds, ra, rb, g); });
       __syncthreads();
     }
@@ -561,8 +586,16 @@ __device__ __noinline__ double wg_gemm_k(int n_, const double2* __restrict__ A_,
     else
       epilogue(EpiMode<2>());
   }
+  return asum;
+}
+
+template <int T, int OPA, int OPB, int CRM>
+__device__ __noinline__ double wg_gemm_k(int n, const double2* __restrict__ A, const double2* __restrict__ B, void* Cout,
+                                         Epi ep, ldsd* lds) {
+  const double asum = gemm_tiles<T, OPA, OPB, CRM>(n, A, B, Cout, ep, lds, 0, 1);
   double s = 0.0;
-  if (ep.abs_sum) s = block_sum(asum, red);
+  // stage 0 is free after the last panel's barrier
+  if (uni(ep.abs_sum)) s = block_sum(asum, lds);
   __syncthreads();
   return s;
 }
@@ -611,7 +644,8 @@ __device__ __noinline__ void wg_ew(int n, double2* out, int out_rowmajor, double
 // next pair's elements are loaded into registers while the current pair is combined.
 // LDS: kAntihermLds doubles; 256 threads.
 constexpr int kAntihermLds = 4 * 32 * 33;
-__device__ __noinline__ void wg_antiherm(int n, const double2* X_, double2* out_, ldsd* lds) {
+// Pairs q = rank, rank + size, ...
+__device__ __noinline__ void antiherm_pairs(int n, const double2* X_, double2* out_, ldsd* lds, int rank, int size) {
   constexpr int TS = 32, LD = TS + 1, PER = TS * TS / 256;
   static_assert(4 * TS * LD == kAntihermLds, "LDS size");
   const gcd2* X = gc(X_);
@@ -639,8 +673,8 @@ __device__ __noinline__ void wg_antiherm(int n, const double2* X_, double2* out_
       rb[k] = X[(size_t)(J * TS + r) + (size_t)(I * TS + c) * n];
     }
   };
-  load(0);
-  for (int q = 0; q < npair; ++q) {
+  if (rank < npair) load(rank);
+  for (int q = rank; q < npair; q += size) {
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int c = c0 + 8 * k;
@@ -648,7 +682,7 @@ __device__ __noinline__ void wg_antiherm(int n, const double2* X_, double2* out_
       Br[c * LD + r] = rb[k].x; Bi[c * LD + r] = rb[k].y;
     }
     __syncthreads();
-    if (q + 1 < npair) load(q + 1);
+    if (q + size < npair) load(q + size);
     int I, J;
     pair_of(q, I, J);
 #pragma unroll
@@ -663,6 +697,9 @@ __device__ __noinline__ void wg_antiherm(int n, const double2* X_, double2* out_
     }
     __syncthreads();
   }
+}
+__device__ __forceinline__ void wg_antiherm(int n, const double2* X, double2* out, ldsd* lds) {
+  antiherm_pairs(n, X, out, lds, 0, 1);
 }
 
 // Y = i Im X (real parts zeroed); Z = X as well when Z is given.  Y, Z must not alias X.
@@ -700,12 +737,14 @@ __device__ __forceinline__ double wg_imtrace(int n, const double2* X, ldsd* red)
 // then lane 15 of rows 0 / 2 into rows 1 / 3 and lane 31 into rows 2, 3; lane 63 holds
 // the maximum of all.
 __device__ __forceinline__ int wave_max_i32(int v) {
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));  // row_mirror
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
+  // (old values chosen so that each exchange folds into its maximum)
+  constexpr int lowest = (int)0x80000000;
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true));  // row_half_mirror
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true));  // row_mirror
+  v = max(v, __builtin_amdgcn_update_dpp(lowest, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
+  v = max(v, __builtin_amdgcn_update_dpp(lowest, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
   return __builtin_amdgcn_readlane(v, 63);
 }
 
@@ -731,16 +770,23 @@ __device__ __forceinline__ int wave_pivot(double v, int row) {
   return __builtin_amdgcn_readlane(row, __builtin_ctzll(hit));
 }
 
-// a row of registers read at a wave-uniform row index
-template <int R, int RT, int CT, typename F>
-__device__ __forceinline__ void with_row(double2 (&a)[RT][CT], int r, const F& f) {
-  if constexpr (R + 1 < RT) {
-    if (r != R) {
-      with_row<R + 1, RT, CT>(a, r, f);
-      return;
-    }
+// f(Index<i>()) for a wave-uniform i in [LO, HI): the registers that f reads keep static
+// indexes, one of log2 uniform branches is taken at each level.
+template <int I>
+struct Index {
+  static constexpr int value = I;
+};
+template <int LO, int HI, typename F>
+__device__ __forceinline__ void at_index(int i, const F& f) {
+  if constexpr (HI - LO == 1) {
+    f(Index<LO>());
+  } else {
+    constexpr int MID = (LO + HI) / 2;
+    if (i < MID)
+      at_index<LO, MID>(i, f);
+    else
+      at_index<MID, HI>(i, f);
   }
-  f(a[R]);
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -749,44 +795,56 @@ typedef __attribute__((address_space(3))) dvec2 ldsv;
 typedef dvec2 ldsv;
 #endif
 
-template <int RT, int HV>
+template <int RT, int CT, int HV>
 struct GjLds {
   static constexpr int ROWS = (64 / HV) * RT;
-  static constexpr int DOUBLES = 2 * (2 * ROWS + 4);  // per parity: the column, its pivot, the pivot's row
+  static constexpr int COL = 2 * ROWS + 4;            // the column, its pivot, the pivot's row
+  static constexpr int ROW = HV == 2 ? 2 * CT * HV : 0;  // a wave's part of the pivot row
+  static constexpr int DOUBLES = 2 * COL + 4 * ROW;   // columns by parity, rows by wave
 };
 
 // Gauss-Jordan sweep of 4 HV CT columns held in registers by 4 waves: lane l of wave w
 // holds rows (l mod 64/HV) + (64/HV) r, r < RT, of the CT columns of column block
-// cb = w HV + l / (64/HV).  Per column the wave that holds it chooses the pivot row (the
-// first maximum of |Re| + |Im| over the rows not yet used, as izamax in zgetrf), and
-// publishes the column through LDS with -1 in the pivot's place; after one barrier every
-// wave takes its own part of the pivot row from the lane that holds it (readlane, no
-// second exchange) and updates a_ij -= (a_ik / a_pk) a_pj.  The pivot row follows from
-// the -1 (a_pj = a_pj / a_pk) and column k from a one in the pivot row's place, so all
-// elements share one formula.  Column buffers alternate by column parity: a column's
+// cb = w HV + l / (64/HV).  Per column k the wave that holds it chooses the pivot row p
+// (the first maximum of |Re| + |Im| over the rows not yet used, as izamax in zgetrf) and
+// publishes the column through LDS with a zero in the pivot's place, then restarts its
+// registers of the column from the unit vector of p; after one barrier every wave takes
+// its own part of row p from the lane that holds it (readlane, no second exchange) and
+// updates a_ij -= (a_ik / a_pk) a_pj.  Row p itself is left as it is (its factor is the
+// published zero) and scaled by 1 / a_pk after the last column, which commutes with the
+// later updates of the row.  Only the holding wave's part depends on the column's
+// register, so the code of a step is short (the fully unrolled sweep of a 256 x 32 panel
+// was 130 KB and ran from L2).  Column buffers alternate by column parity: a column's
 // reads are over before the barrier after which the next write to them starts.
 // A column step is a serial chain (pivot search, exchange, reciprocal, update), so its
 // length counts, not its operations; this split needs one barrier and no broadcast of
 // the pivot row.  Inverse of 256 blocks, one per CU, against one panel row per thread
-// (four candidate rows of 16 exchanged and scaled in every thread): n = 64 159 -> 83 us,
-// 96 300 -> 188, 128 449 -> 294, 192 966 -> 767, 256 1794 -> 1624 (there the passes over
-// W at HBM rate are the rest).
+// (four candidate rows of 16 exchanged and scaled in every thread): n = 32 35 -> 27 us,
+// 64 159 -> 77, 96 300 -> 185, 128 449 -> 298.
 // Returns 0 or the 1-based column without a nonzero pivot; piv[c] is the row of column c.
 template <int RT, int CT, int HV>
 __device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned& used, ldsi* piv, ldsd* xch) {
   constexpr int RL = 64 / HV;
+  static_assert(HV == 1 || RT == 1, "half waves hold one row per lane");
   const int lane = threadIdx.x & 63, wave = uni((int)(threadIdx.x >> 6));
   const int row = lane % RL, half = lane / RL;
-  for (int h = 0; h < 4 * HV; ++h) {  // column block
+  double2 sc[RT];       // 1 / pivot of a row that has been one in this sweep
+  unsigned here = 0;    // bit r: it has
+  int fail = 0;
+  ldsv* prow_mine = (ldsv*)(xch + 2 * GjLds<RT, CT, HV>::COL) + (wave * HV + half) * CT;
 #pragma unroll
-    for (int cc = 0; cc < CT; ++cc) {
-      ldsd* xc = xch + (cc & 1) * (GjLds<RT, HV>::DOUBLES / 2);
-      ldsv* col = (ldsv*)xc;
-      ldsv* pivot = (ldsv*)(xc + 2 * RL * RT);
-      ldsi* prow = (ldsi*)(xc + 2 * RL * RT + 2);
-      const bool holds = wave == h / HV;
-      const bool mine = holds && half == h % HV;
-      if (holds) {
+  for (int r = 0; r < RT; ++r) sc[r] = make_double2(1, 0);
+#pragma unroll 1
+  for (int k = 0; k < 4 * HV * CT; ++k) {
+    ldsd* xc = xch + (k & 1) * (GjLds<RT, CT, HV>::COL);
+    ldsv* col = (ldsv*)xc;
+    ldsv* pivot = (ldsv*)(xc + 2 * RL * RT);
+    ldsi* prow = (ldsi*)(xc + 2 * RL * RT + 2);
+    const int h = k / CT;  // column block
+    if (wave == h / HV) {
+      const bool mine = half == h % HV;
+      at_index<0, CT>(k % CT, [&](auto ix) {
+        constexpr int cc = decltype(ix)::value;
         double bv = -1.0;
         int br = 0;
 #pragma unroll
@@ -797,69 +855,92 @@ __device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned
         const int p = wave_pivot(bv, row + RL * br);
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-          dvec2 v;
           const bool isp = row + RL * r == p;
+          dvec2 v;
           v.x = a[r][cc].x;
           v.y = a[r][cc].y;
-          if (mine && isp) *pivot = v;
-          v.x = isp ? -1.0 : v.x;
-          v.y = isp ? 0.0 : v.y;
-          if (mine) col[row + RL * r] = v;
+          if (mine) {
+            if (isp) *pivot = v;
+            v.x = isp ? 0.0 : v.x;
+            v.y = isp ? 0.0 : v.y;
+            col[row + RL * r] = v;
+            a[r][cc].x = isp ? 1.0 : 0.0;
+            a[r][cc].y = 0.0;
+          }
         }
         if (lane == 0) {
           *prow = p;
-          piv[h * CT + cc] = p;
+          piv[k] = p < 0 ? 0 : p;
         }
-      }
-      __syncthreads();
-      const int p = uni((int)*prow);
-      if (p < 0) return h * CT + cc + 1;
-      const dvec2 pv = *pivot;
-      double2 f[RT];
-#pragma unroll
-      for (int r = 0; r < RT; ++r) {
-        const dvec2 v = col[row + RL * r];
-        f[r] = make_double2(v.x, v.y);
-      }
-      // the pivot row's entries of this wave's columns; its registers restart from zero
-      const int pl = p % RL, pr = p / RL;
-      double2 rw[CT];
-      with_row<0, RT, CT>(a, pr, [&](double2 (&ar)[CT]) {
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          rw[c] = make_double2(lane_f64(ar[c].x, pl), lane_f64(ar[c].y, pl));
-          if constexpr (HV == 2) {
-            const double2 o = make_double2(lane_f64(ar[c].x, pl + RL), lane_f64(ar[c].y, pl + RL));
-            rw[c].x = half ? o.x : rw[c].x;
-            rw[c].y = half ? o.y : rw[c].y;
-          }
-          ar[c].x = row == pl ? 0.0 : ar[c].x;
-          ar[c].y = row == pl ? 0.0 : ar[c].y;
-        }
-        if (row == pl) used |= 1u << pr;
       });
-      if (holds) {
-        rw[cc].x = mine ? 1.0 : rw[cc].x;
-        rw[cc].y = mine ? 0.0 : rw[cc].y;
+    }
+    __syncthreads();
+    const int p0 = *prow;
+    const dvec2 pv = *pivot;
+    double2 g[RT];
 #pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          a[r][cc].x = mine ? 0.0 : a[r][cc].x;
-          a[r][cc].y = mine ? 0.0 : a[r][cc].y;
-        }
-      }
-      const double2 ainv = crecip(make_double2(pv.x, pv.y));
-#pragma unroll
-      for (int r = 0; r < RT; ++r) {
-        const double2 g = cmul(f[r], ainv);
+    for (int r = 0; r < RT; ++r) {
+      const dvec2 v = col[row + RL * r];
+      g[r] = make_double2(v.x, v.y);
+    }
+    // a column without a pivot is noted and the sweep runs on (its results are not used):
+    // a branch here would put the reads above behind the row's
+    const int pu = uni(p0);
+    if (pu < 0 && !fail) fail = k + 1;
+    const int p = pu < 0 ? 0 : pu;
+    // row p's entries of this wave's columns
+    const int pl = p % RL;
+    double2 rw[CT];
+    if constexpr (HV == 2) {
+      // through LDS (a wave's LDS operations are in order, so without a barrier): the
+      // half waves read different columns
+      if (row == pl) {
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-          a[r][c].x = fma(g.y, rw[c].y, fma(-g.x, rw[c].x, a[r][c].x));
-          a[r][c].y = fma(-g.y, rw[c].x, fma(-g.x, rw[c].y, a[r][c].y));
+          dvec2 v;
+          v.x = a[0][c].x;
+          v.y = a[0][c].y;
+          prow_mine[c] = v;
         }
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        const dvec2 v = prow_mine[c];
+        rw[c] = make_double2(v.x, v.y);
+      }
+    } else {
+      // (through LDS one lane's 16 writes alone take longer than 64 readlanes)
+      at_index<0, RT>(p / RL, [&](auto ix) {
+        constexpr int pr = decltype(ix)::value;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) rw[c] = make_double2(lane_f64(a[pr][c].x, pl), lane_f64(a[pr][c].y, pl));
+      });
+    }
+    const double2 ainv = crecip_uniform(make_double2(pv.x, pv.y));
+    const unsigned bit = row == pl ? 1u << (p / RL) : 0u;
+    used |= bit;
+    here |= bit;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      sc[r].x = row + RL * r == p ? ainv.x : sc[r].x;
+      sc[r].y = row + RL * r == p ? ainv.y : sc[r].y;
+      g[r] = cmul(g[r], ainv);
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        a[r][c].x = fma(g[r].y, rw[c].y, fma(-g[r].x, rw[c].x, a[r][c].x));
+        a[r][c].y = fma(-g[r].y, rw[c].x, fma(-g[r].x, rw[c].y, a[r][c].y));
       }
     }
   }
-  return 0;
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    if ((here >> r) & 1u) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) a[r][c] = cmul(a[r][c], sc[r]);
+    }
+  }
+  return fail;
 }
 
 // ------------------------------------------------------------------ inverse
@@ -899,7 +980,7 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
   ldsi* piv = (ldsi*)(Bi + KPI * LDI);
   ldsi* pinv = piv + NMAX;
   static_assert(NMAX <= NTH && NTH == 256, "four waves, one snapshot column per thread");
-  static_assert(GjLds<RT, 1>::DOUBLES <= KPI * LDI, "the column exchange fits the snapshot area");
+  static_assert(GjLds<RT, CT, 1>::DOUBLES <= KPI * LDI, "the column exchange fits the snapshot area");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int arow = (wave % C::WR) * 16 * TA, bcol = (wave / C::WR) * 16 * TB;
   int info = 0;
@@ -1026,6 +1107,204 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
     __syncthreads();
   }
   return 0;
+}
+
+// -------------------------------------------- inverse, 128 < n <= 256
+// The blocked sweep with 32-column panels.  At these sizes the panel updates read and
+// write the whole of W from HBM (256 workgroups hold 256 MB), so the number of passes
+// counts: 32 columns halve those of a 16-column panel.  The swept panel M = F - E (32 x n)
+// fills the LDS; W is updated in strips of 16 columns, each with its part of the pivot
+// rows staged beside M, and the next strip is loaded while the current one is multiplied
+// (without that overlap the 32-column panels are slower: 1844 us, below).
+// Rows of M alternate by 16 doubles (row k's index is xored with 16 (k & 1)) in place of a
+// padded stride, which LDS has no room for: the four k of a fragment read then fall on
+// distinct banks as with a stride of 16 mod 32.
+// Strips belong to the ranks of a group in turn (a lone workgroup has all); every rank
+// sweeps the panel for itself.  A panel's own columns take F one step late, after the
+// ranks have all read the panel.  256 blocks, one per CU, 16-column panels -> this: n = 160
+// 587 -> 553 us, 192 767 -> 776, 224 1287 -> 1159, 256 1624 -> 1527.
+template <int NMAX>
+struct InvStripLds {
+  static constexpr int KPI = 32, SC = 16;
+  static constexpr int S1 = 2 * KPI * SC;  // re / im planes of a strip's pivot rows, two buffers
+  static constexpr int OFF_S = 2 * KPI * NMAX, OFF_PIV = OFF_S + 2 * S1;
+  static constexpr int DOUBLES = OFF_PIV + NMAX;  // + piv, pinv (2 NMAX ints)
+};
+
+template <int NMAX, typename N>
+__device__ __noinline__ int wg_inverse_strip(N n_, double2* W_, double2* out_, ldsd* lds) {
+  using L = InvStripLds<NMAX>;
+  constexpr int KPI = L::KPI, SC = L::SC, NTH = 256;
+  constexpr int RT = NMAX / 64, CT = KPI / 4, PS = KPI * SC / NTH;
+  static_assert(NMAX % 64 == 0 && NMAX <= NTH, "four waves of row tiles");
+  static_assert(GjLds<RT, CT, 1>::DOUBLES <= 2 * L::S1, "the column exchange fits the pivot-row area");
+  const int n = uni((int)n_), rank = uni(group_rank(n_)), size = uni(group_size(n_));
+  double2* Wp = uni(W_);
+  gd2* out = gw(uni(out_));
+  ldsd* Mr = lds;
+  ldsd* Mi = lds + KPI * NMAX;
+  ldsd* S = lds + L::OFF_S;
+  ldsi* piv = (ldsi*)(lds + L::OFF_PIV);
+  ldsi* pinv = piv + NMAX;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  const int m = lane & 15, kq = lane >> 4;
+  auto mix = [&](int k, int i) { return k * NMAX + (i ^ ((k & 1) << 4)); };
+  // columns k0.. of W take F = M + E
+  auto late = [&](int k0) {
+    if ((k0 / SC + (wave >> 1)) % size != rank) return;  // waves 0, 1 hold the first strip
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int i = lane + 64 * r;
+      if (i < n) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          const int k = wave * CT + c;
+          double2 f = make_double2(Mr[mix(k, i)], Mi[mix(k, i)]);
+          f.x += piv[k0 + k] == i ? 1.0 : 0.0;
+          stgb(Wp + k0 + k, 16u * (uint32_t)(i * n), f);
+        }
+      }
+    }
+  };
+  int info = 0;
+  unsigned used = 0;  // bit r: row lane + 64 r has been a pivot
+  for (int k0 = 0; k0 < n; k0 += KPI) {
+    double2 a[RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        a[r][c] = lane + 64 * r < n ? ldgb(Wp + k0 + wave * CT + c, 16u * (uint32_t)((lane + 64 * r) * n)) : make_double2(0, 0);
+    if (k0) late(k0 - KPI);
+    info = gj_sweep<RT, CT, 1>(a, n, used, piv + k0, S);
+    if (info) {
+      info += k0;
+      break;
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        if (lane + 64 * r < n) {
+          Mr[mix(wave * CT + c, lane + 64 * r)] = a[r][c].x;
+          Mi[mix(wave * CT + c, lane + 64 * r)] = a[r][c].y;
+        }
+    __syncthreads();
+    if (tid < KPI) Mr[mix(tid, piv[k0 + tid])] -= 1.0;  // M = F - E
+    // the rank's strips but the panel's own; -1: none left
+    auto next = [&](int s) {
+      while (s < n / SC && s / (KPI / SC) == k0 / KPI) s += size;
+      return s < n / SC ? s : -1;
+    };
+    double2 v[PS];             // the pivot rows' part of a strip, before they are updated
+    d4 cr[RT], ci[RT];         // the strip: rows (wave + 4 q) 16 + 4 r + kq, column m
+    const uint32_t t_off = 16u * (uint32_t)(kq * n + m);
+    auto fetch = [&](int s, double2 (&pv)[PS], d4 (&xr)[RT], d4 (&xi)[RT]) {
+      const double2* Ws = Wp + s * SC;
+#pragma unroll
+      for (int q = 0; q < PS; ++q) {
+        const int idx = q * NTH + tid, c = idx / SC, j = idx % SC;
+        pv[q] = ldgb(Ws, 16u * (uint32_t)(piv[k0 + c] * n + j));
+      }
+#pragma unroll
+      for (int q = 0; q < RT; ++q) {
+        if ((wave + 4 * q) * 16 < n) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double2 o = ldgb(Ws + (size_t)((wave + 4 * q) * 16 + 4 * r) * n, t_off);
+            xr[q][r] = o.x;
+            xi[q][r] = o.y;
+          }
+        }
+      }
+    };
+    int s = next(rank), buf = 0;
+    if (s >= 0) fetch(s, v, cr, ci);
+    while (s >= 0) {
+      ldsd* Sr = S + buf * L::S1;
+      ldsd* Si = Sr + KPI * SC;
+#pragma unroll
+      for (int q = 0; q < PS; ++q) {
+        Sr[q * NTH + tid] = v[q].x;
+        Si[q * NTH + tid] = v[q].y;
+      }
+      __syncthreads();  // this strip's pivot rows (and M) complete; the buffer's last readers are two strips back
+      const int sn = next(s + size);
+      d4 nr[RT], ni[RT];
+      if (sn >= 0) fetch(sn, v, nr, ni);
+      // rows past n are multiplied too (their M is whatever LDS holds) and not stored: a
+      // guard would keep the fragment reads from running ahead of the MFMAs
+#pragma unroll
+      for (int ks = 0; ks < KPI / 4; ++ks) {
+        const int k = ks * 4 + kq;
+        const double br = Sr[k * SC + m], bi = Si[k * SC + m];
+        double ar[RT], ai[RT];
+#pragma unroll
+        for (int q = 0; q < RT; ++q) {
+          ar[q] = Mr[mix(k, (wave + 4 * q) * 16 + m)];
+          ai[q] = Mi[mix(k, (wave + 4 * q) * 16 + m)];
+        }
+#pragma unroll
+        for (int q = 0; q < RT; ++q) cr[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[q], br, cr[q], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < RT; ++q) ci[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[q], bi, ci[q], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < RT; ++q) cr[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai[q], bi, cr[q], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < RT; ++q) ci[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[q], br, ci[q], 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < RT; ++q) {
+        if ((wave + 4 * q) * 16 < n) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            stgb(Wp + s * SC + (size_t)((wave + 4 * q) * 16 + 4 * r) * n, t_off, make_double2(cr[q][r], ci[q][r]));
+        }
+        cr[q] = nr[q];
+        ci[q] = ni[q];
+      }
+      s = sn;
+      buf ^= 1;
+    }
+    group_sync(n_);
+  }
+  if (!info) {
+    late(n - KPI);
+    for (int q = tid; q < n; q += NTH) pinv[piv[q]] = q;  // inverse permutation
+  }
+  group_sync(n_);
+  // out(i, q) = W[piv[i]][pinv[q]], RB rows of out at a time: the source rows are read
+  // whole into LDS and out is written in column segments of RB elements
+  constexpr int RB = 16;
+  static_assert(2 * RB * (NMAX + 1) <= L::OFF_S, "row block fits the panel area");
+  const int ldr = n + 1;  // odd stride: the RB rows of one column sit in distinct banks
+  ldsd* Lr = Mr;
+  ldsd* Li = Mr + RB * ldr;
+  for (int i0 = rank * RB; i0 < n; i0 += size * RB) {
+    if (info) {
+      for (int idx = tid; idx < RB * n; idx += NTH) out[(size_t)(i0 + idx % RB) + (size_t)(idx / RB) * n] = make_double2(0, 0);
+      continue;
+    }
+    if (tid < n) {
+      double2 v[RB];
+#pragma unroll
+      for (int rr = 0; rr < RB; ++rr) v[rr] = ldgb(Wp, 16u * (uint32_t)(piv[i0 + rr] * n + tid));
+#pragma unroll
+      for (int rr = 0; rr < RB; ++rr) {
+        Lr[rr * ldr + tid] = v[rr].x;
+        Li[rr * ldr + tid] = v[rr].y;
+      }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < RB * n; idx += NTH) {
+      const int rr = idx % RB, q = idx / RB;
+      const int c = pinv[q];
+      out[(size_t)(i0 + rr) + (size_t)q * n] = make_double2(Lr[rr * ldr + c], Li[rr * ldr + c]);
+    }
+    __syncthreads();
+  }
+  group_sync(n_);
+  return info;
 }
 
 // ------------------------------------------------------ inverse, n > NTH
@@ -1286,7 +1565,7 @@ template <int T, int N>
 struct InvRegLds {
   static constexpr int HV = N == 32 ? 2 : 1;
   static constexpr int LDO = N + 1;           // odd row stride of the output staging tile
-  static constexpr int XCH = GjLds<1, HV>::DOUBLES;
+  static constexpr int XCH = GjLds<1, N * N / 256, HV>::DOUBLES;
   static constexpr int OUT = 2 * N * LDO;     // re / im planes of the matrix for the final copy
   static constexpr int AREA = XCH > OUT ? XCH : OUT;
   static constexpr int DOUBLES = AREA + N + 8;  // + piv, pinv (2 N ints)
@@ -1337,21 +1616,26 @@ __device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds
 template <int T, int NMAX>
 struct InvLds {
   static constexpr int A =
-      NMAX <= Cfg<T>::NTH ? InvSmallLds<T, NMAX>::DOUBLES : InvBigLds<T, NMAX>::DOUBLES;
+      NMAX <= 128 ? InvSmallLds<T, NMAX>::DOUBLES : NMAX <= 256 ? InvStripLds<NMAX>::DOUBLES : InvBigLds<T, NMAX>::DOUBLES;
   static constexpr int B = (NMAX == 32 || NMAX == 64) ? InvRegLds<T, NMAX>::DOUBLES : 0;
   static constexpr int DOUBLES = A > B ? A : B;
 };
 
 // Inverse of an n x n block (n <= NMAX): the whole matrix in registers when n = NMAX is
-// 32 or 64, one panel row per thread up to NTH rows, several rows per thread with the
+// 32 or 64, panel and pivot rows in LDS up to 128 rows, the panel alone up to 256, the
 // panels staged through `out` above that.
 template <int T, int NMAX>
 __device__ __forceinline__ int wg_inverse(int n, double2* W, double2* out, ldsd* lds) {
   if constexpr (NMAX == 32 || NMAX == 64) {
     if (n == NMAX) return wg_inverse_reg<T, NMAX>(W, out, lds);
     return wg_inverse_small<T, NMAX>(n, W, out, lds);
-  } else if constexpr (NMAX <= Cfg<T>::NTH) {
+  } else if constexpr (NMAX <= 128) {
     return wg_inverse_small<T, NMAX>(n, W, out, lds);
+  } else if constexpr (NMAX <= 256) {
+    if constexpr (NMAX == 256) {
+      if (n <= 192) return wg_inverse_strip<192>(n, W, out, lds);  // no wave multiplies rows past 192
+    }
+    return wg_inverse_strip<NMAX>(n, W, out, lds);
   } else {
     return wg_inverse_big<T, NMAX>(n, W, out, lds);
   }
