@@ -102,7 +102,7 @@ constexpr double kSteinTol = 1e-8;
 // number of doublings, or -1 when kSteinTol is not reached within nmax.
 // t: 8 temporary blocks.
 template <int T>
-__device__ double lead_adjoint(int n, bool left, const double2* C, const double2* g, const double2* Sb,
+__device__ double lead_adjoint(typename Dim<T>::type n, bool left, const double2* C, const double2* g, const double2* Sb,
                                double2* Cbar, double2* t, int nmax, int& steps, ldsd* lds, ldsd* red) {
   const size_t nn = (size_t)n * n;
   double2 *X = t, *P = t + nn, *P2 = t + 2 * nn, *Pn = t + 3 * nn, *P2n = t + 4 * nn, *Tt = t + 5 * nn;
@@ -163,7 +163,9 @@ __device__ double lead_adjoint(int n, bool left, const double2* C, const double2
 
 template <int T, int NMAX>
 __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH, ldsd* lds, ldsd* red) {
-  const int n = a.n, N = a.nx;
+  const typename Dim<T>::type n = a.n;
+  const int N = a.nx;
+  const bool first = threadIdx.x == 0 && group_leader(n);
   const size_t nn = (size_t)n * n;
   const double E = a.E[e];
   const double2 z = make_double2(E, a.eta_dev);
@@ -328,7 +330,7 @@ __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH
     const double a2 = wg_retrace_prod(n, K, T1, red);
     const double trv = -a1 - fR * a2;
     Jv += wtr * trv;
-    if (a.tr && threadIdx.x == 0) a.tr[e] = trv;
+    if (a.tr && first) a.tr[e] = trv;
   }
   Jv += wn(N - 1) * wg_imtrace(n, gl(N - 1), red);
 
@@ -429,7 +431,7 @@ __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH
       double tr_ab = 0.0;
       for (int i = threadIdx.x; i < n; i += blockDim.x) tr_ab += gc(Ab)[i + (size_t)i * n].x;
       tr_ab = block_sum(tr_ab, red);
-      if (threadIdx.x == 0) a.dU[(size_t)e * N + l] = -tr_ab;
+      if (first) a.dU[(size_t)e * N + l] = -tr_ab;
     }
     if (!a.lead && l == N - 1) {
       // Sigma_R-bar = -Abar + fR (Sbar^H - Sbar) + w_tr (G<^H - G<) + 2 w_tr fR (G^H - G)
@@ -470,13 +472,13 @@ __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH
     const double hL = lead_adjoint<T>(n, true, Cb(0), GsL, SLb, dH, Tm(2), a.dec_nmax, stL, lds, red);
     const double hR = lead_adjoint<T>(n, false, Cb(N - 1), Gs, SRb, dH + (size_t)(N - 1) * nn, Tm(2), a.dec_nmax,
                                       stR, lds, red);
-    if (threadIdx.x == 0) {
+    if (first) {
       a.dU[(size_t)e * N] += hL;
       a.dU[(size_t)e * N + N - 1] += hR;
     }
     lead_flags = (stL < 0 ? 4 : 0) | (stR < 0 ? 8 : 0);
   }
-  if (threadIdx.x == 0) {
+  if (first) {
     a.J[e] = Jv;
     if (a.info) {
       a.info[4 * (size_t)e + 0] = itL;
@@ -498,7 +500,7 @@ __global__ __launch_bounds__(Cfg<T>::NTH, Cfg<T>::OCC) void rgf_adjoint(AdjArgs 
 
 // Sum the per-slot coupling adjoints: out[l] = sum_s dH[s][l] for l = 1..nx-2, and at
 // the edges when `edges` (contacts that repeat the edge slabs), else zero there.
-__global__ void k_sum_slots(const double2* __restrict__ dH, int slots, int nx, int n, int edges,
+static __global__ void k_sum_slots(const double2* __restrict__ dH, int slots, int nx, int n, int edges,
                             double2* __restrict__ out) {
   const size_t nn = (size_t)n * n, tot = (size_t)nx * nn;
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < tot; i += (size_t)gridDim.x * blockDim.x) {

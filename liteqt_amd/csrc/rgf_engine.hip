@@ -17,6 +17,7 @@
 
 #include "../../include/rgf.h"
 #include "rgf_adjoint.hpp"
+#include "rgf_group_api.hpp"
 #include "rgf_integrate.hpp"
 #include "rgf_multi.hpp"
 #include "rgf_offdiag.hpp"
@@ -287,7 +288,7 @@ struct Prepared {
   Variant v;
   rgf::SweepArgs a;
   long long slots = 0, slot_elems = 0;
-  int dev = 0;
+  int dev = 0, cus = 0;
   bool nothing = false;
 };
 
@@ -342,6 +343,7 @@ int prepare(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, Prepa
   out->slots = slots;
   out->slot_elems = se;
   out->dev = dev;
+  out->cus = prop.multiProcessorCount;
   fill_args(p, b, se, &out->a);
   if (scba) {
     out->a.scba = 1;
@@ -395,30 +397,55 @@ void fill_args(const rgf_params* p, const rgf_batch* b, long long se, rgf::Sweep
   a.ckpt = std::max(b->ckpt, 0);
 }
 
+// Energies of a launch that a group of workgroups solves each (rgf_group.hpp): the ones
+// left over when full rounds of one energy per compute unit are taken off, where they
+// leave at least half of the compute units idle.  The rounds run first, then the groups,
+// on the same slots; `need` is the number of slots for both.  A caller that limits the
+// slots keeps one workgroup per energy.
+struct Split {
+  long long tail = 0, need = 0;
+  rgf::GroupArgs g{};
+  size_t ctl_bytes() const { return (size_t)tail * rgf::kGroupCtlBytes; }
+};
+Split group_split(int n, long long nE, int cus, long long slots, int max_slots) {
+  Split sp;
+  sp.need = slots;
+  const long long rem = nE % cus;
+  if (max_slots > 0 || rem == 0 || !rgf::group_plan(n, rem, cus, &sp.g)) return sp;
+  sp.tail = rem;
+  sp.g.e0 = (int)(nE - rem);
+  sp.need = std::max(rem, std::min<long long>(nE - rem, cus));
+  return sp;
+}
+
 int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, void* stream) {
   g_err.clear();
   Prepared pr;
   if (int rc = prepare(p, b, scba, &pr)) return rc;
   if (pr.nothing) return 0;
   long long slot_bytes = pr.slot_elems * 16LL;
-  long long slots = pr.slots;
+  Split sp = group_split(b->nm, b->nE, pr.cus, pr.slots, b->max_slots);
   std::lock_guard<std::mutex> lk(g_ws_mu);
   Buf& ws = g_ws[pr.dev];
-  if ((size_t)(slots * slot_bytes) > ws.bytes) {
+  if ((size_t)(sp.need * slot_bytes) + sp.ctl_bytes() > ws.bytes) {
     // HBM admission: fit the stored left-connected blocks into free memory
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     const size_t avail = (size_t)((double)(fr + ws.bytes) * 0.9);
     long long fit = (long long)(avail / (size_t)slot_bytes);
+    if (sp.tail && (size_t)(sp.need * slot_bytes) + sp.ctl_bytes() > avail) {
+      sp = Split();  // one workgroup per energy, on the slots that fit
+      sp.need = pr.slots;
+    }
     // automatic segment recompute: when the full slots leave CUs idle, keep the
     // blocks only at checkpoints every ceil(sqrt(nx)) slabs and one segment, at the
     // cost of one more forward sweep (7 of the 17 GEMM-equivalents of a slab), if
     // that runs more energies per unit of time
     const bool od = has_offdiag(b) || scba;
-    if (b->ckpt == 0 && !od && !b->Sii && fit < slots) {
+    if (b->ckpt == 0 && !od && !b->Sii && fit < sp.need) {
       const int K = std::max(2, (int)std::ceil(std::sqrt((double)b->nx)));
       const long long se_k = slot_elems(b->nm, b->nx, K);
-      const long long fit_k = std::min<long long>(slots, (long long)(avail / (size_t)(se_k * 16LL)));
+      const long long fit_k = std::min<long long>(sp.need, (long long)(avail / (size_t)(se_k * 16LL)));
       if (fit_k * 17 > fit * 24) {
         pr.a.ckpt = K;
         pr.a.ws_slot = se_k;
@@ -427,15 +454,25 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
       }
     }
     if (fit < 1) return fail(RGF_ENOMEM, "not enough device memory for one energy slot");
-    slots = std::min(slots, fit);
-    if ((size_t)(slots * slot_bytes) > ws.bytes) {
+    sp.need = std::min(sp.need, fit);
+    const size_t bytes = (size_t)(sp.need * slot_bytes) + sp.ctl_bytes();
+    if (bytes > ws.bytes) {
       ws.release();
-      if (int rc = ws.ensure((size_t)(slots * slot_bytes))) return rc;
+      if (int rc = ws.ensure(bytes)) return rc;
     }
   }
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   pr.a.ws = reinterpret_cast<double2*>(ws.p);
-  pr.v.launch(pr.a, (int)slots, reinterpret_cast<hipStream_t>(stream));
-  HIPCHK(hipGetLastError());
+  if (sp.tail < b->nE) {
+    rgf::SweepArgs a = pr.a;
+    a.nE = (int)(b->nE - sp.tail);
+    pr.v.launch(a, (int)std::min<long long>(sp.need, a.nE), s);
+    HIPCHK(hipGetLastError());
+  }
+  if (sp.tail) {
+    sp.g.ctl = reinterpret_cast<char*>(ws.p) + (size_t)(sp.need * slot_bytes);
+    HIPCHK(rgf::launch_sweep_grp(pr.a, sp.g, has_offdiag(b) || scba, s));
+  }
   return 0;
 }
 
@@ -1337,6 +1374,8 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
   const long long dh_bytes = (long long)b->nx * nn * 16LL;
   long long slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
   if (b->max_slots > 0) slots = std::min<long long>(slots, b->max_slots);
+  Split sp = group_split(b->nm, b->nE, prop.multiProcessorCount, slots, b->max_slots);
+  slots = sp.need;
   // The larger slot (R, R d and g S kept per slab: 5 fewer GEMMs per slab) is used
   // when every slot still fits; otherwise the small slot, recomputing them.
   const long long keep_bytes = rgf::adj_slot_blocks(b->nx, 1) * nn * 16LL;
@@ -1352,10 +1391,14 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
   int K = b->ckpt > 0 ? b->ckpt : 0;
   if (K) keep = 0;
   long long slot_bytes = K ? rgf::adj_slot_blocks(b->nx, 0, K) * nn * 16LL : keep ? keep_bytes : small_bytes;
-  if ((size_t)(slots * slot_bytes) > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
+  if ((size_t)(slots * slot_bytes) + sp.ctl_bytes() > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     const size_t avail = (size_t)((double)(fr + ws.bytes + dh.bytes) * 0.9);
+    if (sp.tail && (size_t)(slots * ((K ? slot_bytes : small_bytes) + dh_bytes)) + sp.ctl_bytes() > avail) {
+      slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
+      sp = Split();  // one workgroup per energy, on the slots that fit
+    }
     if (keep && (long long)(avail / (size_t)(keep_bytes + dh_bytes)) < slots) {
       keep = 0;
       slot_bytes = small_bytes;
@@ -1373,10 +1416,10 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
     }
     if (fit < 1) return fail(RGF_ENOMEM, "not enough device memory for one adjoint slot");
     slots = std::min(slots, fit);
-    if ((size_t)(slots * slot_bytes) > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
+    if ((size_t)(slots * slot_bytes) + sp.ctl_bytes() > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
       ws.release();
       dh.release();
-      if (int rc = ws.ensure((size_t)(slots * slot_bytes))) return rc;
+      if (int rc = ws.ensure((size_t)(slots * slot_bytes) + sp.ctl_bytes())) return rc;
       if (int rc = dh.ensure((size_t)(slots * dh_bytes))) return rc;
     }
   }
@@ -1403,8 +1446,16 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
   a.ws_slot = slot_bytes / 16LL;
   a.keep = keep;
   a.ckpt = K;
-  v.launch(a, (int)slots, s);
-  HIPCHK(hipGetLastError());
+  if (sp.tail < b->nE) {
+    a.nE = (int)(b->nE - sp.tail);
+    v.launch(a, (int)std::min<long long>(slots, a.nE), s);
+    HIPCHK(hipGetLastError());
+  }
+  if (sp.tail) {
+    a.nE = b->nE;
+    sp.g.ctl = reinterpret_cast<char*>(ws.p) + (size_t)(slots * slot_bytes);
+    HIPCHK(rgf::launch_adjoint_grp(a, sp.g, s));
+  }
   if (dH1i) {
     hipLaunchKernelGGL(rgf::k_sum_slots, dim3(1024), dim3(256), 0, s, reinterpret_cast<const double2*>(dh.p),
                        (int)slots, b->nx, b->nm, lead_H00 ? 0 : 1, reinterpret_cast<double2*>(dH1i));
@@ -1510,9 +1561,14 @@ int rgf_w_solve_batched(const rgf_w_batch* b, void* stream) {
   const size_t avail = (size_t)((double)(fr + ws.bytes) * 0.9);
   if (avail <= fixed) return fail(RGF_ENOMEM, "rgf_w_solve_batched: not enough device memory for the padded blocks");
   long long slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
-  slots = std::min<long long>(slots, (long long)((avail - fixed) / (slot_el * sizeof(double2))));
+  Split sp = group_split(np, b->nE, prop.multiProcessorCount, slots, 0);
+  if (sp.tail && fixed + (size_t)sp.need * slot_el * sizeof(double2) + sp.ctl_bytes() > avail) {
+    sp = Split();  // one workgroup per energy, on the slots that fit
+    sp.need = slots;
+  }
+  slots = std::min<long long>(sp.need, (long long)((avail - fixed) / (slot_el * sizeof(double2))));
   if (slots < 1) return fail(RGF_ENOMEM, "rgf_w_solve_batched: not enough device memory for one energy slot");
-  if (int rc = ws.ensure(fixed + (size_t)slots * slot_el * sizeof(double2))) return rc;
+  if (int rc = ws.ensure(fixed + (size_t)slots * slot_el * sizeof(double2) + sp.ctl_bytes())) return rc;
   double2* base = reinterpret_cast<double2*>(ws.p);
   rgf::WArgs a{};
   a.n = np;
@@ -1556,8 +1612,16 @@ int rgf_w_solve_batched(const rgf_w_batch* b, void* stream) {
   a.ws = base + vc_el + pad_el;
   a.ws_slot = slot_el;
   HIPCHK(hipGetLastError());
-  v.launch(a, (int)slots, s);
-  HIPCHK(hipGetLastError());
+  if (sp.tail < b->nE) {
+    a.nE = (int)(b->nE - sp.tail);
+    v.launch(a, (int)std::min<long long>(slots, a.nE), s);
+    HIPCHK(hipGetLastError());
+  }
+  if (sp.tail) {
+    a.nE = b->nE;
+    sp.g.ctl = reinterpret_cast<char*>(a.ws + (size_t)slots * slot_el);
+    HIPCHK(rgf::launch_wsweep_grp(a, sp.g, s));
+  }
   if (pad) {
     const std::pair<const double2*, double*> outs[4] = {
         {a.WL, b->WL}, {a.WG, b->WG}, {a.WR, b->WR}, {a.WRi1, b->WRi1}};

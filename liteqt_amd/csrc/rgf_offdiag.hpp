@@ -33,7 +33,9 @@ constexpr int kTmpBlocksOd = 36;
 
 template <int T, int NMAX>
 __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* lds, ldsd* red) {
-  const int n = a.n, nx = a.nx, N = nx;
+  const typename Dim<T>::type n = a.n;
+  const int nx = a.nx, N = nx;
+  const bool lead = threadIdx.x == 0 && group_leader(n);
   const size_t nn = (size_t)n * n;
   const double E = a.E[e];
   const double2 z = make_double2(E, a.eta_dev);
@@ -131,13 +133,13 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
   {
     const double a1 = wg_retrace_prod(n, T0, Gp, red);
     const double a2 = wg_retrace_prod(n, T0, Gn, red);
-    if (a.tr && threadIdx.x == 0) a.tr[e] = -(fR * a1 - (fR - 1.0) * a2);
+    if (a.tr && lead) a.tr[e] = -(fR * a1 - (fR - 1.0) * a2);
   }
   if (a.ldos) wg_ew(n, ob(a.ldos, L1), 0, zero, G, one, nullptr, one, nullptr, one);
   if (a.ndens) wg_ew(n, ob(a.ndens, L1), 0, zero, Gn, one, nullptr, one, nullptr, one);
   if (a.pdens) wg_ew(n, ob(a.pdens, L1), 0, zero, Gp, one, nullptr, one, nullptr, one);
-  if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (threadIdx.x == 0) a.dens_n[(size_t)e * nx + L1] = v; }
-  if (a.dens_p) { double v = wg_imtrace(n, Gp, red); if (threadIdx.x == 0) a.dens_p[(size_t)e * nx + L1] = -v; }
+  if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (lead) a.dens_n[(size_t)e * nx + L1] = v; }
+  if (a.dens_p) { double v = wg_imtrace(n, Gp, red); if (lead) a.dens_p[(size_t)e * nx + L1] = -v; }
   refresh(sR(L1), G);
   refresh(sL(L1), Gn);
 
@@ -184,10 +186,10 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
     if (a.ldos) wg_ew(n, ob(a.ldos, l), 0, zero, G, one, nullptr, one, nullptr, one);
     if (a.ndens) wg_ew(n, ob(a.ndens, l), 0, zero, Gn, one, nullptr, one, nullptr, one);
     if (a.pdens) wg_ew(n, ob(a.pdens, l), 0, zero, Gn, one, G, one, G, mone);
-    if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (threadIdx.x == 0) a.dens_n[(size_t)e * nx + l] = v; }
+    if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (lead) a.dens_n[(size_t)e * nx + l] = v; }
     if (a.dens_p) {
       double v = wg_imtrace(n, Gn, red) + 2.0 * wg_imtrace(n, G, red);
-      if (threadIdx.x == 0) a.dens_p[(size_t)e * nx + l] = -v;
+      if (lead) a.dens_p[(size_t)e * nx + l] = -v;
     }
     refresh(sR(l), G);
     refresh(sL(l), Gn);
@@ -199,9 +201,9 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
   {
     const double a1 = wg_retrace_prod(n, T1, T0, red);
     const double a2 = wg_retrace_prod(n, T1, Gn, red);
-    if (a.tre && threadIdx.x == 0) a.tre[e] = fL * a1 - (fL - 1.0) * a2;
+    if (a.tre && lead) a.tre[e] = fL * a1 - (fL - 1.0) * a2;
   }
-  if (a.info && threadIdx.x == 0) {
+  if (a.info && lead) {
     a.info[4 * (size_t)e + 0] = itL;
     a.info[4 * (size_t)e + 1] = itR;
     a.info[4 * (size_t)e + 2] = hitL | (hitR << 1);

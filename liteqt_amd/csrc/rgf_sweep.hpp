@@ -18,6 +18,16 @@ namespace rgf {
 
 constexpr int kTmpBlocks = 30;
 
+// Type of the block dimension that a program of variant T hands to the block operations:
+// int for a lone workgroup; a group of workgroups (rgf_group.hpp) has its own, which
+// selects the operations that share the work.
+template <int T>
+struct Dim {
+  typedef int type;
+};
+// The workgroup that writes a program's scalars.
+__device__ __forceinline__ bool group_leader(int) { return true; }
+
 struct SweepArgs {
   int n, nx, nE, mode, dec_nmax;
   double eta_dev, eta_lead, dec_tol, boltz;
@@ -78,7 +88,7 @@ __device__ __forceinline__ double ferm_dev(double a) { return 1.0 / (1.0 + exp(a
 // right lead H_10 = Hc, H_01 = Hc^H (4035).  Writes the surface function
 // G00 = (z S00 - H_SS)^-1 and returns the iterations run.
 template <int T, int NMAX>
-__device__ int wg_sancho(int n, double E, double eta, double tol, int nmax, const double2* H00,
+__device__ int wg_sancho(typename Dim<T>::type n, double E, double eta, double tol, int nmax, const double2* H00,
                          const double2* Hc, int left, double2* G00, double2* tb, ldsd* lds,
                          ldsd* red, int& hit, int& fails, const double2* S00 = nullptr) {
   const size_t nn = (size_t)n * n;
@@ -149,8 +159,10 @@ __device__ int wg_sancho(int n, double E, double eta, double tol, int nmax, cons
 // whose left-connected G^> is never filled: G^>_ll = g H^H G^>_{l+1} H g^H.
 template <int T, int NMAX, bool CMS = false>
 __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, ldsd* red) {
-  const int n = a.n, nx = a.nx;
+  const typename Dim<T>::type n = a.n;
+  const int nx = a.nx;
   const size_t nn = (size_t)n * n;
+  const bool lead = threadIdx.x == 0 && group_leader(n);
   const bool phys = (a.mode == 1);
   const double E = a.E[e];
   const double2 z = make_double2(E, a.eta_dev);
@@ -304,13 +316,13 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
   {
     const double a1 = wg_retrace_prod(n, T0, Gp, red);
     const double a2 = wg_retrace_prod(n, T0, Gn, red);
-    if (a.tr && threadIdx.x == 0) a.tr[e] = -(fR * a1 - (fR - 1.0) * a2);
+    if (a.tr && lead) a.tr[e] = -(fR * a1 - (fR - 1.0) * a2);
   }
   if (a.ldos) wg_ew(n, ob(a.ldos, L1), 0, zero, G, one, nullptr, one, nullptr, one);
   if (a.ndens) wg_ew(n, ob(a.ndens, L1), 0, zero, Gn, one, nullptr, one, nullptr, one);
   if (a.pdens) wg_ew(n, ob(a.pdens, L1), 0, zero, Gp, one, nullptr, one, nullptr, one);
-  if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (threadIdx.x == 0) a.dens_n[(size_t)e * nx + L1] = v; }
-  if (a.dens_p) { double v = wg_imtrace(n, Gp, red); if (threadIdx.x == 0) a.dens_p[(size_t)e * nx + L1] = -v; }
+  if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (lead) a.dens_n[(size_t)e * nx + L1] = v; }
+  if (a.dens_p) { double v = wg_imtrace(n, Gp, red); if (lead) a.dens_p[(size_t)e * nx + L1] = -v; }
 
   // ---- backward sweep
   const bool want_cur = a.cur != nullptr;
@@ -390,11 +402,11 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
     }
     if (a.GRi1) wg_ew(n, ob(a.GRi1, l), 0, zero, GN0, one, nullptr, one, nullptr, one);
     if (a.GLi1) wg_ew(n, ob(a.GLi1, l), 0, zero, Y2, one, nullptr, one, nullptr, one);
-    if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (threadIdx.x == 0) a.dens_n[(size_t)e * nx + l] = v; }
+    if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (lead) a.dens_n[(size_t)e * nx + l] = v; }
     if (a.dens_p) {
       // -Im Tr G^>_ll with G^> = G^< + G - G^H (CMS: the recursion's G^>)
       double v = CMS ? wg_imtrace(n, Gp, red) : wg_imtrace(n, Gn, red) + 2.0 * wg_imtrace(n, G, red);
-      if (threadIdx.x == 0) a.dens_p[(size_t)e * nx + l] = -v;
+      if (lead) a.dens_p[(size_t)e * nx + l] = -v;
     }
   }
 
@@ -405,9 +417,9 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
     const double fLt = ferm_dev((E - a.mu[0]) / (a.boltz * (phys ? a.temp[0] : a.temp[1])));
     const double a1 = wg_retrace_prod(n, T1, T0, red);
     const double a2 = wg_retrace_prod(n, T1, Gn, red);
-    if (a.tre && threadIdx.x == 0) a.tre[e] = fLt * a1 - (fLt - 1.0) * a2;
+    if (a.tre && lead) a.tre[e] = fLt * a1 - (fLt - 1.0) * a2;
   }
-  if (a.info && threadIdx.x == 0) {
+  if (a.info && lead) {
     a.info[4 * (size_t)e + 0] = itL;
     a.info[4 * (size_t)e + 1] = itR;
     a.info[4 * (size_t)e + 2] = hitL | (hitR << 1);

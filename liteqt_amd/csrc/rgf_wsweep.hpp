@@ -45,7 +45,8 @@ struct WArgs {
 
 template <int T, int NMAX>
 __device__ void w_energy(const WArgs& a, int e, double2* ws, ldsd* lds) {
-  const int n = a.n, nx = a.nx;
+  const typename Dim<T>::type n = a.n;
+  const int nx = a.nx;
   const size_t nn = (size_t)n * n;
   const double2 one = make_double2(1, 0), zero = make_double2(0, 0);
   auto eb = [&](const double2* base, int i) { return base + ((size_t)e * nx + i) * nn; };
@@ -129,7 +130,7 @@ __device__ void w_energy(const WArgs& a, int e, double2* ws, ldsd* lds) {
     lesser(i, a.PG, ebw(a.WG, i));
   }
   if (a.WRi1) wg_ew(n, ebw(a.WRi1, L), 0, zero, nullptr, one, nullptr, one, nullptr, one);
-  if (a.info && threadIdx.x == 0) a.info[e] = bad;
+  if (a.info && threadIdx.x == 0 && group_leader(n)) a.info[e] = bad;
   __syncthreads();
 }
 

@@ -1,0 +1,132 @@
+"""GPU: an energy solved by a group of workgroups (blocks of 96 to 256 orbitals, few
+energies) against the one-workgroup solve of the same energy, which a caller's slot limit
+selects.  Both form every output element from the same products in the same order; the
+bound is the rounding of one reordering, n eps times the conditioning at eta = 1e-3
+(256 * 1.1e-16 * 1e2 < 1e-11), relative per output array."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-11
+
+
+def _env():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("no HIP device visible")
+    from liteqt_amd import configs, rgf
+    return torch, configs, rgf
+
+
+def _device(nm, nx, nE, seed):
+    torch, configs, rgf = _env()
+    Hii, H1i = configs.random_device(nm, nx, seed)
+    E = torch.tensor(np.linspace(-0.6, 0.7, nE) if nE > 1 else np.array([0.1]), dtype=torch.float64, device="cuda")
+    return torch, configs, rgf, rgf.to_device_blocks(Hii), rgf.to_device_blocks(H1i), E
+
+
+def _close(a, b, name):
+    d = (a - b).norm() / b.norm()
+    assert d <= TOL, (name, float(d))
+
+
+# one energy takes the largest group, 9 energies two groups an XCD, 40 the smallest tiles
+# per rank with every variant of the inverse; 300 leaves a tail of 44 behind a full round
+@pytest.mark.parametrize("nm,nE", [(96, 1), (96, 40), (128, 1), (128, 9), (160, 3), (192, 9), (224, 1), (256, 1), (256, 17),
+                                   (96, 300)])
+@pytest.mark.parametrize("mode", ["compat", "physical"])
+def test_group_solve_equals_one_workgroup(nm, nE, mode):
+    torch, configs, rgf, H, C, E = _device(nm, 4, nE, 10 + nm)
+    p = rgf.params(rgf.MODE_COMPAT if mode == "compat" else rgf.MODE_PHYSICAL, eta_dev=1e-3)
+    nx = 4
+    sl, _, sr = configs.scattering_self_energies(nm, nx, 3, E=0.1, scale=1e-2)
+    sig = {} if nE == 9 else {"sigL": rgf.to_device_blocks(sl), "sigR": rgf.to_device_blocks(sr)}
+    res = []
+    for slots in (0, nE):
+        blk = lambda dt: torch.zeros(nE, nx, nm, nm, dtype=dt, device="cuda")
+        out = {k: blk(torch.complex128) for k in ("ldos", "ndens", "pdens", "GRi1", "GLi1", "GGi1")}
+        out["cur"] = blk(torch.float64)
+        for k in ("tr", "tre"):
+            out[k] = torch.zeros(nE, dtype=torch.float64, device="cuda")
+        for k in ("dens_n", "dens_p"):
+            out[k] = torch.zeros(nE, nx, dtype=torch.float64, device="cuda")
+        out["info"] = torch.zeros(nE, 4, dtype=torch.int32, device="cuda")
+        rgf.solve_batched(p, E, (300.0, 300.0), (0.1, -0.1), H, C, out=out, max_slots=slots, **sig)
+        torch.cuda.synchronize()
+        res.append(out)
+    assert torch.equal(res[0]["info"], res[1]["info"])
+    for k in res[0]:
+        if k != "info":
+            _close(res[0][k], res[1][k], k)
+
+
+@pytest.mark.parametrize("nm,nE", [(96, 5), (128, 3), (256, 2)])
+def test_group_offdiag_refresh_equals_one_workgroup(nm, nE):
+    nx = 4
+    torch, configs, rgf, H, C, E = _device(nm, nx, nE, 20 + nm)
+    p = rgf.params(rgf.MODE_PHYSICAL, eta_dev=1e-3)
+    names = ("sigL", "sigR", "sigR_lo", "sigR_up", "sigL_up")
+    blocks = configs.offdiag_self_energies(configs.scattering_blocks(nm, nx, 4, scale=1e-2), 0.4)
+    res = []
+    for slots in (0, nE):
+        sig = {k: rgf.to_device_blocks(b).unsqueeze(0).repeat(nE, 1, 1, 1).contiguous() for k, b in zip(names, blocks)}
+        out = {"tr": torch.zeros(nE, dtype=torch.float64, device="cuda"),
+               "dens_p": torch.zeros(nE, nx, dtype=torch.float64, device="cuda")}
+        rgf.solve_batched(p, E, (300.0, 300.0), (0.1, -0.1), H, C, out=out, max_slots=slots, scba=(1e-2, 0.5), **sig)
+        torch.cuda.synchronize()
+        res.append({**out, **sig})
+    for k in res[0]:
+        _close(res[0][k], res[1][k], k)
+
+
+@pytest.mark.parametrize("nm,nE,ckpt", [(96, 4, 0), (128, 100, 0), (256, 3, 0), (128, 3, 2)])
+def test_group_adjoint_equals_one_workgroup(nm, nE, ckpt):
+    nx = 5
+    torch, configs, rgf, H, C, E = _device(nm, nx, nE, 30 + nm)
+    p = rgf.params(rgf.MODE_PHYSICAL, eta_dev=1e-3)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w_tr = torch.rand(nE, dtype=torch.float64, device="cuda", generator=g)
+    w_n = torch.rand(nE, nx, dtype=torch.float64, device="cuda", generator=g)
+    res = [rgf.adjoint_batched(p, E, (300.0, 300.0), (0.1, -0.1), H, C, w_tr=w_tr, w_n=w_n, max_slots=slots, ckpt=ckpt)
+           for slots in (0, nE)]
+    torch.cuda.synchronize()
+    for a, b, name in zip(res[0], res[1], ("J", "dU", "dH")):
+        _close(a, b, name)
+
+
+# the screened interaction has no slot limit: 3 energies alone (groups) against the same
+# energies as the first of 256 (one workgroup each)
+@pytest.mark.parametrize("nm", [96, 128, 200])
+def test_group_w_equals_one_workgroup(nm):
+    torch, configs, rgf = _env()
+    nx, nE = 4, 3
+    g = torch.Generator(device="cuda").manual_seed(nm)
+    cn = lambda *s: torch.randn(*s, dtype=torch.complex128, device="cuda", generator=g) / nm ** 0.5
+    V, V1, P = cn(nx, nm, nm), cn(nx, nm, nm) * 0.3, [cn(nE, nx, nm, nm) * 0.2 for _ in range(3)]
+    few = rgf.w_solve_batched(V, V1, *P, want_i1=True)
+    many = rgf.w_solve_batched(V, V1, *[torch.cat([x, x[:1].expand(256 - nE, -1, -1, -1)]).contiguous() for x in P],
+                               want_i1=True)
+    torch.cuda.synchronize()
+    for k in ("WL", "WG", "WR", "WRi1"):
+        _close(few[k], many[k][:nE], k)
+    assert int(few["info"].sum()) == 0
+
+
+def test_group_singular_slab_is_zeroed_and_counted():
+    """A singular slab block (above and below 128 orbitals) is zeroed and counted once by a group, as by one workgroup."""
+    for nm in (128, 160):
+        nx, nE = 3, 2
+        torch, configs, rgf, H, C, E = _device(nm, nx, nE, 40 + nm)
+        H, C = torch.zeros_like(H), torch.zeros_like(C)
+        E = torch.zeros_like(E)
+        p = rgf.params(rgf.MODE_PHYSICAL, eta_dev=0.0)
+        res = []
+        for slots in (0, nE):
+            out = {"ldos": torch.full((nE, nx, nm, nm), 7.0, dtype=torch.complex128, device="cuda"),
+                   "info": torch.zeros(nE, 4, dtype=torch.int32, device="cuda")}
+            rgf.solve_batched(p, E, (300.0, 300.0), (0.0, 0.0), H, C, out=out, max_slots=slots)
+            torch.cuda.synchronize()
+            res.append(out)
+        assert torch.equal(res[0]["info"], res[1]["info"]) and int(res[0]["info"][0, 3]) == nx
+        assert torch.equal(res[0]["ldos"], res[1]["ldos"]) and float(res[0]["ldos"].abs().max()) == 0.0
