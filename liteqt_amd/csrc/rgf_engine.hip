@@ -692,7 +692,7 @@ struct MultiPlan {
   std::vector<int2> items;
   long long ws_slot = 0;
   int slots = 0;
-  int dev = 0;
+  int dev = 0, cus = 0;
   int ntuned = 0;
 };
 
@@ -707,6 +707,7 @@ int multi_plan(const rgf_params* p, const rgf_batch* devs, int ndev, int autotun
   int per_cu = 0;
   if (multi_per_cu(&per_cu) || per_cu < 1) return fail(RGF_EHIP, "multi-device kernel does not fit on a CU");
   const int full = prop.multiProcessorCount * per_cu;
+  pl->cus = prop.multiProcessorCount;
   long long nitems = 0, se_max = 0;
   for (auto& a : pl->jobs) {
     nitems += a.nE;
@@ -744,6 +745,42 @@ int multi_plan(const rgf_params* p, const rgf_batch* devs, int ndev, int autotun
     slots = std::min(slots, fit);
   }
   pl->slots = (int)std::max<long long>(slots, 1);
+  return 0;
+}
+
+// Upload the descriptors of a launch with one group per item, and launch it.
+int multi_group_launch(const MultiPlan& pl, const rgf::MultiGroupPlan& gp, Buf* desc, void* ws, hipStream_t s) {
+  const size_t ng = gp.sizes.size();
+  std::vector<int2> items;
+  for (int i : gp.order) items.push_back(pl.items[(size_t)i]);
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = off;
+    off += (bytes + 255) / 256 * 256;
+    return o;
+  };
+  const size_t oJobs = take(sizeof(rgf::SweepArgs) * pl.jobs.size()), oItems = take(sizeof(int2) * items.size());
+  const size_t oFirst = take(sizeof(int) * (ng + 1)), oSizes = take(sizeof(int) * ng);
+  const size_t oBlocks = take(sizeof(int) * gp.block_group.size());
+  const size_t oCtl = take(rgf::kGroupCtlBytes * ng);
+  if (int rc = desc->ensure(off)) return rc;
+  char* base = reinterpret_cast<char*>(desc->p);
+  HIPCHK(hipMemcpy(base + oJobs, pl.jobs.data(), sizeof(rgf::SweepArgs) * pl.jobs.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(base + oItems, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(base + oFirst, gp.first.data(), sizeof(int) * (ng + 1), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(base + oSizes, gp.sizes.data(), sizeof(int) * ng, hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(base + oBlocks, gp.block_group.data(), sizeof(int) * gp.block_group.size(), hipMemcpyHostToDevice));
+  rgf::MultiGroupArgs m;
+  m.jobs = reinterpret_cast<const rgf::SweepArgs*>(base + oJobs);
+  m.items = reinterpret_cast<const int2*>(base + oItems);
+  m.first = reinterpret_cast<const int*>(base + oFirst);
+  m.sizes = reinterpret_cast<const int*>(base + oSizes);
+  m.block_group = reinterpret_cast<const int*>(base + oBlocks);
+  m.ngroups = (int)ng;
+  m.ctl = base + oCtl;
+  m.ws = reinterpret_cast<double2*>(ws);
+  m.ws_slot = pl.ws_slot;
+  HIPCHK(rgf::launch_multi_grp(m, (int)gp.block_group.size(), s));
   return 0;
 }
 }  // namespace
@@ -877,6 +914,18 @@ int rgf_solve_devices(const rgf_params* p, const rgf_batch* devs, int ndev, int 
     if (int rc = ws.ensure((size_t)(pl.ws_slot * 16LL * pl.slots))) return rc;
   }
   Buf& desc = g_multi_desc[dev];
+  if (pl.slots == (int)std::min<size_t>(pl.items.size(), (size_t)pl.cus) &&
+      pl.items.size() <= (size_t)rgf::kMultiGroupItems * pl.cus) {
+    // few items for the compute units: the longer ones get groups of workgroups, the
+    // shorter ones share a workgroup (with more items the shared counter balances them)
+    std::vector<int> in, inx;
+    for (const int2& it : pl.items) {
+      in.push_back(pl.jobs[it.x].n);
+      inx.push_back(pl.jobs[it.x].nx);
+    }
+    rgf::MultiGroupPlan gp;
+    if (rgf::multi_group_plan(in, inx, pl.cus, &gp)) return multi_group_launch(pl, gp, &desc, ws.p, s);
+  }
   const MultiDesc L = multi_layout(ndev, (long long)pl.items.size());
   if (int rc = desc.ensure(L.bytes)) return rc;
   if (int rc = multi_upload(pl.jobs, pl.mv, pl.items, desc.p)) return rc;

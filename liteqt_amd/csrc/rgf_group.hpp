@@ -108,22 +108,12 @@ __device__ __noinline__ void group_barrier() {
 }
 __device__ __forceinline__ void group_sync(GroupN) { group_barrier(); }
 
-// Join the group of this workgroup; false when it is closed (the workgroup leaves).
-// Workgroups are dealt to the XCDs in turn, so a group of up to 32 takes blocks of equal
-// index mod 8: its ranks share an L2.  `spread` groups (more than an XCD holds) take
-// consecutive blocks.
-__device__ __forceinline__ bool group_join(const GroupArgs& g, int& grp) {
-  const int b = blockIdx.x;
-  if (g.spread) {
-    grp = b / g.size;
-  } else {
-    const int q = (b / 8) / g.size;
-    grp = q < g.per_xcd ? q * 8 + b % 8 : g.ngroups;
-  }
-  if (grp >= g.ngroups) return false;
+// Join a group of `size` workgroups at control area ctl; false when it is closed (the
+// workgroup leaves).
+__device__ __forceinline__ bool group_join(char* area, int size) {
   GroupCtx* c = group_ctx();
   if (threadIdx.x == 0) {
-    GroupCtl* ctl = reinterpret_cast<GroupCtl*>(g.ctl + (size_t)grp * kGroupCtlBytes);
+    GroupCtl* ctl = reinterpret_cast<GroupCtl*>(area);
     const unsigned r = __hip_atomic_fetch_add(&ctl->arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     c->ctl = ctl;
     c->epoch = 0;
@@ -131,7 +121,7 @@ __device__ __forceinline__ bool group_join(const GroupArgs& g, int& grp) {
     c->size = 0;
     if (r == 0) {
       const unsigned long long t0 = wall_clock64();
-      while (agent_load(&ctl->arrivals) < (unsigned)g.size && wall_clock64() - t0 < (unsigned long long)kJoinTicks)
+      while (agent_load(&ctl->arrivals) < (unsigned)size && wall_clock64() - t0 < (unsigned long long)kJoinTicks)
         __builtin_amdgcn_s_sleep(1);
       const unsigned m = __hip_atomic_fetch_add(&ctl->arrivals, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       agent_store(&ctl->members, m);
@@ -144,6 +134,15 @@ __device__ __forceinline__ bool group_join(const GroupArgs& g, int& grp) {
   }
   __syncthreads();
   return uni(c->size) > 0;
+}
+
+// The same by block index.  Workgroups are dealt to the XCDs in turn, so a group takes
+// blocks of equal index mod 8: its ranks share an L2.
+__device__ __forceinline__ bool group_join(const GroupArgs& g, int& grp) {
+  const int b = blockIdx.x, q = (b / kXcds) / g.size;
+  grp = q < g.per_xcd ? q * kXcds + b % kXcds : g.ngroups;
+  if (grp >= g.ngroups) return false;
+  return group_join(g.ctl + (size_t)grp * kGroupCtlBytes, g.size);
 }
 
 // ------------------------------------------------------------------- GEMM
@@ -468,6 +467,35 @@ __global__ __launch_bounds__(256, 1) void rgf_wsweep_grp(WArgs a, GroupArgs g) {
   double2* ws = a.ws + (size_t)grp * (size_t)a.ws_slot;
   for (int e = g.e0 + grp; e < a.nE; e += g.ngroups) {
     w_energy<kGrp, NMAX>(a, e, ws, (ldsd*)lds);
+    group_barrier();
+  }
+}
+
+// Several devices on groups of unequal size, each running its list of (device, energy)
+// items.
+struct MultiGroupLds {
+  static constexpr int A = SweepLds<kGrp, 256>::DOUBLES, B = SweepLds<kGrp, 128>::DOUBLES;
+  static constexpr int C = SweepLds<2, 64>::DOUBLES;
+  static constexpr int AB = A > B ? A : B, DOUBLES = AB > C ? AB : C;
+};
+
+__global__ __launch_bounds__(256, 1) void rgf_sweep_multi_grp(MultiGroupArgs m) {
+  __shared__ __attribute__((aligned(16))) double lds[MultiGroupLds::DOUBLES];
+  const int grp = uni(m.block_group[blockIdx.x]);
+  if (grp < 0 || !group_join(m.ctl + (size_t)grp * kGroupCtlBytes, uni(m.sizes[grp]))) return;
+  double2* ws = m.ws + (size_t)grp * (size_t)m.ws_slot;
+  ldsd* L = (ldsd*)lds;
+  for (int i = uni(m.first[grp]); i < uni(m.first[grp + 1]); ++i) {
+    const int job = uni(m.items[i].x), e = uni(m.items[i].y);
+    const SweepArgs& a = m.jobs[job];
+    if (a.n == 32)  // in groups of one workgroup only
+      solve_energy<1, 32>(a, e, ws, L, L);
+    else if (a.n == 64)
+      solve_energy<2, 64>(a, e, ws, L, L);
+    else if (a.n <= 128)
+      solve_energy<kGrp, 128>(a, e, ws, L, L);
+    else
+      solve_energy<kGrp, 256>(a, e, ws, L, L);
     group_barrier();
   }
 }

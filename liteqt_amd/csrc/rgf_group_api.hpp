@@ -2,12 +2,15 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 namespace rgf {
 
 constexpr size_t kGroupCtlBytes = 2048;
+constexpr int kXcds = 8;
 
 struct GroupArgs {
-  int ngroups, size, per_xcd, spread;
+  int ngroups, size, per_xcd;
   int e0;       // first energy of the launch
   int grid;
   char* ctl;    // ngroups control areas of kGroupCtlBytes
@@ -17,6 +20,25 @@ struct SweepArgs;
 struct AdjArgs;
 struct WArgs;
 
+// Many devices with at most kMultiGroupItems (device, energy) items per compute unit:
+// groups of workgroups with lists of items, sizes and lists by the items' costs.
+constexpr int kMultiGroupItems = 2;
+struct MultiGroupArgs {
+  const SweepArgs* jobs;
+  const int2* items;       // (device, energy), group by group
+  const int* first;        // group g runs items first[g] .. first[g + 1] - 1
+  const int* sizes;        // workgroups of each group
+  const int* block_group;  // group of each block, -1: none
+  int ngroups;
+  char* ctl;
+  double2* ws;
+  long long ws_slot;
+};
+struct MultiGroupPlan {
+  std::vector<int> sizes, first, block_group;
+  std::vector<int> order;  // the items, group by group
+};
+
 // Groups for nE energies of n orbitals on `cus` compute units; false where one workgroup
 // per energy is the faster (or only) form.
 bool group_plan(int n, long long nE, int cus, GroupArgs* g);
@@ -25,5 +47,10 @@ bool group_plan(int n, long long nE, int cus, GroupArgs* g);
 hipError_t launch_sweep_grp(const SweepArgs& a, const GroupArgs& g, bool od, hipStream_t s);
 hipError_t launch_adjoint_grp(const AdjArgs& a, const GroupArgs& g, hipStream_t s);
 hipError_t launch_wsweep_grp(const WArgs& a, const GroupArgs& g, hipStream_t s);
+
+// The groups for items of n[i] orbitals and nx[i] slabs, longest first; false where one
+// workgroup per item is as fast.
+bool multi_group_plan(const std::vector<int>& n, const std::vector<int>& nx, int cus, MultiGroupPlan* pl);
+hipError_t launch_multi_grp(const MultiGroupArgs& m, int blocks, hipStream_t s);
 
 }  // namespace rgf

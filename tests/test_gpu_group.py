@@ -130,3 +130,27 @@ def test_group_singular_slab_is_zeroed_and_counted():
             res.append(out)
         assert torch.equal(res[0]["info"], res[1]["info"]) and int(res[0]["info"][0, 3]) == nx
         assert torch.equal(res[0]["ldos"], res[1]["ldos"]) and float(res[0]["ldos"].abs().max()) == 0.0
+
+
+# block sizes of every kind of group (32 and 64 on one workgroup, lists of several items),
+# fewer and more items than the 256 compute units
+@pytest.mark.parametrize("counts", [(3, 2, 5, 2, 1, 2, 1), (200, 40, 9, 7, 3, 2, 4)])
+def test_group_devices_equal_one_workgroup(counts):
+    torch, configs, rgf = _env()
+    p = rgf.params(rgf.MODE_PHYSICAL, eta_dev=1e-3)
+    devs, ref = [], []
+    for j, (nm, nE) in enumerate(zip((32, 64, 96, 128, 160, 192, 256), counts)):
+        nx = 3 + j % 3
+        _, _, _, H, C, E = _device(nm, nx, nE, 50 + nm)
+        new = lambda: {"tr": torch.zeros(nE, dtype=torch.float64, device="cuda"),
+                       "dens_n": torch.zeros(nE, nx, dtype=torch.float64, device="cuda"),
+                       "info": torch.zeros(nE, 4, dtype=torch.int32, device="cuda")}
+        devs.append({"E": E, "temp": (300.0, 300.0), "mu": (0.1, -0.1), "Hii": H, "H1i": C, "out": new()})
+        ref.append(rgf.solve_batched(p, E, (300.0, 300.0), (0.1, -0.1), H, C, out=new(), max_slots=nE))
+    _, rep = rgf.solve_devices(p, devs)
+    torch.cuda.synchronize()
+    assert rep["items"] == sum(counts)
+    for d, r in zip(devs, ref):
+        assert torch.equal(d["out"]["info"], r["info"])
+        _close(d["out"]["tr"], r["tr"], "tr")
+        _close(d["out"]["dens_n"], r["dens_n"], "dens_n")
