@@ -252,6 +252,9 @@ __device__ __forceinline__ void block_argmax(double& v, int& idx, ldsd* redv, ld
 // are compiled for (their launch bounds): the same code at OCC = 2 is a
 // separate instantiation of every block function, so the register budget of
 // two workgroups per CU applies to it alone.
+// Variant kReg32 is for blocks of exactly 32 orbitals at four workgroups per CU, with its
+// own GEMM.
+constexpr int kReg32 = 25;
 template <int V>
 struct Cfg {
   static constexpr int T = V & 7;
@@ -365,7 +368,7 @@ __device__ __forceinline__ void mma_steps(d4 (&cr)[TA][TB], d4 (&ci)[TA][TB],
 // value in every thread).
 template <int T>
 struct GemmLds {
-  static constexpr int DOUBLES = 2 * Cfg<T>::STAGE;  // two stages (the abs-sum reduction reuses stage 0)
+  static constexpr int DOUBLES = T == kReg32 ? 64 : 2 * Cfg<T>::STAGE;  // two stages (the abs-sum reduction reuses stage 0)
 };
 
 // Byte offset of each of a thread's panel elements from the panel origin.
@@ -590,14 +593,114 @@ __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__
 }
 
 template <int T, int OPA, int OPB, int CRM>
-__device__ __noinline__ double wg_gemm_k(int n, const double2* __restrict__ A, const double2* __restrict__ B, void* Cout,
-                                         Epi ep, ldsd* lds) {
+__device__ __noinline__ double gemm_panels(int n, const double2* __restrict__ A, const double2* __restrict__ B, void* Cout,
+                                           Epi ep, ldsd* lds) {
   const double asum = gemm_tiles<T, OPA, OPB, CRM>(n, A, B, Cout, ep, lds, 0, 1);
   double s = 0.0;
   // stage 0 is free after the last panel's barrier
   if (uni(ep.abs_sum)) s = block_sum(asum, lds);
   __syncthreads();
   return s;
+}
+
+// GEMM of 32-orbital blocks: one 16 x 16 tile per wave, its MFMA fragments loaded straight
+// from memory, all 16 loads of a lane (and the D1 terms) in flight at once.  At this size
+// a GEMM is 0.87 us of MFMAs on a CU and its time the latency of its loads, which panels
+// through LDS paid three times (two panels, the epilogue) with a barrier each; without
+// LDS stages four workgroups fit on a CU and fill each other's waits.  The products are
+// summed in the order of mma_steps.
+template <int OPA, int OPB, int CRM>
+__device__ __noinline__ double gemm_reg32(const double2* __restrict__ A_, const double2* __restrict__ B_, void* Cout_,
+                                          Epi ep_, ldsd* lds) {
+  constexpr int n = 32, NK = n / 4;
+  const double2* A = uni(A_);
+  const double2* B = uni(B_);
+  void* Cout = uni(Cout_);
+  Epi ep;
+  ep.diag = uni(ep_.diag); ep.sacc = uni(ep_.sacc);
+  ep.D1 = uni(ep_.D1); ep.s1 = uni(ep_.s1);
+  ep.D2 = uni(ep_.D2); ep.s2 = uni(ep_.s2);
+  ep.D3 = uni(ep_.D3); ep.s3 = uni(ep_.s3);
+  ep.real_out = uni(ep_.real_out); ep.abs_sum = uni(ep_.abs_sum);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = lane & 15, kq = lane >> 4;
+  const int arow = (wave & 1) * 16, bcol = (wave >> 1) * 16;
+  // op(A)(arow + m, 4 ks + kq), op(B)(4 ks + kq, bcol + m)
+  const uint32_t ao = 16u * (uint32_t)(OPA == OP_N ? arow + m + kq * n : kq + (arow + m) * n);
+  const uint32_t bo = 16u * (uint32_t)(OPB == OP_N ? kq + (bcol + m) * n : bcol + m + kq * n);
+  double2 a[NK], b[NK];
+#pragma unroll
+  for (int ks = 0; ks < NK; ++ks) {
+    a[ks] = ldgb(A + (OPA == OP_N ? 4 * ks * n : 4 * ks), ao);
+    b[ks] = ldgb(B + (OPB == OP_N ? 4 * ks : 4 * ks * n), bo);
+  }
+  const int i0 = arow + (CRM ? kq : m), j0 = bcol + (CRM ? m : kq);  // element r: (i0 + 4 r, j0) or (i0, j0 + 4 r)
+  const uint32_t cm = 16u * (uint32_t)(i0 + j0 * n), tr = 16u * (uint32_t)(j0 + i0 * n);
+  constexpr int DCM = CRM ? 4 : 4 * n, DTR = CRM ? 4 * n : 4;  // steps of r, in elements
+  double2 d1[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) d1[r] = make_double2(0, 0);
+  if (ep.D1) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d1[r] = ldgb(ep.D1 + r * DCM, cm);
+  }
+  d4 cr = d4{0, 0, 0, 0}, ci = d4{0, 0, 0, 0};
+#pragma unroll
+  for (int ks = 0; ks < NK; ++ks) {
+    const double ar = a[ks].x, ai = OPA == OP_C ? -a[ks].y : a[ks].y;
+    const double br = b[ks].x, bi = OPB == OP_C ? -b[ks].y : b[ks].y;
+    if (CRM) {
+      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ci, 0, 0, 0);
+      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ci, 0, 0, 0);
+    } else {
+      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ar, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, ar, ci, 0, 0, 0);
+      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, -ai, cr, 0, 0, 0);
+      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ai, ci, 0, 0, 0);
+    }
+  }
+  double2 d2[4], d3[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) d2[r] = d3[r] = make_double2(0, 0);
+  if (ep.D2) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d2[r] = ldgb(ep.D2 + r * DCM, cm);
+  }
+  if (ep.D3) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d3[r] = ldgb(ep.D3 + r * DTR, tr);
+  }
+  double asum = 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = CRM ? i0 + 4 * r : i0, j = CRM ? j0 : j0 + 4 * r;
+    double2 v = make_double2(ep.sacc * cr[r], ep.sacc * ci[r]);
+    const double2 vd = cadd(v, ep.diag);
+    v.x = (i == j) ? vd.x : v.x;
+    v.y = (i == j) ? vd.y : v.y;
+    if (ep.D1) v = cadd(v, cmul(ep.s1, d1[r]));
+    if (ep.D2) v = cadd(v, cmul(ep.s2, d2[r]));
+    if (ep.D3) v = cadd(v, cmul(ep.s3, cconj(d3[r])));
+    if (ep.abs_sum) asum += sqrt(v.y * v.y + v.x * v.x);
+    if (ep.real_out)
+      stgb_re((double*)Cout + r * (CRM ? DTR : DCM), (CRM ? tr : cm) / 2, v.x);
+    else
+      stgb((double2*)Cout + r * (CRM ? DTR : DCM), CRM ? tr : cm, v);
+  }
+  double s = 0.0;
+  if (ep.abs_sum) s = block_sum(asum, lds);
+  __syncthreads();
+  return s;
+}
+
+template <int T, int OPA, int OPB, int CRM>
+__device__ __forceinline__ double wg_gemm_k(int n, const double2* A, const double2* B, void* Cout, Epi ep, ldsd* lds) {
+  if constexpr (T == kReg32)
+    return gemm_reg32<OPA, OPB, CRM>(A, B, Cout, ep, lds);
+  else
+    return gemm_panels<T, OPA, OPB, CRM>(n, A, B, Cout, ep, lds);
 }
 
 template <int T>
@@ -622,19 +725,63 @@ __device__ __forceinline__ double wg_gemm(int n, int opA, const double2* A, int 
 // --------------------------------------------------------------- elementwise
 // out(i,j) = diag*[i==j] + s1*D1(i,j) + s2*D2(i,j) + s3*conj(D3(j,i)); row-major
 // output when out_rowmajor.  D1/D2 may alias out (not D3).
+// The elements of share `rank` of `size`: a thread takes four at a time with all their
+// loads in flight (one at a time the operation is as long as its loads' latencies), and
+// steps its row and column instead of dividing the index.
+__device__ __forceinline__ void ew_elements(int n, double2* out_, int out_rowmajor, double2 diag, const double2* D1_,
+                                            double2 s1, const double2* D2_, double2 s2, const double2* D3_, double2 s3,
+                                            int rank, int size) {
+  constexpr int U = 4;
+  const int nn = n * n, step = 256 * size, first = rank * 256 + (int)threadIdx.x;
+  const int dslow = step / n, dfast = step - dslow * n;
+  int slow = first / n, fast = first - slow * n;  // (j, i), or (i, j) when row-major
+  double2* out = uni(out_);
+  const double2 *D1 = uni(D1_), *D2 = uni(D2_), *D3 = uni(D3_);
+  for (int idx = first; idx < nn; idx += U * step) {
+    uint32_t o[U], t[U];  // offsets of the element and of its transpose, column-major
+    bool in[U], dg[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      in[u] = idx + u * step < nn;
+      const int i = in[u] ? (out_rowmajor ? slow : fast) : 0, j = in[u] ? (out_rowmajor ? fast : slow) : 0;
+      o[u] = 16u * (uint32_t)(i + j * n);
+      t[u] = 16u * (uint32_t)(j + i * n);
+      dg[u] = i == j;
+      fast += dfast;
+      slow += dslow;
+      if (fast >= n) {
+        fast -= n;
+        ++slow;
+      }
+    }
+    double2 d1[U], d2[U], d3[U];
+    if (D1) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) d1[u] = ldgb(D1, o[u]);
+    }
+    if (D2) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) d2[u] = ldgb(D2, o[u]);
+    }
+    if (D3) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) d3[u] = ldgb(D3, t[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      double2 v = make_double2(dg[u] ? diag.x : 0.0, dg[u] ? diag.y : 0.0);
+      if (D1) v = cadd(v, cmul(s1, d1[u]));
+      if (D2) v = cadd(v, cmul(s2, d2[u]));
+      if (D3) v = cadd(v, cmul(s3, cconj(d3[u])));
+      if (in[u]) stgb(out, out_rowmajor ? t[u] : o[u], v);
+    }
+  }
+}
+
 __device__ __noinline__ void wg_ew(int n, double2* out, int out_rowmajor, double2 diag,
                                    const double2* D1, double2 s1, const double2* D2, double2 s2,
                                    const double2* D3, double2 s3) {
-  const int nn = n * n;
-  for (int idx = threadIdx.x; idx < nn; idx += blockDim.x) {
-    int i, j;
-    if (out_rowmajor) { j = idx % n; i = idx / n; } else { i = idx % n; j = idx / n; }
-    double2 v = (i == j) ? diag : make_double2(0, 0);
-    if (D1) v = cadd(v, cmul(s1, gc(D1)[i + (size_t)j * n]));
-    if (D2) v = cadd(v, cmul(s2, gc(D2)[i + (size_t)j * n]));
-    if (D3) v = cadd(v, cmul(s3, cconj(gc(D3)[j + (size_t)i * n])));
-    gw(out)[out_rowmajor ? (size_t)i * n + j : (size_t)i + (size_t)j * n] = v;
-  }
+  ew_elements(uni(n), out, uni(out_rowmajor), diag, D1, s1, D2, s2, D3, s3, 0, 1);
   __syncthreads();
 }
 
@@ -950,7 +1097,7 @@ __device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned
 // the inverse is written column-major to out.  Returns 0, or k+1 when column k
 // has no nonzero pivot, in which case out is zeroed (src/green_rgf.f90:4429-4437).
 //
-// Panel step (16 or 32 columns K, pivot rows P): the panel is swept in registers
+// Panel step (32 columns K, pivot rows P): the panel is swept in registers
 // (gj_sweep), giving F_P = A_PK^-1 and F_R = -A_RK A_PK^-1; the other
 // columns J are updated by one MFMA GEMM W[:,J] += (F - E) W[P,J] with E the pivot
 // incidence (accumulating onto the loaded tiles of W), and columns K take F.
@@ -959,9 +1106,7 @@ __device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned
 template <int T, int NMAX>
 struct InvSmallLds {
   static constexpr int LDI = NMAX + PAD;
-  // columns per panel: 32 where the swept panel and the pivot rows fit in LDS (half the
-  // passes over W), else 16; 16 up to 64 rows, where two workgroups share a CU's LDS
-  static constexpr int KPI = NMAX > 64 && NMAX <= 128 ? 32 : 16;
+  static constexpr int KPI = 32;  // columns per panel: the swept panel and the pivot rows fit in LDS
   static constexpr int DOUBLES = 4 * KPI * LDI + 2 * NMAX + 16;
 };
 
@@ -1615,20 +1760,18 @@ __device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds
 
 template <int T, int NMAX>
 struct InvLds {
-  static constexpr int A =
-      NMAX <= 128 ? InvSmallLds<T, NMAX>::DOUBLES : NMAX <= 256 ? InvStripLds<NMAX>::DOUBLES : InvBigLds<T, NMAX>::DOUBLES;
-  static constexpr int B = (NMAX == 32 || NMAX == 64) ? InvRegLds<T, NMAX>::DOUBLES : 0;
-  static constexpr int DOUBLES = A > B ? A : B;
+  static constexpr int DOUBLES = NMAX <= 64    ? InvRegLds<T, NMAX>::DOUBLES
+                                 : NMAX <= 128 ? InvSmallLds<T, NMAX>::DOUBLES
+                                 : NMAX <= 256 ? InvStripLds<NMAX>::DOUBLES
+                                               : InvBigLds<T, NMAX>::DOUBLES;
 };
 
-// Inverse of an n x n block (n <= NMAX): the whole matrix in registers when n = NMAX is
-// 32 or 64, panel and pivot rows in LDS up to 128 rows, the panel alone up to 256, the
+// Inverse of an n x n block (n <= NMAX): the whole matrix in registers at 32 and 64, panel and pivot rows in LDS up to 128 rows, the panel alone up to 256, the
 // panels staged through `out` above that.
 template <int T, int NMAX>
 __device__ __forceinline__ int wg_inverse(int n, double2* W, double2* out, ldsd* lds) {
   if constexpr (NMAX == 32 || NMAX == 64) {
-    if (n == NMAX) return wg_inverse_reg<T, NMAX>(W, out, lds);
-    return wg_inverse_small<T, NMAX>(n, W, out, lds);
+    return wg_inverse_reg<T, NMAX>(W, out, lds);  // these variants are chosen for n = NMAX only
   } else if constexpr (NMAX <= 128) {
     return wg_inverse_small<T, NMAX>(n, W, out, lds);
   } else if constexpr (NMAX <= 256) {

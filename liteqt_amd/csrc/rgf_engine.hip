@@ -119,7 +119,7 @@ bool pick_adj(int n, AdjVariant* v) {
   if (n % 32 != 0 || n < 32 || n > 256) return false;
 #define ADJV(T, NM) {launch_adj<T, NM>, reinterpret_cast<const void*>(&rgf::rgf_adjoint<T, NM>), rgf::Cfg<T>::NTH}
   switch (n) {
-    case 32: *v = ADJV(1, 32); return true;
+    case 32: *v = ADJV(rgf::kReg32, 32); return true;
     case 64: *v = ADJV(2, 64); return true;
     case 96: *v = ADJV(3, 96); return true;
     case 128: *v = ADJV(4, 128); return true;
@@ -188,7 +188,7 @@ bool pick_variant(int n, Variant* v) {
   }
   if (n % 32 != 0 || n < 32 || n > 256) return false;
   switch (n) {
-    case 32: *v = {launch_sweep<kOcc2 + 1, 32>, sweep_fn<kOcc2 + 1, 32>(), 1, 32, rgf::Cfg<1>::NTH}; return true;
+    case 32: *v = {launch_sweep<rgf::kReg32, 32>, sweep_fn<rgf::kReg32, 32>(), 1, 32, rgf::Cfg<1>::NTH}; return true;
     case 64: *v = {launch_sweep<kOcc2 + 2, 64>, sweep_fn<kOcc2 + 2, 64>(), 2, 64, rgf::Cfg<2>::NTH}; return true;
     case 96: *v = {launch_sweep<3, 96>, sweep_fn<3, 96>(), 3, 96, rgf::Cfg<3>::NTH}; return true;
     case 128: *v = {launch_sweep<4, 128>, sweep_fn<4, 128>(), 4, 128, rgf::Cfg<4>::NTH}; return true;
@@ -202,7 +202,7 @@ bool pick_variant(int n, Variant* v) {
 bool pick_variant_od(int n, Variant* v) {
   if (n % 32 != 0 || n < 32 || n > 256) return false;
   switch (n) {
-    case 32: *v = {launch_sweep_od<kOcc2 + 1, 32>, sweep_od_fn<kOcc2 + 1, 32>(), 1, 32, rgf::Cfg<1>::NTH}; return true;
+    case 32: *v = {launch_sweep_od<rgf::kReg32, 32>, sweep_od_fn<rgf::kReg32, 32>(), 1, 32, rgf::Cfg<1>::NTH}; return true;
     case 64: *v = {launch_sweep_od<kOcc2 + 2, 64>, sweep_od_fn<kOcc2 + 2, 64>(), 2, 64, rgf::Cfg<2>::NTH}; return true;
     case 96: *v = {launch_sweep_od<3, 96>, sweep_od_fn<3, 96>(), 3, 96, rgf::Cfg<3>::NTH}; return true;
     case 128: *v = {launch_sweep_od<4, 128>, sweep_od_fn<4, 128>(), 4, 128, rgf::Cfg<4>::NTH}; return true;
@@ -251,7 +251,7 @@ bool pick_w(int n, WVariant* v) {
   }
   if (n % 32 != 0 || n < 32 || n > 256) return false;
   switch (n) {
-    case 32: *v = WV(kOcc2 + 1, 32); return true;
+    case 32: *v = WV(rgf::kReg32, 32); return true;
     case 64: *v = WV(kOcc2 + 2, 64); return true;
     case 96: *v = WV(3, 96); return true;
     case 128: *v = WV(4, 128); return true;

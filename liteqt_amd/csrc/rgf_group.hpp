@@ -360,16 +360,7 @@ __device__ __forceinline__ double wg_gemm(GroupN n, int opA, const double2* A, i
 // ----------------------------------------------------- elementwise, reductions
 __device__ __noinline__ void wg_ew(GroupN n_, double2* out, int out_rowmajor, double2 diag, const double2* D1, double2 s1,
                                    const double2* D2, double2 s2, const double2* D3, double2 s3) {
-  const int n = uni((int)n_), nn = n * n, step = 256 * group_size(n_);
-  for (int idx = group_rank(n_) * 256 + threadIdx.x; idx < nn; idx += step) {
-    int i, j;
-    if (out_rowmajor) { j = idx % n; i = idx / n; } else { i = idx % n; j = idx / n; }
-    double2 v = (i == j) ? diag : make_double2(0, 0);
-    if (D1) v = cadd(v, cmul(s1, gc(D1)[i + (size_t)j * n]));
-    if (D2) v = cadd(v, cmul(s2, gc(D2)[i + (size_t)j * n]));
-    if (D3) v = cadd(v, cmul(s3, cconj(gc(D3)[j + (size_t)i * n])));
-    gw(out)[out_rowmajor ? (size_t)i * n + j : (size_t)i + (size_t)j * n] = v;
-  }
+  ew_elements(uni((int)n_), out, uni(out_rowmajor), diag, D1, s1, D2, s2, D3, s3, group_rank(n_), group_size(n_));
   group_barrier();
 }
 
@@ -489,7 +480,7 @@ __global__ __launch_bounds__(256, 1) void rgf_sweep_multi_grp(MultiGroupArgs m) 
     const int job = uni(m.items[i].x), e = uni(m.items[i].y);
     const SweepArgs& a = m.jobs[job];
     if (a.n == 32)  // in groups of one workgroup only
-      solve_energy<1, 32>(a, e, ws, L, L);
+      solve_energy<kReg32, 32>(a, e, ws, L, L);
     else if (a.n == 64)
       solve_energy<2, 64>(a, e, ws, L, L);
     else if (a.n <= 128)
