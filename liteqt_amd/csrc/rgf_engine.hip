@@ -18,6 +18,7 @@
 #include "../../include/rgf.h"
 #include "rgf_adjoint.hpp"
 #include "rgf_group_api.hpp"
+#include "rgf_hostcopy.hpp"
 #include "rgf_integrate.hpp"
 #include "rgf_multi.hpp"
 #include "rgf_offdiag.hpp"
@@ -103,6 +104,7 @@ __global__ void unpad_blocks(const V* __restrict__ src, int np, V* __restrict__ 
 }
 
 Buf g_stage[kMaxDev];
+rgf::PinnedAreas g_pinned[kMaxDev];  // guarded by g_mu, as g_stage
 Buf g_adj_dh[kMaxDev];
 
 typedef void (*AdjLaunch)(const rgf::AdjArgs&, int grid, hipStream_t);
@@ -1146,16 +1148,17 @@ static int rs_core(const rgf_params* p, const double temp[2], int nm, int nx, co
   char* base = (char*)g_stage[dev].p;
   auto D = [&](size_t o) { return (void*)(base + o); };
   hipStream_t s = nullptr;
+  HIPCHK(g_pinned[dev].ensure((size_t)nout * cslab_u * C + (has_cur ? rslab_u * C : 0) + 4096));
+  rgf::HostCopier copier(g_pinned[dev], s);
   const double2 fill = make_double2(1.0e3, 0.0);
   // (count) energies' (nm, nm, nx) complex slabs, energy e0 + i of `a`, into a padded
   // device area; `diag` fills the padded diagonal
   auto h2d = [&](const EArr& a, long long e0, long long count, size_t dst_off, double2 diag) -> int {
     char* stage = padded ? (char*)D(oU) : (char*)D(dst_off);
     if (a.strided()) {
-      HIPCHK(hipMemcpyAsync(stage, a.at(e0), cslab_u * count, hipMemcpyHostToDevice, s));
+      HIPCHK(copier.to_device(stage, a.at(e0), cslab_u * count));
     } else {
-      for (long long i = 0; i < count; ++i)
-        HIPCHK(hipMemcpyAsync(stage + cslab_u * i, a.at(e0 + i), cslab_u, hipMemcpyHostToDevice, s));
+      for (long long i = 0; i < count; ++i) HIPCHK(copier.to_device(stage + cslab_u * i, a.at(e0 + i), cslab_u));
     }
     if (padded) {
       hipLaunchKernelGGL(pad_blocks, dim3(1024), dim3(256), 0, s, (const double2*)D(oU), nm, (double2*)D(dst_off),
@@ -1182,7 +1185,7 @@ static int rs_core(const rgf_params* p, const double temp[2], int nm, int nx, co
       if (io.sigL.present()) if (int rc = h2d(io.sigL, e0, ce, oSL, make_double2(0, 0))) return rc;
       if (io.sigR.present()) if (int rc = h2d(io.sigR, e0, ce, oSR, make_double2(0, 0))) return rc;
     }
-    HIPCHK(hipMemcpyAsync(D(oE), io.E + e0, 8 * ce, hipMemcpyHostToDevice, s));
+    HIPCHK(copier.to_device(D(oE), io.E + e0, 8 * ce));
     rgf_batch b;
     std::memset(&b, 0, sizeof(b));
     b.nm = np; b.nx = nx; b.nE = (int)ce;
@@ -1201,12 +1204,7 @@ static int rs_core(const rgf_params* p, const double temp[2], int nm, int nx, co
     if (int rc = rgf_solve_batched(p, &b, s)) return rc;
     // outputs: diagonal blocks for l = 1..nx, off-diagonal and cur for l = 1..nx-1
     auto d2h = [&](const EArr& a, const void* src, size_t slab, size_t bytes) -> int {
-      if (a.strided()) {
-        HIPCHK(hipMemcpy2DAsync(a.at(e0), slab, src, slab, bytes, ce, hipMemcpyDeviceToHost, s));
-      } else {
-        for (long long i = 0; i < ce; ++i)
-          HIPCHK(hipMemcpyAsync(a.at(e0 + i), (const char*)src + slab * i, bytes, hipMemcpyDeviceToHost, s));
-      }
+      for (long long i = 0; i < ce; ++i) HIPCHK(copier.to_host(a.at(e0 + i), (const char*)src + slab * i, bytes));
       return 0;
     };
     for (int k = 0; k < 6; ++k) {
@@ -1231,10 +1229,10 @@ static int rs_core(const rgf_params* p, const double temp[2], int nm, int nx, co
       }
       if (int rc = d2h(io.cur, src, rslab_u, (size_t)(nx - 1) * bn * 8)) return rc;
     }
-    HIPCHK(hipMemcpyAsync(trh.data(), D(oTr), 8 * ce, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(treh.data(), D(oTre), 8 * ce, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(infoh.data(), D(oInfo), 16 * ce, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(copier.to_host(trh.data(), D(oTr), 8 * ce));
+    HIPCHK(copier.to_host(treh.data(), D(oTre), 8 * ce));
+    HIPCHK(copier.to_host(infoh.data(), D(oInfo), 16 * ce));
+    HIPCHK(copier.finish());
     for (long long i = 0; i < ce; ++i) {
       if (io.tr.present()) *(double*)io.tr.at(e0 + i) = trh[(size_t)i];
       if (io.tre.present()) *(double*)io.tre.at(e0 + i) = treh[(size_t)i];
@@ -1715,10 +1713,12 @@ int rgf_integrate(int nk, int nE, int nx, const double* E, const double* midgap,
 void rgf_release(void) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return;
+  std::lock_guard<std::mutex> lh(g_mu);
   std::lock_guard<std::mutex> lk(g_ws_mu);
   g_ws[dev].release();
   g_stage[dev].release();
   g_adj_dh[dev].release();
+  g_pinned[dev].release();
 }
 
 }  // extern "C"
