@@ -252,9 +252,6 @@ __device__ __forceinline__ void block_argmax(double& v, int& idx, ldsd* redv, ld
 // are compiled for (their launch bounds): the same code at OCC = 2 is a
 // separate instantiation of every block function, so the register budget of
 // two workgroups per CU applies to it alone.
-// Variant kReg32 is for blocks of exactly 32 orbitals at four workgroups per CU, with its
-// own GEMM.
-constexpr int kReg32 = 25;
 template <int V>
 struct Cfg {
   static constexpr int T = V & 7;
@@ -368,7 +365,7 @@ __device__ __forceinline__ void mma_steps(d4 (&cr)[TA][TB], d4 (&ci)[TA][TB],
 // value in every thread).
 template <int T>
 struct GemmLds {
-  static constexpr int DOUBLES = T == kReg32 ? 64 : 2 * Cfg<T>::STAGE;  // two stages (the abs-sum reduction reuses stage 0)
+  static constexpr int DOUBLES = 2 * Cfg<T>::STAGE;  // two stages (the abs-sum reduction reuses stage 0)
 };
 
 // Byte offset of each of a thread's panel elements from the panel origin.
@@ -593,114 +590,14 @@ __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__
 }
 
 template <int T, int OPA, int OPB, int CRM>
-__device__ __noinline__ double gemm_panels(int n, const double2* __restrict__ A, const double2* __restrict__ B, void* Cout,
-                                           Epi ep, ldsd* lds) {
+__device__ __noinline__ double wg_gemm_k(int n, const double2* __restrict__ A, const double2* __restrict__ B, void* Cout,
+                                         Epi ep, ldsd* lds) {
   const double asum = gemm_tiles<T, OPA, OPB, CRM>(n, A, B, Cout, ep, lds, 0, 1);
   double s = 0.0;
   // stage 0 is free after the last panel's barrier
   if (uni(ep.abs_sum)) s = block_sum(asum, lds);
   __syncthreads();
   return s;
-}
-
-// GEMM of 32-orbital blocks: one 16 x 16 tile per wave, its MFMA fragments loaded straight
-// from memory, all 16 loads of a lane (and the D1 terms) in flight at once.  At this size
-// a GEMM is 0.87 us of MFMAs on a CU and its time the latency of its loads, which panels
-// through LDS paid three times (two panels, the epilogue) with a barrier each; without
-// LDS stages four workgroups fit on a CU and fill each other's waits.  The products are
-// summed in the order of mma_steps.
-template <int OPA, int OPB, int CRM>
-__device__ __noinline__ double gemm_reg32(const double2* __restrict__ A_, const double2* __restrict__ B_, void* Cout_,
-                                          Epi ep_, ldsd* lds) {
-  constexpr int n = 32, NK = n / 4;
-  const double2* A = uni(A_);
-  const double2* B = uni(B_);
-  void* Cout = uni(Cout_);
-  Epi ep;
-  ep.diag = uni(ep_.diag); ep.sacc = uni(ep_.sacc);
-  ep.D1 = uni(ep_.D1); ep.s1 = uni(ep_.s1);
-  ep.D2 = uni(ep_.D2); ep.s2 = uni(ep_.s2);
-  ep.D3 = uni(ep_.D3); ep.s3 = uni(ep_.s3);
-  ep.real_out = uni(ep_.real_out); ep.abs_sum = uni(ep_.abs_sum);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int m = lane & 15, kq = lane >> 4;
-  const int arow = (wave & 1) * 16, bcol = (wave >> 1) * 16;
-  // op(A)(arow + m, 4 ks + kq), op(B)(4 ks + kq, bcol + m)
-  const uint32_t ao = 16u * (uint32_t)(OPA == OP_N ? arow + m + kq * n : kq + (arow + m) * n);
-  const uint32_t bo = 16u * (uint32_t)(OPB == OP_N ? kq + (bcol + m) * n : bcol + m + kq * n);
-  double2 a[NK], b[NK];
-#pragma unroll
-  for (int ks = 0; ks < NK; ++ks) {
-    a[ks] = ldgb(A + (OPA == OP_N ? 4 * ks * n : 4 * ks), ao);
-    b[ks] = ldgb(B + (OPB == OP_N ? 4 * ks : 4 * ks * n), bo);
-  }
-  const int i0 = arow + (CRM ? kq : m), j0 = bcol + (CRM ? m : kq);  // element r: (i0 + 4 r, j0) or (i0, j0 + 4 r)
-  const uint32_t cm = 16u * (uint32_t)(i0 + j0 * n), tr = 16u * (uint32_t)(j0 + i0 * n);
-  constexpr int DCM = CRM ? 4 : 4 * n, DTR = CRM ? 4 * n : 4;  // steps of r, in elements
-  double2 d1[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) d1[r] = make_double2(0, 0);
-  if (ep.D1) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) d1[r] = ldgb(ep.D1 + r * DCM, cm);
-  }
-  d4 cr = d4{0, 0, 0, 0}, ci = d4{0, 0, 0, 0};
-#pragma unroll
-  for (int ks = 0; ks < NK; ++ks) {
-    const double ar = a[ks].x, ai = OPA == OP_C ? -a[ks].y : a[ks].y;
-    const double br = b[ks].x, bi = OPB == OP_C ? -b[ks].y : b[ks].y;
-    if (CRM) {
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ci, 0, 0, 0);
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ci, 0, 0, 0);
-    } else {
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ar, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, ar, ci, 0, 0, 0);
-      cr = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, -ai, cr, 0, 0, 0);
-      ci = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ai, ci, 0, 0, 0);
-    }
-  }
-  double2 d2[4], d3[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) d2[r] = d3[r] = make_double2(0, 0);
-  if (ep.D2) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) d2[r] = ldgb(ep.D2 + r * DCM, cm);
-  }
-  if (ep.D3) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) d3[r] = ldgb(ep.D3 + r * DTR, tr);
-  }
-  double asum = 0.0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = CRM ? i0 + 4 * r : i0, j = CRM ? j0 : j0 + 4 * r;
-    double2 v = make_double2(ep.sacc * cr[r], ep.sacc * ci[r]);
-    const double2 vd = cadd(v, ep.diag);
-    v.x = (i == j) ? vd.x : v.x;
-    v.y = (i == j) ? vd.y : v.y;
-    if (ep.D1) v = cadd(v, cmul(ep.s1, d1[r]));
-    if (ep.D2) v = cadd(v, cmul(ep.s2, d2[r]));
-    if (ep.D3) v = cadd(v, cmul(ep.s3, cconj(d3[r])));
-    if (ep.abs_sum) asum += sqrt(v.y * v.y + v.x * v.x);
-    if (ep.real_out)
-      stgb_re((double*)Cout + r * (CRM ? DTR : DCM), (CRM ? tr : cm) / 2, v.x);
-    else
-      stgb((double2*)Cout + r * (CRM ? DTR : DCM), CRM ? tr : cm, v);
-  }
-  double s = 0.0;
-  if (ep.abs_sum) s = block_sum(asum, lds);
-  __syncthreads();
-  return s;
-}
-
-template <int T, int OPA, int OPB, int CRM>
-__device__ __forceinline__ double wg_gemm_k(int n, const double2* A, const double2* B, void* Cout, Epi ep, ldsd* lds) {
-  if constexpr (T == kReg32)
-    return gemm_reg32<OPA, OPB, CRM>(A, B, Cout, ep, lds);
-  else
-    return gemm_panels<T, OPA, OPB, CRM>(n, A, B, Cout, ep, lds);
 }
 
 template <int T>

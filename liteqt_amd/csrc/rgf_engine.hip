@@ -22,6 +22,7 @@
 #include "rgf_integrate.hpp"
 #include "rgf_multi.hpp"
 #include "rgf_offdiag.hpp"
+#include "rgf_small.hpp"
 #include "rgf_sweep.hpp"
 #include "rgf_wsweep.hpp"
 

@@ -31,6 +31,7 @@
 #include "rgf_adjoint.hpp"
 #include "rgf_group_api.hpp"
 #include "rgf_offdiag.hpp"
+#include "rgf_small.hpp"
 #include "rgf_sweep.hpp"
 #include "rgf_wsweep.hpp"
 

@@ -25,6 +25,13 @@ template <int T>
 struct Dim {
   typedef int type;
 };
+// Where temporary k of a program is: in the workspace slot, or for some variants in LDS.
+// The decimation's are kTmpSancho + 0 .. 10.
+constexpr int kTmpSancho = 19;
+template <int T>
+struct Temp {
+  static __device__ __forceinline__ double2* at(double2* tb, size_t nn, int k, ldsd*) { return tb + (size_t)k * nn; }
+};
 // The workgroup that writes a program's scalars.
 __device__ __forceinline__ bool group_leader(int) { return true; }
 
@@ -100,11 +107,12 @@ __device__ int wg_sancho(typename Dim<T>::type n, double E, double eta, double t
   double2* h10n = tb + 3 * nn;
   double2* h01 = tb + 4 * nn;
   double2* h01n = tb + 5 * nn;
-  double2* A = tb + 6 * nn;
-  double2* B = tb + 7 * nn;
-  double2* C = tb + 8 * nn;
-  double2* B2 = tb + 9 * nn;
-  double2* W = tb + 10 * nn;
+  auto tmp = [&](int k) { return Temp<T>::at(tb - kTmpSancho * nn, nn, kTmpSancho + k, lds); };
+  double2* A = tmp(6);
+  double2* B = tmp(7);
+  double2* C = tmp(8);
+  double2* B2 = tmp(9);
+  double2* W = tmp(10);
   if (left) {
     wg_ew(n, h10, 0, zero, nullptr, one, nullptr, one, Hc, one);
     wg_ew(n, h01, 0, zero, Hc, one, nullptr, one, nullptr, one);
@@ -175,26 +183,27 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
   double2* Gl = ws;
   double2* Gln = ws + (size_t)nstore * nn;
   double2* tb = ws + 2 * (size_t)nstore * nn;
-  double2* G = tb + 0 * nn;
-  double2* Gn = tb + 1 * nn;
-  double2* Gp = tb + 2 * nn;
-  double2* SL = tb + 3 * nn;
-  double2* SR = tb + 4 * nn;
-  double2* W = tb + 5 * nn;
-  double2* H00 = tb + 6 * nn;
-  double2* T0 = tb + 7 * nn;
-  double2* T1 = tb + 8 * nn;
-  double2* T2 = tb + 9 * nn;
-  double2* T3 = tb + 10 * nn;
-  double2* X = tb + 11 * nn;
-  double2* P7 = tb + 12 * nn;
-  double2* Wm = tb + 13 * nn;
-  double2* Y2 = tb + 14 * nn;
-  double2* GN0 = tb + 15 * nn;
-  double2* V = tb + 16 * nn;
-  double2* S = tb + 17 * nn;
-  double2* sig = tb + 18 * nn;
-  double2* stmp = tb + 19 * nn;  // 11 blocks for the decimation
+  auto tmp = [&](int k) { return Temp<T>::at(tb, nn, k, lds); };
+  double2* G = tmp(0);
+  double2* Gn = tmp(1);
+  double2* Gp = tmp(2);
+  double2* SL = tmp(3);
+  double2* SR = tmp(4);
+  double2* W = tmp(5);
+  double2* H00 = tmp(6);
+  double2* T0 = tmp(7);
+  double2* T1 = tmp(8);
+  double2* T2 = tmp(9);
+  double2* T3 = tmp(10);
+  double2* X = tmp(11);
+  double2* P7 = tmp(12);
+  double2* Wm = tmp(13);
+  double2* Y2 = tmp(14);
+  double2* GN0 = tmp(15);
+  double2* V = tmp(16);
+  double2* S = tmp(17);
+  double2* sig = tmp(18);
+  double2* stmp = tb + kTmpSancho * nn;  // 11 blocks for the decimation
   auto Hb = [&](int l) { return a.Hii + (size_t)l * nn; };
   auto Cb = [&](int l) { return a.H1i + (size_t)l * nn; };
   auto sR = [&](int l) -> const double2* { return a.sigR ? a.sigR + (size_t)e * a.sig_stride + (size_t)l * nn : nullptr; };
