@@ -212,6 +212,17 @@ typedef struct rgf_scba {
 
 int rgf_scba_step(const rgf_params *p, const rgf_batch *b, const rgf_scba *scba, void *stream);
 
+/* rgf_solve_batched with a block-tridiagonal Sigma (physical mode) and a second lesser
+ * source: `second` holds Sigma^< blocks (sigL diagonal, sigL_up first off-diagonal, either
+ * may be NULL, same energy stride as the batch's) and ndens, which receives its diagonal
+ * G^< blocks.  The retarded blocks are formed once for both sources; the contacts enter
+ * the second source as they enter the first. */
+typedef struct rgf_lesser {
+  const double *sigL, *sigL_up;
+  double *ndens;
+} rgf_lesser;
+int rgf_solve_two_lesser(const rgf_params *p, const rgf_batch *b, const rgf_lesser *second, void *stream);
+
 /* HIP-graph form of rgf_solve_batched / rgf_scba_step: rgf_graph_create
  * captures one launch on `stream` (a created stream, not NULL) into an
  * executable graph that owns its workspace; rgf_graph_launch replays it

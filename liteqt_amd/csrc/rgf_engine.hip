@@ -275,7 +275,7 @@ __global__ void conj_blocks(const double2* __restrict__ src, double2* __restrict
 long long slot_elems(int n, int nx, int ckpt = 0) {
   return rgf::sweep_slot_blocks(nx, ckpt, rgf::kTmpBlocks) * n * n;
 }
-long long slot_elems_od(int n, int nx) { return (long long)(2 * nx + rgf::kTmpBlocksOd) * n * n; }
+long long slot_elems_od(int n, int nx, bool second) { return (long long)((second ? 3 : 2) * nx + rgf::kTmpBlocksOd) * n * n; }
 
 bool has_offdiag(const rgf_batch* b) { return b->sigR_lo || b->sigR_up || b->sigL_up; }
 
@@ -299,7 +299,8 @@ void fill_args(const rgf_params* p, const rgf_batch* b, long long se, rgf::Sweep
 
 // Validate a batch, pick the kernel and size the slots (HBM admission).  The
 // workspace pointer is left null; the caller binds the shared or an owned one.
-int prepare(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, Prepared* out) {
+int prepare(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, Prepared* out,
+            const rgf_lesser* second = nullptr) {
   if (int rc = check_params(p)) return rc;
   if (!b) return fail(RGF_EINVAL, "batch is NULL");
   if (b->nx < 2) return fail(RGF_EINVAL, "nx must be >= 2 (the reference reads Gl(:,:,nx-1))");
@@ -309,8 +310,9 @@ int prepare(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, Prepa
     return 0;
   }
   if (!b->E || !b->Hii || !b->H1i) return fail(RGF_EINVAL, "E, Hii and H1i are required");
-  const bool od = has_offdiag(b) || scba;
+  const bool od = has_offdiag(b) || scba || second;
   const bool cms = b->Sii != nullptr;
+  if (second && scba) return fail(RGF_EINVAL, "the SCBA refresh takes one lesser source");
   if (od && p->mode != RGF_MODE_PHYSICAL)
     return fail(RGF_EINVAL, "off-diagonal Sigma and the SCBA refresh need RGF_MODE_PHYSICAL");
   if (cms && (od || p->mode != RGF_MODE_COMPAT))
@@ -340,7 +342,7 @@ int prepare(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, Prepa
   int per_cu = 0;
   HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, v.fn, v.nth, 0));
   if (per_cu < 1) return fail(RGF_EHIP, "sweep kernel does not fit on a CU");
-  const long long se = od ? slot_elems_od(b->nm, b->nx) : slot_elems(b->nm, b->nx, std::max(b->ckpt, 0));
+  const long long se = od ? slot_elems_od(b->nm, b->nx, second != nullptr) : slot_elems(b->nm, b->nx, std::max(b->ckpt, 0));
   long long slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
   if (b->max_slots > 0) slots = std::min<long long>(slots, b->max_slots);
   out->slots = slots;
@@ -348,6 +350,11 @@ int prepare(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, Prepa
   out->dev = dev;
   out->cus = prop.multiProcessorCount;
   fill_args(p, b, se, &out->a);
+  if (second) {
+    out->a.sigL2 = reinterpret_cast<const double2*>(second->sigL);
+    out->a.sigL2_up = reinterpret_cast<const double2*>(second->sigL_up);
+    out->a.ndens2 = reinterpret_cast<double2*>(second->ndens);
+  }
   if (scba) {
     out->a.scba = 1;
     out->a.scba_D = scba->D;
@@ -421,11 +428,13 @@ Split group_split(int n, long long nE, int cus, long long slots, int max_slots) 
   return sp;
 }
 
-int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, void* stream) {
+int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, void* stream,
+               const rgf_lesser* second = nullptr) {
   g_err.clear();
   Prepared pr;
-  if (int rc = prepare(p, b, scba, &pr)) return rc;
+  if (int rc = prepare(p, b, scba, &pr, second)) return rc;
   if (pr.nothing) return 0;
+  const bool od = has_offdiag(b) || scba || second;
   long long slot_bytes = pr.slot_elems * 16LL;
   Split sp = group_split(b->nm, b->nE, pr.cus, pr.slots, b->max_slots);
   std::lock_guard<std::mutex> lk(g_ws_mu);
@@ -444,7 +453,6 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
     // blocks only at checkpoints every ceil(sqrt(nx)) slabs and one segment, at the
     // cost of one more forward sweep (7 of the 17 GEMM-equivalents of a slab), if
     // that runs more energies per unit of time
-    const bool od = has_offdiag(b) || scba;
     if (b->ckpt == 0 && !od && !b->Sii && fit < sp.need) {
       const int K = std::max(2, (int)std::ceil(std::sqrt((double)b->nx)));
       const long long se_k = slot_elems(b->nm, b->nx, K);
@@ -474,7 +482,7 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
   }
   if (sp.tail) {
     sp.g.ctl = reinterpret_cast<char*>(ws.p) + (size_t)(sp.need * slot_bytes);
-    HIPCHK(rgf::launch_sweep_grp(pr.a, sp.g, has_offdiag(b) || scba, s));
+    HIPCHK(rgf::launch_sweep_grp(pr.a, sp.g, od, s));
   }
   return 0;
 }
@@ -821,6 +829,14 @@ int rgf_scba_step(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba,
     return fail(RGF_EINVAL, "rgf_scba_step: scba is NULL");
   }
   return solve_impl(p, b, scba, stream);
+}
+
+int rgf_solve_two_lesser(const rgf_params* p, const rgf_batch* b, const rgf_lesser* second, void* stream) {
+  if (!second || !second->ndens) {
+    g_err.clear();
+    return fail(RGF_EINVAL, "rgf_solve_two_lesser: second and its ndens are required");
+  }
+  return solve_impl(p, b, nullptr, stream, second);
 }
 
 struct rgf_graph_s {

@@ -18,6 +18,10 @@
 // off-diagonal blocks vanish.  The contacts, tr, tre, cur and the output set
 // follow the physical mode.
 //
+// A second lesser source (a.ndens2 with a.sigL2, a.sigL2_up) is carried along: its
+// G^< follows from the same retarded blocks (8 products a slab besides the source, where
+// a solve of its own would repeat the 8 products and the inverse of the retarded ones).
+//
 // With a.scba set, each block of Sigma that was given is refreshed in place
 // once its Green's function block is final:
 //   Sigma <- (1 - mix) Sigma + mix * D * G     (elastic scattering, same energy)
@@ -40,26 +44,34 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
   const double E = a.E[e];
   const double2 z = make_double2(E, a.eta_dev);
   const double2 one = make_double2(1, 0), mone = make_double2(-1, 0), zero = make_double2(0, 0);
+  const int nsrc = a.ndens2 ? 2 : 1;  // lesser sources
   double2* gv = ws;
-  double2* gnv = ws + (size_t)nx * nn;
-  double2* tb = ws + 2 * (size_t)nx * nn;
+  double2* gnv = ws + (size_t)nx * nn;  // g^< of the first, then of the second source
+  double2* tb = ws + (size_t)(1 + nsrc) * nx * nn;
   auto Tm = [&](int k) { return tb + (size_t)k * nn; };
   double2 *H00 = Tm(0), *W = Tm(1), *SL = Tm(2), *SR = Tm(3), *T0 = Tm(4), *T1 = Tm(5), *T2 = Tm(6);
   double2 *Dd = Tm(7), *Du = Tm(8), *V = Tm(9), *G = Tm(10), *Gn = Tm(11), *Q = Tm(12), *R = Tm(13);
   double2 *Glo = Tm(14), *QGn = Tm(15), *gs = Tm(16), *M = Tm(17), *Gnn = Tm(18), *Rd = Tm(19), *Z = Tm(20);
-  double2 *W1 = Tm(21), *K1 = Tm(22), *Gs = Tm(23);
+  double2 *W1 = Tm(21), *K1 = Tm(22), *Gs = Tm(23), *Gn2 = Tm(24);
   double2* stmp = Tm(25);  // 11 blocks for the decimation
   const size_t so = (size_t)e * a.sig_stride;
   auto Hb = [&](int l) { return a.Hii + (size_t)l * nn; };
   auto Cb = [&](int l) { return a.H1i + (size_t)l * nn; };
   auto sR = [&](int l) -> const double2* { return a.sigR ? a.sigR + so + (size_t)l * nn : nullptr; };
-  auto sL = [&](int l) -> const double2* { return a.sigL ? a.sigL + so + (size_t)l * nn : nullptr; };
+  auto sL = [&](int l, int q = 0) -> const double2* {
+    const double2* b = q ? a.sigL2 : a.sigL;
+    return b ? b + so + (size_t)l * nn : nullptr;
+  };
   auto sRlo = [&](int l) -> const double2* { return a.sigR_lo ? a.sigR_lo + so + (size_t)l * nn : nullptr; };
   auto sRup = [&](int l) -> const double2* { return a.sigR_up ? a.sigR_up + so + (size_t)l * nn : nullptr; };
-  auto sLup = [&](int l) -> const double2* { return a.sigL_up ? a.sigL_up + so + (size_t)l * nn : nullptr; };
+  auto sLup = [&](int l, int q = 0) -> const double2* {
+    const double2* b = q ? a.sigL2_up : a.sigL_up;
+    return b ? b + so + (size_t)l * nn : nullptr;
+  };
   auto ob = [&](double2* arr, int l) -> double2* { return arr ? arr + ((size_t)e * nx + l) * nn : nullptr; };
   auto g = [&](int l) { return gv + (size_t)l * nn; };
-  auto gn = [&](int l) { return gnv + (size_t)l * nn; };
+  auto gn = [&](int l, int q = 0) { return gnv + (size_t)(q * nx + l) * nn; };
+  auto Gnq = [&](int q) { return q ? Gn2 : Gn; };
   const Epi st = epi_store();
   auto acc = [&](const double2* D) { Epi x = epi_store(); x.D1 = D; return x; };
   const double2 keep = make_double2(1.0 - a.scba_mix, 0), take = make_double2(a.scba_mix * a.scba_D, 0);
@@ -92,13 +104,14 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
   wg_ew(n, T1, 0, zero, Hb(0), one, sR(0), one, nullptr, one);
   wg_ew(n, W, 1, z, T1, mone, SL, mone, nullptr, one);
   if (wg_inverse<T, NMAX>(n, W, g(0), lds)) ++fails;
-  wg_ew(n, T2, 0, zero, SL, make_double2(-fL, 0), sL(0), one, SL, make_double2(fL, 0));
-  wg_gemm<T>(n, OP_N, g(0), OP_N, T2, T0, 0, st, lds);
-  wg_gemm<T>(n, OP_N, T0, OP_C, g(0), gn(0), 0, st, lds);
+  for (int q = 0; q < nsrc; ++q) {
+    wg_ew(n, T2, 0, zero, SL, make_double2(-fL, 0), sL(0, q), one, SL, make_double2(fL, 0));
+    wg_gemm<T>(n, OP_N, g(0), OP_N, T2, T0, 0, st, lds);
+    wg_gemm<T>(n, OP_N, T0, OP_C, g(0), gn(0, q), 0, st, lds);
+  }
   for (int l = 1; l < N; ++l) {
     const bool last = (l == N - 1);
     double2* gg = last ? G : g(l);
-    double2* gng = last ? Gn : gn(l);
     couple(l);
     wg_gemm<T>(n, OP_N, Dd, OP_N, g(l - 1), T0, 0, st, lds);   // d g_{l-1}
     Epi ew = epi_store();
@@ -109,20 +122,22 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
     }
     wg_gemm<T>(n, OP_N, T0, OP_N, Du, W, 1, ew, lds);          // z - H - Sigma^R - d g u
     if (wg_inverse<T, NMAX>(n, W, gg, lds)) ++fails;
-    Epi es = epi_store();
-    es.D1 = sL(l);
-    if (sLup(l)) {
-      wg_gemm<T>(n, OP_N, T0, OP_N, sLup(l), V, 0, st, lds);   // V = d g s
-      es.D2 = V; es.D3 = V; es.s3 = mone;
+    for (int q = 0; q < nsrc; ++q) {
+      Epi es = epi_store();
+      es.D1 = sL(l, q);
+      if (sLup(l, q)) {
+        wg_gemm<T>(n, OP_N, T0, OP_N, sLup(l, q), V, 0, st, lds);  // V = d g s
+        es.D2 = V; es.D3 = V; es.s3 = mone;
+      }
+      if (last) {
+        wg_ew(n, T2, 0, zero, SR, make_double2(-fR, 0), sL(l, q), one, SR, make_double2(fR, 0));
+        es.D1 = T2;
+      }
+      wg_gemm<T>(n, OP_N, Dd, OP_N, gn(l - 1, q), T1, 0, st, lds);  // d g<_{l-1}
+      wg_gemm<T>(n, OP_N, T1, OP_C, Dd, T2, 0, es, lds);            // + Sigma^< + V - V^H
+      wg_gemm<T>(n, OP_N, gg, OP_N, T2, T1, 0, st, lds);
+      wg_gemm<T>(n, OP_N, T1, OP_C, gg, last ? Gnq(q) : gn(l, q), 0, st, lds);
     }
-    if (last) {
-      wg_ew(n, T2, 0, zero, SR, make_double2(-fR, 0), sL(l), one, SR, make_double2(fR, 0));
-      es.D1 = T2;
-    }
-    wg_gemm<T>(n, OP_N, Dd, OP_N, gn(l - 1), T1, 0, st, lds);  // d g<_{l-1}
-    wg_gemm<T>(n, OP_N, T1, OP_C, Dd, T2, 0, es, lds);         // + Sigma^< + V - V^H
-    wg_gemm<T>(n, OP_N, gg, OP_N, T2, T0, 0, st, lds);
-    wg_gemm<T>(n, OP_N, T0, OP_C, gg, gng, 0, st, lds);
   }
 
   // ---- last slab outputs and tr
@@ -137,6 +152,7 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
   }
   if (a.ldos) wg_ew(n, ob(a.ldos, L1), 0, zero, G, one, nullptr, one, nullptr, one);
   if (a.ndens) wg_ew(n, ob(a.ndens, L1), 0, zero, Gn, one, nullptr, one, nullptr, one);
+  if (a.ndens2) wg_ew(n, ob(a.ndens2, L1), 0, zero, Gn2, one, nullptr, one, nullptr, one);
   if (a.pdens) wg_ew(n, ob(a.pdens, L1), 0, zero, Gp, one, nullptr, one, nullptr, one);
   if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (lead) a.dens_n[(size_t)e * nx + L1] = v; }
   if (a.dens_p) { double v = wg_imtrace(n, Gp, red); if (lead) a.dens_p[(size_t)e * nx + L1] = -v; }
@@ -144,6 +160,8 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
   refresh(sL(L1), Gn);
 
   // ---- backward sweep
+  // G^<_{l,l+1} is formed where an output or a refresh takes it
+  const bool want_nn = a.GLi1 || a.GGi1 || a.cur || (a.scba && a.sigL_up);
   const bool want_lo = a.GGi1 || a.GRi1_lo || (a.scba && a.sigR_lo);
   for (int l = N - 2; l >= 0; --l) {
     const double2* s = sLup(l + 1);
@@ -155,13 +173,13 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
       wg_gemm<T>(n, OP_N, T0, OP_N, g(l), Glo, 0, st, lds);     // G_{l+1,l}
     }
     wg_gemm<T>(n, OP_N, Q, OP_N, Gn, QGn, 0, st, lds);          // Q G<
-    Epi em = epi_store();
-    if (s) {
-      wg_gemm<T>(n, OP_N, g(l), OP_N, s, gs, 0, st, lds);       // g s
-      em.D1 = gs;
+    if (s) wg_gemm<T>(n, OP_N, g(l), OP_N, s, gs, 0, st, lds);  // g s
+    if (want_nn) {
+      Epi em = epi_store();
+      if (s) em.D1 = gs;
+      wg_gemm<T>(n, OP_N, gn(l), OP_C, Dd, M, 0, em, lds);      // g< d^H + g s
+      wg_gemm<T>(n, OP_N, M, OP_C, G, Gnn, 0, acc(QGn), lds);   // G<_{l,l+1}
     }
-    wg_gemm<T>(n, OP_N, gn(l), OP_C, Dd, M, 0, em, lds);        // g< d^H + g s
-    wg_gemm<T>(n, OP_N, M, OP_C, G, Gnn, 0, acc(QGn), lds);     // G<_{l,l+1}
     if (a.GRi1) wg_ew(n, ob(a.GRi1, l), 0, zero, R, one, nullptr, one, nullptr, one);
     if (a.GLi1) wg_ew(n, ob(a.GLi1, l), 0, zero, Gnn, one, nullptr, one, nullptr, one);
     if (a.GGi1) wg_ew(n, ob(a.GGi1, l), 0, zero, Gnn, one, R, one, Glo, mone);
@@ -178,13 +196,22 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
     refresh(s, Gnn);
     wg_gemm<T>(n, OP_N, R, OP_N, Dd, Rd, 0, st, lds);           // R d
     wg_gemm<T>(n, OP_N, Rd, OP_N, g(l), G, 0, acc(g(l)), lds);  // G_ll = g + R d g
-    wg_gemm<T>(n, OP_N, QGn, OP_C, Q, T0, 0, acc(gn(l)), lds);  // g< + Q G< Q^H
-    wg_gemm<T>(n, OP_N, Rd, OP_N, gn(l), Z, 0, st, lds);        // Z = R d g<
-    if (s) wg_gemm<T>(n, OP_N, gs, OP_C, R, W1, 0, acc(Z), lds);  // Z + g s R^H
-    const double2* ZY = s ? W1 : Z;
-    wg_ew(n, Gn, 0, zero, T0, one, ZY, one, ZY, mone);          // G<_ll
+    for (int q = 0; q < nsrc; ++q) {
+      const double2* sq = sLup(l + 1, q);
+      if (q) {
+        wg_gemm<T>(n, OP_N, Q, OP_N, Gn2, QGn, 0, st, lds);
+        if (sq) wg_gemm<T>(n, OP_N, g(l), OP_N, sq, gs, 0, st, lds);
+      }
+      wg_gemm<T>(n, OP_N, Rd, OP_N, gn(l, q), Z, 0, st, lds);        // Z = R d g<
+      if (sq) wg_gemm<T>(n, OP_N, gs, OP_C, R, W1, 0, acc(Z), lds);  // Z + g s R^H
+      Epi eq = acc(gn(l, q));
+      eq.D2 = sq ? W1 : Z;
+      eq.D3 = eq.D2; eq.s3 = mone;
+      wg_gemm<T>(n, OP_N, QGn, OP_C, Q, Gnq(q), 0, eq, lds);  // G<_ll = g< + Q G< Q^H + (Z + Y) - (Z + Y)^H
+    }
     if (a.ldos) wg_ew(n, ob(a.ldos, l), 0, zero, G, one, nullptr, one, nullptr, one);
     if (a.ndens) wg_ew(n, ob(a.ndens, l), 0, zero, Gn, one, nullptr, one, nullptr, one);
+    if (a.ndens2) wg_ew(n, ob(a.ndens2, l), 0, zero, Gn2, one, nullptr, one, nullptr, one);
     if (a.pdens) wg_ew(n, ob(a.pdens, l), 0, zero, Gn, one, G, one, G, mone);
     if (a.dens_n) { double v = wg_imtrace(n, Gn, red); if (lead) a.dens_n[(size_t)e * nx + l] = v; }
     if (a.dens_p) {

@@ -77,6 +77,10 @@ struct SweepArgs {
   int ckpt;
   // G^R_{l+1,l} per bond (rgf_offdiag.hpp only), or null
   double2* GRi1_lo;
+  // a second lesser source and its G^<_ll (rgf_offdiag.hpp only), or null
+  const double2* sigL2;
+  const double2* sigL2_up;
+  double2* ndens2;
 };
 
 // Workspace blocks of one energy slot: the stored left-connected blocks (all slabs,

@@ -138,7 +138,7 @@ def w_blocks(Vii, V1i, PL, PG, PR, WL=None, WG=None, WR=None, chunk=256):
     with H = 0, z = 0, Sigma^R = -M (diagonal and off-diagonal super-blocks, so A = M and
     the zero edge couplings leave the contacts out) and Sigma^< = S.  Then W^r_ii =
     X_{i,i-1} V_{i-1,i} + X_ii V_ii + X_{i,i+1} V_{i+1,i}, W^<_ii = (X S X^H)_ii, and W^>
-    by a second solve with S = V P^> V^H.  The solve takes Sigma^<_{l,l-1} =
+    with S = V P^> V^H as the solve's second lesser source.  The solve takes Sigma^<_{l,l-1} =
     -(Sigma^<_{l-1,l})^H, so P^< and P^> must be anti-Hermitian, as the polarization step
     makes them (then S is too); P^r and V are general.  Needs 2 nm a multiple of 32,
     at most 256.  Tensors as in w_full; `chunk` energies per solve."""
@@ -220,18 +220,19 @@ def w_blocks(Vii, V1i, PL, PG, PR, WL=None, WG=None, WR=None, chunk=256):
         X = torch.empty(shape, dtype=torch.complex128, device=dev)
         Xu = torch.zeros(shape, dtype=torch.complex128, device=dev)
         Xl = torch.zeros(shape, dtype=torch.complex128, device=dev)
-        for P, Wout, first in ((PL, WL, True), (PG, WG, False)):
-            Sd, Su = lesser_source(pad(P[e0:e1]))
-            Gn = torch.empty(shape, dtype=torch.complex128, device=dev)
-            out = {"ndens": Gn}
-            if first:
-                out.update(ldos=X, GRi1=Xu, GRi1_lo=Xl)
-            rgf.solve_batched(p, E, (300.0, 300.0), (0.0, 0.0), zsup, zsup, sigL=Sd, sigR=sig["sigR"],
-                              sigR_lo=sig["sigR_lo"], sigR_up=sig["sigR_up"], sigL_up=Su, out=out)
+        Sd, Su = lesser_source(pad(PL[e0:e1]))
+        Sd2, Su2 = lesser_source(pad(PG[e0:e1]))
+        Gl, Gg = torch.empty(shape, dtype=torch.complex128, device=dev), torch.empty(shape, dtype=torch.complex128, device=dev)
+        rgf.solve_batched(p, E, (300.0, 300.0), (0.0, 0.0), zsup, zsup, sigL=Sd, sigR=sig["sigR"],
+                          sigR_lo=sig["sigR_lo"], sigR_up=sig["sigR_up"], sigL_up=Su,
+                          out={"ndens": Gl, "ldos": X, "GRi1": Xu, "GRi1_lo": Xl},
+                          second={"sigL": Sd2, "sigL_up": Su2, "ndens": Gg})
+        for Gn, Wout in ((Gl, WL), (Gg, WG)):
             Gt = tm(Gn)
             Wd = torch.stack([Gt[..., :nm, :nm], Gt[..., nm:, nm:]], dim=2).reshape(ce, nx2, nm, nm)
             Wout[e0:e1] = tm(Wd[:, :nx])
-            del Sd, Su, Gn, Gt, Wd
+            del Gt, Wd
+        del Sd, Su, Sd2, Su2, Gl, Gg
         Xt, Xut, Xlt = tm(X), tm(Xu), tm(Xl)
         Wr = torch.zeros((ce, nx2, nm, nm), dtype=torch.complex128, device=dev)
         Vu = H_(V1)

@@ -61,6 +61,10 @@ class Scba(ctypes.Structure):
     _fields_ = [("D", ctypes.c_double), ("mix", ctypes.c_double)]
 
 
+class Lesser(ctypes.Structure):
+    _fields_ = [("sigL", ctypes.c_void_p), ("sigL_up", ctypes.c_void_p), ("ndens", ctypes.c_void_p)]
+
+
 class WBatch(ctypes.Structure):
     _fields_ = [("nm", ctypes.c_int), ("nx", ctypes.c_int), ("nE", ctypes.c_int), ("nbc", ctypes.c_int),
                 ("Vii", ctypes.c_void_p), ("V1i", ctypes.c_void_p), ("PL", ctypes.c_void_p),
@@ -75,7 +79,7 @@ EXPORTS = ("rgf_params_reference", "rgf_last_error", "rgf_version", "rgf_rs", "r
            "rgf_zgemm_batched", "rgf_zinv_batched", "rgf_adjoint_batched", "rgf_adjoint_workspace_bytes",
            "rgf_scba_step", "rgf_graph_create", "rgf_graph_launch", "rgf_graph_destroy", "rgf_solve_devices",
            "rgf_graph_create_devices", "rgf_cms", "rgf_cms_ex", "rgf_cms_energies", "rgf_solve_batched_noalloc",
-           "rgf_integrate", "rgf_w_solve_batched")
+           "rgf_integrate", "rgf_w_solve_batched", "rgf_solve_two_lesser")
 
 _lib = None
 
@@ -97,6 +101,7 @@ def lib():
     L.rgf_rs_energies.argtypes = ([ctypes.POINTER(Params), vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp,
                                    vp, vp, vp, vp, vp, ctypes.c_int] + [vp] * 10)
     L.rgf_solve_batched.argtypes = [ctypes.POINTER(Params), ctypes.POINTER(Batch), vp]
+    L.rgf_solve_two_lesser.argtypes = [ctypes.POINTER(Params), ctypes.POINTER(Batch), ctypes.POINTER(Lesser), vp]
     L.rgf_solve_batched_noalloc.argtypes = [ctypes.POINTER(Params), ctypes.POINTER(Batch), vp]
     L.rgf_integrate.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, vp, vp, vp, ctypes.c_double,
                                 vp, vp, vp, vp]
@@ -279,7 +284,7 @@ def plain_lib():
 
 
 def solve_batched(p, E, temp, mu, Hii, H1i, sigL=None, sigR=None, out=None, max_slots=0, stream=None,
-                  plain=False, sigR_lo=None, sigR_up=None, sigL_up=None, scba=None, ckpt=0):
+                  plain=False, sigR_lo=None, sigR_up=None, sigL_up=None, scba=None, ckpt=0, second=None):
     """Device-resident batched solve (plain=True: the per-energy rocBLAS/rocSOLVER
     comparison path with the same arguments).  E, Hii, H1i, sig*, out[...] are torch
     tensors on the HIP device: complex blocks as complex128 tensors of shape
@@ -290,8 +295,9 @@ def solve_batched(p, E, temp, mu, Hii, H1i, sigL=None, sigR=None, out=None, max_
     Sigma blocks (physical mode).  scba=(D, mix): one SCBA iteration that also
     refreshes the given Sigma tensors in place (rgf_scba_step).  ckpt: storage of
     the left-connected blocks (rgf_batch.ckpt: -1 every slab, K > 0 checkpoints every
-    K slabs with segment recompute, 0 automatic).  Asynchronous on `stream`
-    (default: torch's current stream)."""
+    K slabs with segment recompute, 0 automatic).  second: dict sigL, sigL_up, ndens of
+    a second lesser source carried along (rgf_solve_two_lesser; physical mode, Sigma per
+    energy as the others).  Asynchronous on `stream` (default: torch's current stream)."""
     import torch
     out = out or {}
     b = _batch(torch, E, temp, mu, Hii, H1i, sigL, sigR, max_slots, sigR_lo, sigR_up, sigL_up)
@@ -304,7 +310,17 @@ def solve_batched(p, E, temp, mu, Hii, H1i, sigL=None, sigR=None, out=None, max_
         if rc != 0:
             raise RgfError(f"plain path error {rc}: {plain_lib().rgf_plain_last_error().decode()}")
         return out
-    if scba is not None:
+    if second is not None:
+        if scba is not None:
+            raise RgfError("second: the SCBA refresh takes one lesser source")
+        blk = b.nx * b.nm * b.nm
+        need = blk + b.sig_stride * (b.nE - 1)
+        sec = Lesser(_req(second.get("sigL"), "second sigL", torch.complex128, need, E.device),
+                     _req(second.get("sigL_up"), "second sigL_up", torch.complex128, need, E.device),
+                     _req(second["ndens"], "second ndens", torch.complex128, blk * b.nE, E.device))
+        rc = lib().rgf_solve_two_lesser(ctypes.byref(p), ctypes.byref(b), ctypes.byref(sec),
+                                        ctypes.c_void_p(stream.cuda_stream))
+    elif scba is not None:
         sc = Scba(float(scba[0]), float(scba[1]))
         rc = lib().rgf_scba_step(ctypes.byref(p), ctypes.byref(b), ctypes.byref(sc), ctypes.c_void_p(stream.cuda_stream))
     else:
