@@ -5,18 +5,20 @@
 //
 // Work per band element is a 1D correlation of length nen: O(nen^2) FP64 FMAs against
 // O(nen) data, so one workgroup takes one element, stages its energy series in LDS
-// and runs the correlation from LDS at the FP64 FMA rate.  The reference zeroes the
-// real parts of G before this step (src/green_rgf.f90:3186-3188), so the G series are
+// and runs the correlation as Toeplitz products on the matrix cores.  The reference zeroes
+// the real parts of G before this step (src/green_rgf.f90:3186-3188), so the G series are
 // real (their imaginary parts): P^< = dE_P * (-sum a d) etc. are sums of real
 // products, Sigma sums real G times complex W.
 //
-// Lane mapping: each lane owns R = 4 consecutive outputs and slides an R-value register window along the shifted ("Y") series,
-// so one LDS read per series and step feeds R outputs; the other series ("X") is read
-// at the same address by the whole wave (broadcast).  The Y series are stored
-// zero-padded and R-way de-interleaved (padded index p at (p % R) * Q + p / R), so the
-// lanes' reads, R elements apart, fall on consecutive words.  Zero padding also takes
-// the place of every index bound of the reference's loops: a term outside them reads
-// a zero.
+// 256 consecutive outputs n = n0 + 16 u + v form a 16 x 16 tile D[v][u]: with a step m the
+// sum over energies is sum_m X[v][m] Y[m][u], where X is a series at m -+ v and Y one at
+// 16 u +- m, so a 16x16x4 FP64 MFMA does 1024 terms of one product for two 8-byte LDS
+// reads per lane.  (On the vector units, 4 outputs to a lane in a sliding window, the LDS
+// reads set the pace: 39% and 47% of the FP64 rate, P and Sigma, 32-orbital full band, 2000
+// energies.)  The series are zero-padded: a term outside the reference's index bounds reads
+// a zero.  The Y series skip one word after every 16 (lanes 16 apart would fall on two banks).
+// The steps of all tiles are dealt evenly to the workgroup's waves; where several waves
+// share a tile their partial sums are added in the waves' order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,14 +44,48 @@ int fail(int code, const std::string& msg) {
     if (e_ != hipSuccess) return fail(2, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// polarization: 8 waves x 64 lanes x 4 outputs = 2048 outputs per pass (two waves per SIMD)
-constexpr int NTH_P = 512, RP = 4, SP = 64 * RP;
-constexpr int PADP = SP;   // a wave's window reaches SP - 1 below its first output's series start
-// self-energy: 8 waves x 64 lanes x 4 outputs = 2048 outputs per pass (two waves per SIMD)
-constexpr int NTH_S = 512, RS = 4, SS_ = 64 * RS;
-constexpr int PADY = 260;  // zero padding of a self-energy Y series on each side (reach 258)
+constexpr int kPadX = 32;   // zero padding of an X series on each side (reach 30)
+constexpr int kPadY = 256;  // zero padding of a Y series on each side (reach 255)
 // largest nen of the direct forms (an element's series live in LDS)
 constexpr int kPolDirectMax = 3072, kSigDirectMax = 2040;
+
+constexpr int kLdsCu = 160 * 1024;
+constexpr int kMaxWaves = 16;  // 12 tiles at the longest series
+
+// What one wave of a workgroup computes: blocks c0 .. c1 - 1 of 16 steps of a tile of 256
+// outputs, as part `part` of `parts`.  Part p > 0 leaves its sums at slot, part 0 adds
+// those at slot .. slot + parts - 2.  part = -1: nothing.
+struct WaveShare {
+  int tile, c0, c1, part, parts, slot;
+};
+
+// Steps m of a tile: blocks of 16 from m0 (a multiple of 16).
+struct Steps {
+  int m0, blocks;
+};
+
+__host__ __device__ inline Steps steps(int lo, int hi) {  // lo <= m < hi
+  const int m0 = lo & ~15;
+  return {m0, hi > m0 ? (hi - m0 + 15) / 16 : 0};
+}
+
+// polarization, nop = nlo + 16 u + v: X at m - v, Y at m + 16 u + nlo, both in 0 .. nen - 1
+__host__ __device__ inline Steps pol_steps(int nen, int nopmax, int tile) {
+  const int nlo = 256 * tile - nopmax;
+  return steps(nlo < -240 ? -nlo - 240 : 0, nlo < -15 ? nen + 15 : nen - nlo);
+}
+
+// self-energy, E = e0 + 16 u + v: X (frequencies) at m + v in -nopmax .. nopmax, Y at
+// e0 + 16 u - m in 0 .. nen - 2
+__host__ __device__ inline Steps sig_steps(int nen, int nopmax, int tile) {
+  const int e0 = 256 * tile;
+  const int lo = e0 - (nen - 2), hi = e0 + 240;
+  return steps(lo > -nopmax - 15 ? lo : -nopmax - 15, (hi < nopmax ? hi : nopmax) + 1);
+}
+
+// words of a padded Y series
+__host__ __device__ inline int pol_series(int nen) { return (nen + 527) / 16 + nen + 528; }
+__host__ __device__ inline int sig_series(int nen) { return (nen + 510) / 16 + nen + 511; }
 
 struct GwArgs {
   int nm, nx, nen, nd, nopmax, half;  // nd = min(ndiag, nm - 1), half = nen / 2
@@ -68,6 +104,8 @@ struct GwArgs {
   double* Og;
   double* Or;
   double* X;   // polarization: Im G^<, Im G^>, Im G^r of every band element, energy-contiguous
+  int slots;   // partial tiles of the waves
+  WaveShare share[kMaxWaves];
 };
 
 // Index (in series of nen doubles) of series s (0: G^<, 1: G^>, 2: G^r) of band element
@@ -111,9 +149,6 @@ __global__ __launch_bounds__(256) void k_pol_gather(GwArgs a) {
   }
 }
 
-template <int R>
-__device__ __forceinline__ int dpos(int p, int q) { return (p % R) * q + p / R; }  // p >= 0, R a power of 2
-
 // Element (i, j, slab) of a workgroup.  Logical block b = (slab' * nm + j) * (2 nd + 1) +
 // (i - j + nd): consecutive blocks are consecutive rows i of one column j, whose energy
 // series are adjacent in memory.  Workgroups are dealt round-robin to the 8 XCDs (each
@@ -146,320 +181,286 @@ __device__ __forceinline__ bool element(const GwArgs& a, int& i, int& j, int& ix
   return i >= 0 && i < a.nm;
 }
 
-template <int NENMAX>
-struct PolLds {
-  static constexpr int XL = NENMAX + RP;                              // X read up to nen + RP - 2
-  static constexpr int YL = (NENMAX + PADP + SP + RP + RP - 1) / RP * RP;  // Y index up to nen + SP + RP - 3
-  static constexpr int DOUBLES = 3 * XL + 3 * YL;
-};
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ v4d mfma(double x, double y, v4d c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, c, 0, 0, 0);
+}
+
+// Position in a padded Y series: one word skipped after every 16.
+__device__ __forceinline__ int skew(int p) { return p + (p >> 4); }
+
+// Sums `n` partial tiles of a tile's other waves (in the order of the waves) into acc.
+template <int K>
+__device__ __forceinline__ void add_partials(v4d (&acc)[K], const double* slots, int n, int lane) {
+  for (int q = 0; q < n; ++q)
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[k][r] += slots[((q * K + k) * 4 + r) * 64 + lane];
+}
+
+template <int K>
+__device__ __forceinline__ void put_partials(const v4d (&acc)[K], double* slot, int lane) {
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) slot[(k * 4 + r) * 64 + lane] = acc[k][r];
+}
 
 // P^<_ij(w) = dE_P sum_E G^<_ij(E) G^>_ji(E-w), P^>_ij(w) = dE_P sum_E G^>_ij(E) G^<_ji(E-w),
 // P^r_ij(w) = dE_P sum_E [G^<_ij(E) conj(G^r_ij(E-w)) + G^r_ij(E) G^<_ji(E-w)]
 // (src/green_rgf.f90:3199-3218).  With G = i g: G^< G^> = -a d, G^< conj(G^r) +
-// G^r G^<_ji = a f - c e (a, b, c = g^<_ij, g^>_ij, g^r_ij; d, e = g^>_ji, g^<_ji; f = c).
-template <int NENMAX>
-__global__ __launch_bounds__(NTH_P) void k_polarization(GwArgs a) {
-  using L = PolLds<NENMAX>;
-  __shared__ double lds[L::DOUBLES];
+// G^r G^<_ji = a c - c e (a, c = g^<_ij, g^r_ij; d, e = g^>_ji, g^<_ji).  The sum of
+// P^>_ji(-w) has the terms of P^<_ij(w), so the workgroup of ij writes both and three
+// products are left of four.
+// Output tile t: n = nlo + 16 u + v.  X = the ji series (and c) at m - v, Y = a and -c at
+// m + 16 u + nlo, m over the steps that reach both.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_polarization(GwArgs a) {
+  extern __shared__ double lds[];
+  constexpr int NTH = 64 * NW;
   int i, j, ix;
   if (!element(a, i, j, ix)) return;  // uniform over the workgroup, before any barrier
   const int nen = a.nen, tid = threadIdx.x;
   const size_t ES = (size_t)a.nm * a.nm * a.nx;  // energy stride (complex elements)
   const size_t eij = (size_t)i + (size_t)a.nm * j + (size_t)a.nm * a.nm * ix;
   const size_t eji = (size_t)j + (size_t)a.nm * i + (size_t)a.nm * a.nm * ix;
-  // dense bands: the series of ij and ji come gathered (energy-contiguous); else strided
-  const double* xij = a.X ? a.X + xseries(a, i, j, ix, 0) * nen : nullptr;
-  const double* xji = a.X ? a.X + xseries(a, j, i, ix, 0) * nen : nullptr;
-  double* xa = lds;
-  double* xb = xa + L::XL;
-  double* xc = xb + L::XL;
-  double* yd = xc + L::XL;
-  double* ye = yd + L::YL;
-  double* yf = ye + L::YL;
-  constexpr int Q = L::YL / RP;
-  // staging: every load of a thread is issued before its LDS stores (one HBM latency
-  // per group instead of one per energy block)
+  const int xl = nen + 2 * kPadX, yl = pol_series(nen), sh = kPadY + (a.nopmax & 15);
+  double* xd = lds;
+  double* xe = xd + xl;
+  double* xf = xe + xl;
+  double* ya = xf + xl;
+  double* yc = ya + yl;
   {
-    constexpr int NI = (L::XL + NTH_P - 1) / NTH_P;
-    double va[NI], vb[NI], vc[NI];
+    // dense bands: the series of ij and ji come gathered (energy-contiguous); else strided
+    const size_t st = a.X ? 1 : 2 * ES;
+    const double* pa = a.X ? a.X + xseries(a, i, j, ix, 0) * nen : a.Gl + 2 * eij + 1;
+    const double* pc = a.X ? a.X + xseries(a, i, j, ix, 2) * nen : a.Gr + 2 * eij + 1;
+    const double* pd = a.X ? a.X + xseries(a, j, i, ix, 1) * nen : a.Gg + 2 * eji + 1;
+    const double* pe = a.X ? a.X + xseries(a, j, i, ix, 0) * nen : a.Gl + 2 * eji + 1;
+    // the loads of two positions are issued before their LDS stores
+    for (int p0 = tid; p0 < nen; p0 += 2 * NTH) {
+      double va[2], vc[2], vd[2], ve[2];
 #pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int p = tid + u * NTH_P;
-      va[u] = vb[u] = vc[u] = 0.0;
-      if (p < nen) {
-        if (xij) {
-          va[u] = xij[p];
-          vb[u] = xij[nen + p];
-          vc[u] = xij[2 * nen + p];
-        } else {
-          va[u] = a.Gl[2 * (eij + ES * p) + 1];
-          vb[u] = a.Gg[2 * (eij + ES * p) + 1];
-          vc[u] = a.Gr[2 * (eij + ES * p) + 1];
+      for (int q = 0; q < 2; ++q) {
+        const size_t o = st * (size_t)min(p0 + q * NTH, nen - 1);
+        va[q] = pa[o]; vc[q] = pc[o]; vd[q] = pd[o]; ve[q] = pe[o];
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int p = p0 + q * NTH;
+        if (p < nen) {
+          xd[p + kPadX] = vd[q];
+          xe[p + kPadX] = ve[q];
+          xf[p + kPadX] = vc[q];
+          ya[skew(p + sh)] = va[q];
+          yc[skew(p + sh)] = -vc[q];
         }
       }
     }
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int p = tid + u * NTH_P;
-      if (p < L::XL) {
-        xa[p] = va[u];
-        xb[p] = vb[u];
-        xc[p] = vc[u];
-      }
+    for (int p = tid; p < 2 * kPadX; p += NTH) {
+      const int q = p < kPadX ? p : nen + p;
+      xd[q] = xe[q] = xf[q] = 0.0;
+    }
+    for (int p = tid; p < 2 * kPadY + 16; p += NTH) {
+      const int q = p < sh ? p : nen + p;
+      ya[skew(q)] = yc[skew(q)] = 0.0;
     }
   }
-  {
-    constexpr int NI = (L::YL + NTH_P - 1) / NTH_P;
-    double vd[NI], ve[NI];
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int k = tid + u * NTH_P - PADP;
-      vd[u] = ve[u] = 0.0;
-      if (k >= 0 && k < nen) {
-        if (xji) {
-          vd[u] = xji[nen + k];
-          ve[u] = xji[k];
-        } else {
-          vd[u] = a.Gg[2 * (eji + ES * k) + 1];
-          ve[u] = a.Gl[2 * (eji + ES * k) + 1];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int p = tid + u * NTH_P;
-      if (p < L::YL) {
-        const int q = dpos<RP>(p, Q);
-        yd[q] = vd[u];
-        ye[q] = ve[u];
-      }
-    }
-  }
-  __syncthreads();
-  for (int p = tid; p < L::YL; p += NTH_P) {  // the shifted copy of g^r_ij comes from LDS
-    const int k = p - PADP;
-    yf[dpos<RP>(p, Q)] = (k >= 0 && k < nen) ? xc[k] : 0.0;
-  }
-  __syncthreads();
   const int nout = 2 * a.nopmax + 1;
   const int lo_iop = a.half - 1 - a.nopmax;  // 0-based energy index of nop = -nopmax
   // indices outside the frequency window hold zero (the reference zeroes P first)
-  for (int p = tid; p < nen; p += NTH_P) {
+  for (int p = tid; p < nen; p += NTH) {
     if (p < lo_iop || p >= lo_iop + nout) {
-      const size_t o = 2 * (eij + ES * p);
-      a.Ol[o] = 0.0; a.Ol[o + 1] = 0.0;
-      a.Og[o] = 0.0; a.Og[o + 1] = 0.0;
-      a.Or[o] = 0.0; a.Or[o + 1] = 0.0;
+      const size_t o = eij + ES * p;
+      reinterpret_cast<double2*>(a.Ol)[o] = make_double2(0, 0);
+      reinterpret_cast<double2*>(a.Og)[o] = make_double2(0, 0);
+      reinterpret_cast<double2*>(a.Or)[o] = make_double2(0, 0);
     }
   }
-  const int wave = tid >> 6, lane = tid & 63;
-  for (int ow = SP * wave; ow < nout; ow += (NTH_P / 64) * SP) {
-    const int nop_lo = ow - a.nopmax;
-    const int nop_hi = min(ow + SP - 1, nout - 1) - a.nopmax;
-    const int elo = max(nop_lo, 0);                 // union over the wave of the
-    const int ehi = min(nen - 1, nen - 1 + nop_hi); // valid energies of its outputs
-    const int nb = nop_lo + RP * lane;              // this lane's outputs: nop = nb .. nb+RP-1
-    double rd[RP], re[RP], rf[RP];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const WaveShare w = a.share[wave];
+  v4d acc[2] = {};  // a d, a c - c e
+  {
+    const Steps st = pol_steps(nen, a.nopmax, w.tile);
+    const int u = lane & 15, kk = lane >> 4;
+    const int px = st.m0 + 16 * w.c0 + kk - u + kPadX;
+    const int py = 17 * ((st.m0 + 256 * w.tile - a.nopmax + sh) / 16 + u + w.c0) + kk;
+    const double *d = xd + px, *e = xe + px, *f = xf + px, *ra = ya + py, *rc = yc + py;
+    for (int c = w.c0; c < w.c1; ++c) {
 #pragma unroll
-    for (int s = 1; s < RP; ++s) {  // slots of energies elo-1 .. elo-RP+1
-      const int q = dpos<RP>(elo - s - nb + PADP, Q);
-      rd[RP - s] = yd[q];
-      re[RP - s] = ye[q];
-      rf[RP - s] = yf[q];
-    }
-    // Y(e + s - nb) for e = elo + RP it sits at off[s] + it (the residue mod RP of the
-    // padded index is fixed per s, its quotient grows by one per iteration)
-    int off[RP];
-#pragma unroll
-    for (int s = 0; s < RP; ++s) off[s] = dpos<RP>(elo + s - nb + PADP, Q);
-    double sl[RP], sg[RP], sr[RP];
-#pragma unroll
-    for (int r = 0; r < RP; ++r) sl[r] = sg[r] = sr[r] = 0.0;
-    for (int e = elo, it = 0; e <= ehi; e += RP, ++it) {
-#pragma unroll
-      for (int s = 0; s < RP; ++s) {
-        const int m = e + s;
-        rd[s] = yd[off[s] + it];
-        re[s] = ye[off[s] + it];
-        rf[s] = yf[off[s] + it];
-        const double va = xa[m], vb = xb[m], vc = xc[m];
-#pragma unroll
-        for (int r = 0; r < RP; ++r) {  // output nb + r reads Y(m - nb - r), slot (s - r) mod RP
-          const int q = (s - r) & (RP - 1);
-          sl[r] = fma(va, rd[q], sl[r]);
-          sg[r] = fma(vb, re[q], sg[r]);
-          sr[r] = fma(va, rf[q], sr[r]);
-          sr[r] = fma(-vc, re[q], sr[r]);
-        }
+      for (int s = 0; s < 16; s += 4) {
+        const double va = ra[s], vc = rc[s];
+        acc[0] = mfma(d[s], va, acc[0]);
+        acc[1] = mfma(f[s], va, acc[1]);
+        acc[1] = mfma(e[s], vc, acc[1]);
       }
+      d += 16; e += 16; f += 16; ra += 17; rc += 17;
     }
+  }
+  if (a.slots) {  // the partial sums take the place of the series
+    __syncthreads();
+    if (w.part > 0) put_partials(acc, lds + (size_t)w.slot * 2 * 256, lane);
+    __syncthreads();
+  }
+  if (w.part != 0) return;
+  add_partials(acc, lds + (size_t)w.slot * 2 * 256, w.parts - 1, lane);
 #pragma unroll
-    for (int r = 0; r < RP; ++r) {
-      const int o = ow + RP * lane + r;
-      if (o < nout) {
-        const size_t w = 2 * (eij + ES * (size_t)(lo_iop + o));
-        a.Ol[w] = -sl[r] * a.dr; a.Ol[w + 1] = -sl[r] * a.di;
-        a.Og[w] = -sg[r] * a.dr; a.Og[w + 1] = -sg[r] * a.di;
-        a.Or[w] = sr[r] * a.dr;  a.Or[w + 1] = sr[r] * a.di;
-      }
+  for (int r = 0; r < 4; ++r) {
+    const int o = 256 * w.tile + 16 * (lane & 15) + 4 * r + (lane >> 4);
+    if (o < nout) {
+      const double sl = acc[0][r], sr = acc[1][r];
+      const size_t q = eij + ES * (size_t)(lo_iop + o), qg = eji + ES * (size_t)(lo_iop + 2 * a.nopmax - o);
+      reinterpret_cast<double2*>(a.Ol)[q] = make_double2(-sl * a.dr, -sl * a.di);
+      reinterpret_cast<double2*>(a.Og)[qg] = make_double2(-sl * a.dr, -sl * a.di);
+      reinterpret_cast<double2*>(a.Or)[q] = make_double2(sr * a.dr, sr * a.di);
     }
   }
 }
 
-template <int NENMAX>
-struct SigLds {
-  static constexpr int WL = NENMAX + 4;  // W over o = nop + nopmax (nout <= nen - 1), zero tail
-  static constexpr int YL = (NENMAX + 2 * PADY + 3) / 4 * 4;
-  static constexpr int DOUBLES = 3 * 2 * WL + 3 * YL;
-};
-
 // Sigma_new^x(E) = dE_S sum_w G^x(E-w) W^x(w) over the reference's terms (E_ie with
 // ie > max(nop, 1) and ie < nen + nop: G's index ie - nop in 1..nen-1, output ie = 1
 // empty), Im Sigma_new^r = Im(Sigma_new^> - Sigma_new^<)/2, mixing and edge copy
-// (src/green_rgf.f90:3247-3290).  With G = i g: (i g) W = (-g Im W, g Re W).
-template <int NENMAX>
-__global__ __launch_bounds__(NTH_S) void k_selfenergy(GwArgs a) {
-  using L = SigLds<NENMAX>;
-  __shared__ double lds[L::DOUBLES];
+// (src/green_rgf.f90:3247-3290).  With G = i g: dE_S (i g) W = g (t + i s), t and s the
+// parts of i dE_S W, staged in W's place; of Sigma^r = dE_S sum [G^< W^r + G^r (W^< + W^r)]
+// only the real part g^< t^r + g^r (t^< + t^r) is wanted, so t^r alone is staged: six
+// products.
+// Output tile t: E = 256 t + 16 u + v.  X = t, s at m + v, Y = g at 256 t + 16 u - m.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_selfenergy(GwArgs a) {
+  extern __shared__ double lds[];
+  constexpr int NTH = 64 * NW;
   int i, j, ix;
   if (!element(a, i, j, ix)) return;
   const int nen = a.nen, tid = threadIdx.x;
   const size_t ES = (size_t)a.nm * a.nm * a.nx;
   const size_t SS = (size_t)a.nm * a.nm;  // slab stride
   const size_t eij = (size_t)i + (size_t)a.nm * j + SS * ix;
-  double* wl = lds;
-  double* wg = wl + 2 * L::WL;
-  double* wr = wg + 2 * L::WL;
-  double* yl = wr + 2 * L::WL;
-  double* yg = yl + L::YL;
-  double* yr = yg + L::YL;
-  constexpr int Q = L::YL / 4;
   const int nout = 2 * a.nopmax + 1;
   const int lo_iop = a.half - 1 - a.nopmax;
-  {  // staging: every load of a thread is issued before its LDS stores
-    constexpr int NI = (L::WL + NTH_S - 1) / NTH_S;
-    double2 vl[NI], vg[NI], vr[NI];
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int p = tid + u * NTH_S;
-      vl[u] = vg[u] = vr[u] = make_double2(0, 0);
-      if (p < nout) {
-        const size_t o = eij + ES * (size_t)(lo_iop + p);
-        vl[u] = reinterpret_cast<const double2*>(a.Wl)[o];
-        vg[u] = reinterpret_cast<const double2*>(a.Wg)[o];
-        vr[u] = reinterpret_cast<const double2*>(a.Wr)[o];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int p = tid + u * NTH_S;
-      if (p < L::WL) {
-        wl[2 * p] = vl[u].x; wl[2 * p + 1] = vl[u].y;
-        wg[2 * p] = vg[u].x; wg[2 * p + 1] = vg[u].y;
-        wr[2 * p] = vr[u].x; wr[2 * p + 1] = vr[u].y;
-      }
-    }
-  }
+  const int xl = nout + 2 * kPadX, yl = sig_series(nen);
+  double* xtl = lds;
+  double* xsl = xtl + xl;
+  double* xtg = xsl + xl;
+  double* xsg = xtg + xl;
+  double* xtr = xsg + xl;
+  double* yl_ = xtr + xl;
+  double* yg_ = yl_ + yl;
+  double* yr_ = yg_ + yl;
   {
-    constexpr int NI = (L::YL + NTH_S - 1) / NTH_S;
-    double vl[NI], vg[NI], vr[NI];
+    const double2* Wl = reinterpret_cast<const double2*>(a.Wl) + eij + ES * (size_t)lo_iop;
+    const double2* Wg = reinterpret_cast<const double2*>(a.Wg) + eij + ES * (size_t)lo_iop;
+    const double2* Wr = reinterpret_cast<const double2*>(a.Wr) + eij + ES * (size_t)lo_iop;
+    // the loads of two positions are issued before their LDS stores
+    for (int p0 = tid; p0 < nout; p0 += 2 * NTH) {
+      double2 vl[2], vg[2], vr[2];
 #pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int k = tid + u * NTH_S - PADY;
-      vl[u] = vg[u] = vr[u] = 0.0;
-      if (k >= 0 && k < nen - 1) {  // the last energy of G never enters
-        vl[u] = a.Gl[2 * (eij + ES * k) + 1];
-        vg[u] = a.Gg[2 * (eij + ES * k) + 1];
-        vr[u] = a.Gr[2 * (eij + ES * k) + 1];
+      for (int q = 0; q < 2; ++q) {
+        const size_t o = ES * (size_t)min(p0 + q * NTH, nout - 1);
+        vl[q] = Wl[o]; vg[q] = Wg[o]; vr[q] = Wr[o];
       }
-    }
 #pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int p = tid + u * NTH_S;
-      if (p < L::YL) {
-        const int q = dpos<RS>(p, Q);
-        yl[q] = vl[u];
-        yg[q] = vg[u];
-        yr[q] = vr[u];
-      }
-    }
-  }
-  __syncthreads();
-  const int wave = tid >> 6, lane = tid & 63;
-  const int last = a.nx - 3;
-  for (int ew = SS_ * wave; ew < nen; ew += 8 * SS_) {
-    const int e_hi = min(ew + SS_ - 1, nen - 1);
-    const int nlo = max(-a.nopmax, ew - (nen - 2));
-    const int nhi = min(a.nopmax, e_hi);
-    const int eb = ew + 4 * lane;  // this lane's outputs: e = eb .. eb+3
-    const int c = eb - nlo;        // step t reads G(c - t)
-    double gl[4], gg[4], gr[4];
-#pragma unroll
-    for (int s = 1; s < 4; ++s) {  // slots of steps -1, -2, -3: G(c+1), G(c+2), G(c+3)
-      const int q = dpos<RS>(c + s + PADY, Q);
-      gl[4 - s] = yl[q];
-      gg[4 - s] = yg[q];
-      gr[4 - s] = yr[q];
-    }
-    // G(c - t) for t = 4 it + s sits at off[s] - it
-    int off[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) off[s] = dpos<RS>(c - s + PADY, Q);
-    double lr[4] = {0, 0, 0, 0}, li[4] = {0, 0, 0, 0}, gre[4] = {0, 0, 0, 0}, gim[4] = {0, 0, 0, 0};
-    double rr[4] = {0, 0, 0, 0}, ri[4] = {0, 0, 0, 0};
-    for (int t0 = 0, it = 0; t0 <= nhi - nlo; t0 += 4, ++it) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int o = nlo + t0 + s + a.nopmax;  // W index of nop = nlo + t0 + s
-        gl[s] = yl[off[s] - it];
-        gg[s] = yg[off[s] - it];
-        gr[s] = yr[off[s] - it];
-        const double wlr = wl[2 * o], wli = wl[2 * o + 1];
-        const double wgr = wg[2 * o], wgi = wg[2 * o + 1];
-        const double wrr = wr[2 * o], wri = wr[2 * o + 1];
-        const double wsr = wlr + wrr, wsi = wli + wri;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {  // output eb + r reads G(c + r - t), slot (s - r) & 3
-          const int q = (s - r) & 3;
-          lr[r] = fma(-gl[q], wli, lr[r]);
-          li[r] = fma(gl[q], wlr, li[r]);
-          gre[r] = fma(-gg[q], wgi, gre[r]);
-          gim[r] = fma(gg[q], wgr, gim[r]);
-          rr[r] = fma(-gl[q], wri, rr[r]);
-          rr[r] = fma(-gr[q], wsi, rr[r]);
-          ri[r] = fma(gl[q], wrr, ri[r]);
-          ri[r] = fma(gr[q], wsr, ri[r]);
+      for (int q = 0; q < 2; ++q) {
+        const int p = p0 + q * NTH;
+        if (p < nout) {
+          xtl[p + kPadX] = -vl[q].y * a.dr - vl[q].x * a.di;
+          xsl[p + kPadX] = vl[q].x * a.dr - vl[q].y * a.di;
+          xtg[p + kPadX] = -vg[q].y * a.dr - vg[q].x * a.di;
+          xsg[p + kPadX] = vg[q].x * a.dr - vg[q].y * a.di;
+          xtr[p + kPadX] = -vr[q].y * a.dr - vr[q].x * a.di;
         }
       }
     }
+    for (int p = tid; p < 2 * kPadX; p += NTH) {
+      const int q = p < kPadX ? p : nout + p;
+      xtl[q] = xsl[q] = xtg[q] = xsg[q] = xtr[q] = 0.0;
+    }
+    const double* Gl = a.Gl + 2 * eij + 1;
+    const double* Gg = a.Gg + 2 * eij + 1;
+    const double* Gr = a.Gr + 2 * eij + 1;
+    for (int p0 = tid; p0 < nen - 1; p0 += 2 * NTH) {  // the last energy of G never enters
+      double vl[2], vg[2], vr[2];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int e = eb + r;
-      if (e >= nen) continue;
-      const bool first = (e == 0);  // ie = 1 has no term
-      const double2 al = first ? make_double2(0, 0) : make_double2(lr[r], li[r]);
-      const double2 ag = first ? make_double2(0, 0) : make_double2(gre[r], gim[r]);
-      const double2 ar = first ? make_double2(0, 0) : make_double2(rr[r], ri[r]);
-      const double2 nl = make_double2(al.x * a.dr - al.y * a.di, al.x * a.di + al.y * a.dr);
-      const double2 ng = make_double2(ag.x * a.dr - ag.y * a.di, ag.x * a.di + ag.y * a.dr);
-      const double2 nr = make_double2(ar.x * a.dr - ar.y * a.di, (ng.y - nl.y) / 2.0);
-      const size_t o = eij + ES * (size_t)e;
-      double2* Sl = reinterpret_cast<double2*>(a.Ol);
-      double2* Sg = reinterpret_cast<double2*>(a.Og);
-      double2* Sr = reinterpret_cast<double2*>(a.Or);
-      const double2 ol = Sl[o], og = Sg[o], orr = Sr[o];
-      const double2 ml = make_double2(ol.x + a.alpha * (nl.x - ol.x), ol.y + a.alpha * (nl.y - ol.y));
-      const double2 mg = make_double2(og.x + a.alpha * (ng.x - og.x), og.y + a.alpha * (ng.y - og.y));
-      const double2 mr = make_double2(orr.x + a.alpha * (nr.x - orr.x), orr.y + a.alpha * (nr.y - orr.y));
-      Sl[o] = ml; Sg[o] = mg; Sr[o] = mr;
-      if (ix == 2) {  // slabs 1-2 (1-based) take slab 3
-        Sl[o - 2 * SS] = ml; Sg[o - 2 * SS] = mg; Sr[o - 2 * SS] = mr;
-        Sl[o - SS] = ml; Sg[o - SS] = mg; Sr[o - SS] = mr;
+      for (int q = 0; q < 2; ++q) {
+        const size_t o = 2 * ES * (size_t)min(p0 + q * NTH, nen - 2);
+        vl[q] = Gl[o]; vg[q] = Gg[o]; vr[q] = Gr[o];
       }
-      if (ix == last) {  // slabs nx-1..nx take slab nx-2
-        Sl[o + SS] = ml; Sg[o + SS] = mg; Sr[o + SS] = mr;
-        Sl[o + 2 * SS] = ml; Sg[o + 2 * SS] = mg; Sr[o + 2 * SS] = mr;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int p = p0 + q * NTH;
+        if (p < nen - 1) {
+          const int k = skew(p + kPadY - 1);
+          yl_[k] = vl[q];
+          yg_[k] = vg[q];
+          yr_[k] = vr[q];
+        }
       }
+    }
+    for (int p = tid; p < 2 * kPadY; p += NTH) {
+      const int k = skew(p < kPadY - 1 ? p : nen - 1 + p);
+      yl_[k] = yg_[k] = yr_[k] = 0.0;
+    }
+  }
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const WaveShare w = a.share[wave];
+  v4d acc[5] = {};  // t^< g^<, s^< g^<, t^> g^>, s^> g^>, Re Sigma^r
+  {
+    const Steps st = sig_steps(nen, a.nopmax, w.tile);
+    const int u = lane & 15, kk = lane >> 4;
+    const int px = st.m0 + 16 * w.c0 + kk + u + a.nopmax + kPadX;
+    const int py = 17 * ((256 * w.tile - st.m0 + kPadY - 16) / 16 + u - w.c0) + 15 - kk;
+    const double *tl = xtl + px, *sl = xsl + px, *tg = xtg + px, *sg = xsg + px, *tr = xtr + px;
+    const double *gl = yl_ + py, *gg = yg_ + py, *gr = yr_ + py;
+    for (int c = w.c0; c < w.c1; ++c) {
+#pragma unroll
+      for (int s = 0; s < 16; s += 4) {
+        const double vl = gl[-s], vg = gg[-s], vr = gr[-s], a0 = tl[s], a4 = tr[s];
+        acc[0] = mfma(a0, vl, acc[0]);
+        acc[1] = mfma(sl[s], vl, acc[1]);
+        acc[2] = mfma(tg[s], vg, acc[2]);
+        acc[3] = mfma(sg[s], vg, acc[3]);
+        acc[4] = mfma(a4, vl, acc[4]);
+        acc[4] = mfma(a0 + a4, vr, acc[4]);
+      }
+      tl += 16; sl += 16; tg += 16; sg += 16; tr += 16;
+      gl -= 17; gg -= 17; gr -= 17;
+    }
+  }
+  if (a.slots) {  // the partial sums take the place of the series
+    __syncthreads();
+    if (w.part > 0) put_partials(acc, lds + (size_t)w.slot * 5 * 256, lane);
+    __syncthreads();
+  }
+  if (w.part != 0) return;
+  add_partials(acc, lds + (size_t)w.slot * 5 * 256, w.parts - 1, lane);
+  const int last = a.nx - 3;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int e = 256 * w.tile + 16 * (lane & 15) + 4 * r + (lane >> 4);
+    if (e >= nen) continue;
+    const bool first = (e == 0);  // ie = 1 has no term
+    const double2 nl = first ? make_double2(0, 0) : make_double2(acc[0][r], acc[1][r]);
+    const double2 ng = first ? make_double2(0, 0) : make_double2(acc[2][r], acc[3][r]);
+    const double2 nr = make_double2(first ? 0.0 : acc[4][r], (ng.y - nl.y) / 2.0);
+    const size_t o = eij + ES * (size_t)e;
+    double2* Sl = reinterpret_cast<double2*>(a.Ol);
+    double2* Sg = reinterpret_cast<double2*>(a.Og);
+    double2* Sr = reinterpret_cast<double2*>(a.Or);
+    const double2 ol = Sl[o], og = Sg[o], orr = Sr[o];
+    const double2 ml = make_double2(ol.x + a.alpha * (nl.x - ol.x), ol.y + a.alpha * (nl.y - ol.y));
+    const double2 mg = make_double2(og.x + a.alpha * (ng.x - og.x), og.y + a.alpha * (ng.y - og.y));
+    const double2 mr = make_double2(orr.x + a.alpha * (nr.x - orr.x), orr.y + a.alpha * (nr.y - orr.y));
+    Sl[o] = ml; Sg[o] = mg; Sr[o] = mr;
+    if (ix == 2) {  // slabs 1-2 (1-based) take slab 3
+      Sl[o - 2 * SS] = ml; Sg[o - 2 * SS] = mg; Sr[o - 2 * SS] = mr;
+      Sl[o - SS] = ml; Sg[o - SS] = mg; Sr[o - SS] = mr;
+    }
+    if (ix == last) {  // slabs nx-1..nx take slab nx-2
+      Sl[o + SS] = ml; Sg[o + SS] = mg; Sr[o + SS] = mr;
+      Sl[o + 2 * SS] = ml; Sg[o + 2 * SS] = mg; Sr[o + 2 * SS] = mr;
     }
   }
 }
@@ -832,6 +833,36 @@ GwArgs args(const gw_params* p) {
   return a;
 }
 
+// Deals the blocks of the ceil(nout / 256) tiles to at most `most` waves: a wave to each
+// tile, then one more to the tile with the most blocks per wave, while the partial tiles
+// (K accumulators each) fit the space of the series.  Returns the waves in use.
+template <bool POL>
+int deal(GwArgs& a, int nout, int most, int K, int series) {
+  const int tiles = (nout + 255) / 256;
+  int blocks[kMaxWaves], parts[kMaxWaves], used = tiles;
+  for (int t = 0; t < tiles; ++t) {
+    blocks[t] = (POL ? pol_steps(a.nen, a.nopmax, t) : sig_steps(a.nen, a.nopmax, t)).blocks;
+    parts[t] = 1;
+  }
+  while (used < most && (used - tiles + 1) * K * 256 <= series) {
+    int b = 0;
+    for (int t = 1; t < tiles; ++t)
+      if ((long long)blocks[t] * parts[b] > (long long)blocks[b] * parts[t]) b = t;
+    if (blocks[b] <= parts[b]) break;
+    ++parts[b];
+    ++used;
+  }
+  for (WaveShare& w : a.share) w = {0, 0, 0, -1, 0, 0};
+  a.slots = 0;
+  for (int t = 0, w = 0; t < tiles; ++t) {
+    for (int p = 0; p < parts[t]; ++p, ++w)
+      a.share[w] = {t, blocks[t] * p / parts[t], blocks[t] * (p + 1) / parts[t], p, parts[t],
+                    a.slots + (p > 0 ? p - 1 : 0)};
+    a.slots += parts[t] - 1;
+  }
+  return used;
+}
+
 unsigned grid8(long long nel) { return (unsigned)((nel + 7) / 8 * 8); }
 
 // (pair blocks, row stride) of the off-band kernels: ~16k workgroups in flight
@@ -841,6 +872,25 @@ dim3 offband_grid(int nm, long long rows) {
   return dim3(gx, (unsigned)std::min<long long>(gy, 65535));
 }
 
+
+template <bool POL, int NW>
+int band_kernel(const GwArgs& a, int series, hipStream_t s) {
+  auto* k = POL ? k_polarization<NW> : k_selfenergy<NW>;
+  const int bytes = series * (int)sizeof(double);
+  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  hipLaunchKernelGGL(k, dim3(grid8(a.nel)), dim3(64 * NW), bytes, s, a);
+  return 0;
+}
+
+// Band kernel with as many waves as the tiles give work: 8 where two or more workgroups
+// share a CU, 16 where the series leave room for one.
+template <bool POL>
+int band_launch(GwArgs& a, int nout, int K, int series, hipStream_t s) {
+  const int used = deal<POL>(a, nout, series * 8 > kLdsCu / 2 ? 16 : 8, K, series);
+  if (used <= 4) return band_kernel<POL, 4>(a, series, s);
+  if (used <= 8) return band_kernel<POL, 8>(a, series, s);
+  return band_kernel<POL, 16>(a, series, s);
+}
 
 // FFT form: workspace bytes per slab of series (K kinds per slot) and the launches.
 constexpr size_t kFftChunkBytes = size_t(4) << 30;  // spectra of one chunk of slabs
@@ -1054,12 +1104,7 @@ int gw_polarization(const gw_params* p, const double* Gl, const double* Gg, cons
     hipLaunchKernelGGL(k_pol_gather, dim3((unsigned)((a.nen + 63) / 64), gy), dim3(256), 0, s, a);
     HIPCHK(hipGetLastError());
   }
-  if (a.nen <= 1024)
-    hipLaunchKernelGGL(k_polarization<1024>, dim3(grid8(nel)), dim3(NTH_P), 0, s, a);
-  else if (a.nen <= 2048)
-    hipLaunchKernelGGL(k_polarization<2048>, dim3(grid8(nel)), dim3(NTH_P), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_polarization<3072>, dim3(grid8(nel)), dim3(NTH_P), 0, s, a);
+  if (int rc = band_launch<true>(a, 2 * a.nopmax + 1, 2, 3 * (a.nen + 2 * kPadX) + 2 * pol_series(a.nen), s)) return rc;
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1090,10 +1135,7 @@ int gw_selfenergy(const gw_params* p, const double* Gl, const double* Gg, const 
     hipLaunchKernelGGL(k_sig_offband, offband_grid(a.nm, (long long)(a.nx - 4) * a.nen), dim3(256), 0, s, a);
     HIPCHK(hipGetLastError());
   }
-  if (a.nen <= 1024)
-    hipLaunchKernelGGL(k_selfenergy<1024>, dim3(grid8(nel)), dim3(NTH_S), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_selfenergy<2040>, dim3(grid8(nel)), dim3(NTH_S), 0, s, a);
+  if (int rc = band_launch<false>(a, a.nen, 5, 5 * (2 * a.nopmax + 1 + 2 * kPadX) + 3 * sig_series(a.nen), s)) return rc;
   HIPCHK(hipGetLastError());
   return 0;
 }
