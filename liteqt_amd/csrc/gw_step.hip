@@ -50,6 +50,7 @@ constexpr int kPadY = 256;  // zero padding of a Y series on each side (reach 25
 constexpr int kPolDirectMax = 3072, kSigDirectMax = 2040;
 
 constexpr int kLdsCu = 160 * 1024;
+constexpr int kOffRows = 4;  // rows of an off-band block in a launch with band blocks
 constexpr int kMaxWaves = 16;  // 12 tiles at the longest series
 
 // What one wave of a workgroup computes: blocks c0 .. c1 - 1 of 16 steps of a tile of 256
@@ -105,6 +106,7 @@ struct GwArgs {
   double* Or;
   double* X;   // polarization: Im G^<, Im G^>, Im G^r of every band element, energy-contiguous
   int slots;   // partial tiles of the waves
+  unsigned gg, og, ox;  // groups of 8 blocks, those of the off-band elements, blocks per row of pairs
   WaveShare share[kMaxWaves];
 };
 
@@ -149,6 +151,75 @@ __global__ __launch_bounds__(256) void k_pol_gather(GwArgs a) {
   }
 }
 
+// P outside the band (|i - j| > nd): zero.  One pair ij of a slab (32-bit index math), rows
+// (slab, energy) r0, r0 + dr, ...
+__device__ __forceinline__ void pol_offband(const GwArgs& a, int ij, long long r0, long long dr) {
+  const int nn = a.nm * a.nm;
+  if (ij >= nn) return;
+  const int i = ij % a.nm, j = ij / a.nm;
+  if (abs(i - j) <= a.nd) return;
+  const long long rows = (long long)a.nx * a.nen;
+  for (long long r = r0; r < rows; r += dr) {
+    const size_t o = (size_t)r * nn + ij;
+    reinterpret_cast<double2*>(a.Ol)[o] = make_double2(0, 0);
+    reinterpret_cast<double2*>(a.Og)[o] = make_double2(0, 0);
+    reinterpret_cast<double2*>(a.Or)[o] = make_double2(0, 0);
+  }
+}
+
+// Sigma outside the band: Sigma_new = 0, so Sigma_gw += alpha (0 - Sigma_gw), on slabs
+// 3..nx-2 (1-based), with the same edge copy.  Rows are (energy, interior slab) pairs, two
+// at a time (six loads in flight).
+__device__ __forceinline__ void sig_offband(const GwArgs& a, int ij, long long r0, long long dr) {
+  const int nn = a.nm * a.nm;
+  if (ij >= nn) return;
+  const int i = ij % a.nm, j = ij / a.nm;
+  if (abs(i - j) <= a.nd) return;
+  const size_t SS = (size_t)nn;
+  const int ns = a.nx - 4;
+  const int last = a.nx - 3;
+  const long long rows = (long long)ns * a.nen;
+  double2* S[3] = {reinterpret_cast<double2*>(a.Ol), reinterpret_cast<double2*>(a.Og),
+                   reinterpret_cast<double2*>(a.Or)};
+  for (long long r = r0; r < rows; r += 2 * dr) {
+    const bool two = r + dr < rows;
+    int ix[2];
+    size_t o[2];
+    double2 v[2][3];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const long long rq = q && two ? r + dr : r;
+      ix[q] = 2 + (int)(rq % ns);
+      o[q] = (size_t)ij + SS * ix[q] + SS * a.nx * (size_t)(rq / ns);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v[q][k] = S[k][o[q]];
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (q && !two) break;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double2 m = make_double2(v[q][k].x + a.alpha * (0.0 - v[q][k].x), v[q][k].y + a.alpha * (0.0 - v[q][k].y));
+        double2* s = S[k] + o[q];
+        s[0] = m;
+        if (ix[q] == 2) { s[-2 * (ptrdiff_t)SS] = m; s[-(ptrdiff_t)SS] = m; }
+        if (ix[q] == last) { s[SS] = m; s[2 * SS] = m; }
+      }
+    }
+  }
+}
+
+// Block of a launch that holds both kinds: groups of 8 consecutive blocks (one to an XCD)
+// belong to the off-band elements evenly, a.og of a.gg, so both kinds end together.
+// Returns true for an off-band block; b is its index among its kind.
+__device__ __forceinline__ bool offband_block(const GwArgs& a, unsigned& b) {
+  const unsigned g = blockIdx.x / 8;
+  const unsigned before = (unsigned)((unsigned long long)g * a.og / a.gg);
+  const bool off = (unsigned)((unsigned long long)(g + 1) * a.og / a.gg) > before;
+  b = (off ? before : g - before) * 8 + blockIdx.x % 8;
+  return off;
+}
+
 // Element (i, j, slab) of a workgroup.  Logical block b = (slab' * nm + j) * (2 nd + 1) +
 // (i - j + nd): consecutive blocks are consecutive rows i of one column j, whose energy
 // series are adjacent in memory.  Workgroups are dealt round-robin to the 8 XCDs (each
@@ -158,10 +229,10 @@ __global__ __launch_bounds__(256) void k_pol_gather(GwArgs a) {
 // Dense bands (nd >= 8) use 8 x 4 tiles of (i, j) instead, i fastest: the 32 workgroups
 // an XCD runs at once share the lines of the ij series 8 ways and, in the polarization,
 // those of the transposed ji series 4 ways.
-__device__ __forceinline__ bool element(const GwArgs& a, int& i, int& j, int& ix) {
+__device__ __forceinline__ bool element(const GwArgs& a, unsigned block, int& i, int& j, int& ix) {
   const int band = 2 * a.nd + 1;
-  const long long per = gridDim.x / 8;
-  long long b = (long long)(blockIdx.x % 8) * per + blockIdx.x / 8;
+  const long long per = a.gg - a.og;
+  long long b = (long long)(block % 8) * per + block / 8;
   if (b >= a.nel) return false;
   if (a.tiled) {
     const int ti = (a.nm + 7) / 8;
@@ -221,7 +292,13 @@ __global__ __launch_bounds__(64 * NW) void k_polarization(GwArgs a) {
   extern __shared__ double lds[];
   constexpr int NTH = 64 * NW;
   int i, j, ix;
-  if (!element(a, i, j, ix)) return;  // uniform over the workgroup, before any barrier
+  unsigned b;
+  if (offband_block(a, b)) {
+    const unsigned dr = 8 * a.og / a.ox;
+    if (b / a.ox < dr) pol_offband(a, b % a.ox * NTH + threadIdx.x, b / a.ox, dr);
+    return;
+  }
+  if (!element(a, b, i, j, ix)) return;  // uniform over the workgroup, before any barrier
   const int nen = a.nen, tid = threadIdx.x;
   const size_t ES = (size_t)a.nm * a.nm * a.nx;  // energy stride (complex elements)
   const size_t eij = (size_t)i + (size_t)a.nm * j + (size_t)a.nm * a.nm * ix;
@@ -333,7 +410,13 @@ __global__ __launch_bounds__(64 * NW) void k_selfenergy(GwArgs a) {
   extern __shared__ double lds[];
   constexpr int NTH = 64 * NW;
   int i, j, ix;
-  if (!element(a, i, j, ix)) return;
+  unsigned b;
+  if (offband_block(a, b)) {
+    const unsigned dr = 8 * a.og / a.ox;
+    if (b / a.ox < dr) sig_offband(a, b % a.ox * NTH + threadIdx.x, b / a.ox, dr);
+    return;
+  }
+  if (!element(a, b, i, j, ix)) return;
   const int nen = a.nen, tid = threadIdx.x;
   const size_t ES = (size_t)a.nm * a.nm * a.nx;
   const size_t SS = (size_t)a.nm * a.nm;  // slab stride
@@ -465,50 +548,12 @@ __global__ __launch_bounds__(64 * NW) void k_selfenergy(GwArgs a) {
   }
 }
 
-// P outside the band (|i - j| > nd): zero.  blockIdx.x covers the nm^2 pairs of a slab
-// (32-bit index math), blockIdx.y strides over the nx * nen (slab, energy) rows.
 __global__ __launch_bounds__(256) void k_pol_offband(GwArgs a) {
-  const int nn = a.nm * a.nm;
-  const int ij = blockIdx.x * 256 + threadIdx.x;
-  if (ij >= nn) return;
-  const int i = ij % a.nm, j = ij / a.nm;
-  if (abs(i - j) <= a.nd) return;
-  const long long rows = (long long)a.nx * a.nen;
-  for (long long r = blockIdx.y; r < rows; r += gridDim.y) {
-    const size_t o = (size_t)r * nn + ij;
-    reinterpret_cast<double2*>(a.Ol)[o] = make_double2(0, 0);
-    reinterpret_cast<double2*>(a.Og)[o] = make_double2(0, 0);
-    reinterpret_cast<double2*>(a.Or)[o] = make_double2(0, 0);
-  }
+  pol_offband(a, blockIdx.x * 256 + threadIdx.x, blockIdx.y, gridDim.y);
 }
 
-// Sigma outside the band: Sigma_new = 0, so Sigma_gw += alpha (0 - Sigma_gw), on slabs
-// 3..nx-2 (1-based), with the same edge copy.  Rows are (energy, interior slab) pairs.
 __global__ __launch_bounds__(256) void k_sig_offband(GwArgs a) {
-  const int nn = a.nm * a.nm;
-  const int ij = blockIdx.x * 256 + threadIdx.x;
-  if (ij >= nn) return;
-  const int i = ij % a.nm, j = ij / a.nm;
-  if (abs(i - j) <= a.nd) return;
-  const size_t SS = (size_t)nn;
-  const int ns = a.nx - 4;
-  const int last = a.nx - 3;
-  const long long rows = (long long)ns * a.nen;
-  double2* S[3] = {reinterpret_cast<double2*>(a.Ol), reinterpret_cast<double2*>(a.Og),
-                   reinterpret_cast<double2*>(a.Or)};
-  for (long long r = blockIdx.y; r < rows; r += gridDim.y) {
-    const int ix = 2 + (int)(r % ns);
-    const long long e = r / ns;
-    const size_t o = (size_t)ij + SS * ix + SS * a.nx * (size_t)e;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const double2 v = S[k][o];
-      const double2 m = make_double2(v.x + a.alpha * (0.0 - v.x), v.y + a.alpha * (0.0 - v.y));
-      S[k][o] = m;
-      if (ix == 2) { S[k][o - 2 * SS] = m; S[k][o - SS] = m; }
-      if (ix == last) { S[k][o + SS] = m; S[k][o + 2 * SS] = m; }
-    }
-  }
+  sig_offband(a, blockIdx.x * 256 + threadIdx.x, blockIdx.y, gridDim.y);
 }
 
 // ---------------------------------------------------------------------------------
@@ -863,7 +908,7 @@ int deal(GwArgs& a, int nout, int most, int K, int series) {
   return used;
 }
 
-unsigned grid8(long long nel) { return (unsigned)((nel + 7) / 8 * 8); }
+
 
 // (pair blocks, row stride) of the off-band kernels: ~16k workgroups in flight
 dim3 offband_grid(int nm, long long rows) {
@@ -872,13 +917,34 @@ dim3 offband_grid(int nm, long long rows) {
   return dim3(gx, (unsigned)std::min<long long>(gy, 65535));
 }
 
-
+// The band kernel, and the off-band elements: in the same launch while two workgroups fit
+// a CU, so that the matrix products run under the off-band elements' memory traffic; where
+// the LDS holds one, an off-band block would take a CU's place and goes by itself.  (Separate
+// -> one launch, polarization / self-energy: 64 orbitals, 12 slabs, ndiag 1, 600 energies 566 /
+// 850 -> 464 / 720 us, 900 energies 911 / 1330 -> 900 / 1090; memory-bound: 3.4 GB of writes and
+// 1.6 GB of reads in the two passes at 600.)
 template <bool POL, int NW>
-int band_kernel(const GwArgs& a, int series, hipStream_t s) {
+int band_kernel(GwArgs& a, int series, hipStream_t s) {
   auto* k = POL ? k_polarization<NW> : k_selfenergy<NW>;
   const int bytes = series * (int)sizeof(double);
+  const long long rows = (long long)(POL ? a.nx : a.nx - 4) * a.nen;
+  a.gg = (unsigned)((a.nel + 7) / 8);
+  a.og = 0;
+  a.ox = 1;
+  if (a.nd < a.nm - 1) {
+    const long long ox = ((long long)a.nm * a.nm + 64 * NW - 1) / (64 * NW);
+    const long long og = (ox * std::max(1LL, rows / kOffRows) + 7) / 8;
+    if (2 * bytes <= kLdsCu && (a.gg + og) * 8 * 64 * NW < (1LL << 32)) {
+      a.ox = (unsigned)ox;
+      a.og = (unsigned)og;
+      a.gg += a.og;
+    } else {
+      hipLaunchKernelGGL(POL ? k_pol_offband : k_sig_offband, offband_grid(a.nm, rows), dim3(256), 0, s, a);
+      HIPCHK(hipGetLastError());
+    }
+  }
   HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-  hipLaunchKernelGGL(k, dim3(grid8(a.nel)), dim3(64 * NW), bytes, s, a);
+  hipLaunchKernelGGL(k, dim3(8 * a.gg), dim3(64 * NW), bytes, s, a);
   return 0;
 }
 
@@ -1095,10 +1161,6 @@ int gw_polarization(const gw_params* p, const double* Gl, const double* Gg, cons
     }
   }
   a.X = need ? reinterpret_cast<double*>(ws.p) : nullptr;
-  if (a.nd < a.nm - 1) {
-    hipLaunchKernelGGL(k_pol_offband, offband_grid(a.nm, (long long)a.nx * a.nen), dim3(256), 0, s, a);
-    HIPCHK(hipGetLastError());
-  }
   if (a.X) {
     const unsigned gy = (unsigned)std::min<long long>((long long)a.nm * a.nx, 65535);
     hipLaunchKernelGGL(k_pol_gather, dim3((unsigned)((a.nen + 63) / 64), gy), dim3(256), 0, s, a);
@@ -1131,10 +1193,6 @@ int gw_selfenergy(const gw_params* p, const double* Gl, const double* Gg, const 
   const long long per_slab = a.tiled ? 32LL * ((a.nm + 7) / 8) * ((a.nm + 3) / 4) : (long long)a.nm * (2 * a.nd + 1);
   const long long nel = per_slab * (a.nx - 4);
   a.nel = nel;
-  if (a.nd < a.nm - 1) {
-    hipLaunchKernelGGL(k_sig_offband, offband_grid(a.nm, (long long)(a.nx - 4) * a.nen), dim3(256), 0, s, a);
-    HIPCHK(hipGetLastError());
-  }
   if (int rc = band_launch<false>(a, a.nen, 5, 5 * (2 * a.nopmax + 1 + 2 * kPadX) + 3 * sig_series(a.nen), s)) return rc;
   HIPCHK(hipGetLastError());
   return 0;
