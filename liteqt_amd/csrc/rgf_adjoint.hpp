@@ -243,7 +243,7 @@ __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH
     }
   };
   auto uo = [&](int op) { return op ^ uC; };
-  int fails = 0, hitL = 0, hitR = 0;
+  int fails = 0;
   double Jv = 0.0;
 
   // ---- contacts (fixed)
@@ -251,16 +251,15 @@ __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH
     wg_ew(n, H00, 0, zero, a.lead, one, nullptr, one, nullptr, one);
   else
     wg_ew(n, H00, 0, zero, Hb(0), one, sR(0), one, nullptr, one);
-  const int itL = wg_sancho<T, NMAX>(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, H00, Cb(0), 1, GsL, stmp, lds, red,
-                                     hitL, fails);
+  if (a.lead)
+    wg_ew(n, W, 0, zero, a.lead + nn, one, nullptr, one, nullptr, one);
+  else
+    wg_ew(n, W, 0, zero, Hb(N - 1), one, sR(N - 1), one, nullptr, one);
+  Lead left{H00, Cb(0), 1, GsL, stmp, nullptr}, right{W, Cb(N - 1), 0, Gs, Dd, nullptr};
+  Leads<T, NMAX>::run(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, left, right, lds, red);
+  fails += left.fails + right.fails;
   wg_gemm<T>(n, OP_N, Cb(0), OP_N, GsL, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_C, Cb(0), SL, 0, st, lds);
-  if (a.lead)
-    wg_ew(n, H00, 0, zero, a.lead + nn, one, nullptr, one, nullptr, one);
-  else
-    wg_ew(n, H00, 0, zero, Hb(N - 1), one, sR(N - 1), one, nullptr, one);
-  const int itR = wg_sancho<T, NMAX>(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, H00, Cb(N - 1), 0, Gs, stmp, lds,
-                                     red, hitR, fails);
   wg_gemm<T>(n, OP_C, Cb(N - 1), OP_N, Gs, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_N, Cb(N - 1), SR, 0, st, lds);
   const double fL = ferm_dev((E - a.mu[0]) / (a.boltz * a.temp[0]));
@@ -481,9 +480,9 @@ __device__ void adjoint_energy(const AdjArgs& a, int e, double2* ws, double2* dH
   if (first) {
     a.J[e] = Jv;
     if (a.info) {
-      a.info[4 * (size_t)e + 0] = itL;
-      a.info[4 * (size_t)e + 1] = itR;
-      a.info[4 * (size_t)e + 2] = hitL | (hitR << 1) | lead_flags;
+      a.info[4 * (size_t)e + 0] = left.it;
+      a.info[4 * (size_t)e + 1] = right.it;
+      a.info[4 * (size_t)e + 2] = left.hit | (right.hit << 1) | lead_flags;
       a.info[4 * (size_t)e + 3] = fails;
     }
   }

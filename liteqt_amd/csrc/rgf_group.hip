@@ -23,21 +23,25 @@ hipError_t clear(char* ctl, int ngroups, hipStream_t s) {
 }
 
 // Microseconds of one energy on a group of G workgroups: the measured times of the block
-// operations as functions of the block size, a slab of 16 GEMMs and an inverse, 36
-// decimation iterations of 6 GEMMs and an inverse.  GEMM from 96 orbitals: barrier 5, 1.6
-// us per 32 x 32 tile and K panel, or 0.33 us per 128 x 64 tile and k; inverse: rank 0
-// alone up to 128 orbitals, above it the column steps (475 us at 256) and 62 us per round
-// of the strips.  32 and 64 orbitals run on one workgroup.
+// operations as functions of the block size, a slab of 16 GEMMs and an inverse, 18
+// decimation iterations of 6 GEMMs and an inverse per contact, each on half of the group.
+// GEMM from 96 orbitals: barrier 5, 1.6 us per 32 x 32 tile and K panel, or 0.33 us per
+// 128 x 64 tile and k; inverse: rank 0 alone up to 128 orbitals, above it the column steps
+// (475 us at 256) and 62 us per round of the strips.  32 and 64 orbitals run on one
+// workgroup.
 double item_us(int n, int nx, int G) {
   const int t = n / 32;
-  double gemm = 5.0 + ((t * t + G - 1) / G) * 1.6 * t;
-  double inv = n <= 128 ? 1.85 * n : 475.0 * n / 256 + 62.0 * ((n / 16 + G - 1) / G) * n * n / 65536.0;
-  if (n % 128 == 0) gemm = std::min(gemm, 5.0 + ((t * t / 8 + G - 1) / G) * 0.33 * n);
-  if (n < 96) {
-    gemm = n == 64 ? 14.0 : 6.0;
-    inv = 1.2 * n;
-  }
-  return nx * (16 * gemm + inv) + 36 * (6 * gemm + inv);
+  auto us = [&](int gemms, int ranks) {
+    double gemm = 5.0 + ((t * t + ranks - 1) / ranks) * 1.6 * t;
+    double inv = n <= 128 ? 1.85 * n : 475.0 * n / 256 + 62.0 * ((n / 16 + ranks - 1) / ranks) * n * n / 65536.0;
+    if (n % 128 == 0) gemm = std::min(gemm, 5.0 + ((t * t / 8 + ranks - 1) / ranks) * 0.33 * n);
+    if (n < 96) {
+      gemm = n == 64 ? 14.0 : 6.0;
+      inv = 1.2 * n;
+    }
+    return gemms * gemm + inv;
+  };
+  return nx * us(16, G) + 18 * (G > 1 ? us(6, G / 2) : 2 * us(6, 1));
 }
 
 }  // namespace

@@ -50,14 +50,16 @@ struct GroupCtl {
   unsigned barrier, pad2[31];   // arrivals at the barriers, all of them
   int info[2], pad3[30];        // rank 0's result of an operation, by barrier parity
   double part[2][kMaxTiles];    // partial sums of a GEMM's tiles, by barrier parity
+  int lead[2][3];               // a contact's iterations, limit flag, singular inverses
 };
 constexpr unsigned kClosed = 1u << 16;
-static_assert(sizeof(GroupCtl) <= kGroupCtlBytes, "control area of a group");
+static_assert(sizeof(GroupCtl) <= kCtlBytes, "control area of a group");
 
 struct GroupCtx {  // in LDS, one per workgroup
   GroupCtl* ctl;
   int rank, size;
   unsigned epoch;  // barriers passed
+  unsigned half_epoch;  // barriers of this workgroup's half
 };
 
 __device__ __forceinline__ GroupCtx* group_ctx() {
@@ -117,7 +119,7 @@ __device__ __forceinline__ bool group_join(char* area, int size) {
     GroupCtl* ctl = reinterpret_cast<GroupCtl*>(area);
     const unsigned r = __hip_atomic_fetch_add(&ctl->arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     c->ctl = ctl;
-    c->epoch = 0;
+    c->epoch = c->half_epoch = 0;
     c->rank = (int)r;
     c->size = 0;
     if (r == 0) {
@@ -412,6 +414,63 @@ __device__ __forceinline__ int wg_inverse(GroupN n, double2* W, double2* out, ld
     return wg_inverse_strip<256>(n, W, out, lds);
   }
 }
+
+// ----------------------------------------------------------------- contacts
+// The decimations of the two contacts do not depend on each other and are half of a solve's
+// inverses, which do not get faster with the ranks: each half of the group runs one.
+// Between the split and the merge a workgroup is a rank of its half, which has a control
+// area of its own.
+template <int NMAX>
+struct Leads<kGrp, NMAX> {
+  static __device__ __noinline__ void run(GroupN n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
+                                          ldsd* lds, ldsd* red) {
+    const int size = group_size(n), rank = group_rank(n), first = (size + 1) / 2;
+    if (size == 1) {
+      for (int h = 0; h < 2; ++h) one(n, E, eta, tol, nmax, h ? R : L, lds, red);
+      return;
+    }
+    const int h = rank >= first ? 1 : 0;
+    GroupCtx* c = group_ctx();
+    GroupCtl* ctl = uni(c->ctl);
+    const unsigned epoch = uni((int)c->epoch);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      c->ctl = reinterpret_cast<GroupCtl*>(reinterpret_cast<char*>(ctl) + kCtlBytes * (1 + h));
+      c->rank = h ? rank - first : rank;
+      c->size = h ? size - first : first;
+      c->epoch = c->half_epoch;
+    }
+    __syncthreads();
+    Lead& m = h ? R : L;
+    one(n, E, eta, tol, nmax, m, lds, red);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      if (c->rank == 0) {
+        agent_store(&ctl->lead[h][0], m.it);
+        agent_store(&ctl->lead[h][1], m.hit);
+        agent_store(&ctl->lead[h][2], m.fails);
+      }
+      c->half_epoch = c->epoch;
+      c->ctl = ctl;
+      c->rank = rank;
+      c->size = size;
+      c->epoch = epoch;
+    }
+    group_barrier();
+    for (int k = 0; k < 2; ++k) {
+      Lead& x = k ? R : L;
+      x.it = uni(agent_load(&ctl->lead[k][0]));
+      x.hit = uni(agent_load(&ctl->lead[k][1]));
+      x.fails = uni(agent_load(&ctl->lead[k][2]));
+    }
+  }
+
+  static __device__ __noinline__ void one(GroupN n, double E, double eta, double tol, int nmax, Lead& m, ldsd* lds,
+                                          ldsd* red) {
+    m.hit = m.fails = 0;
+    m.it = wg_sancho<kGrp, NMAX>(n, E, eta, tol, nmax, m.H00, m.C, m.left, m.G, m.tb, lds, red, m.hit, m.fails);
+  }
+};
 
 // ------------------------------------------------------------------ kernels
 template <int NMAX>

@@ -6,7 +6,8 @@
 
 namespace rgf {
 
-constexpr size_t kGroupCtlBytes = 2048;
+constexpr size_t kCtlBytes = 2048;  // control words of a group, of each of its halves
+constexpr size_t kGroupCtlBytes = 3 * kCtlBytes;
 constexpr int kXcds = 8;
 
 struct GroupArgs {

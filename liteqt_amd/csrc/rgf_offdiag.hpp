@@ -84,18 +84,17 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
     wg_ew(n, Dd, 0, zero, Cb(l), one, sRlo(l), one, nullptr, one);
     wg_ew(n, Du, 0, zero, sRup(l), one, nullptr, one, Cb(l), one);
   };
-  int fails = 0, hitL = 0, hitR = 0;
+  int fails = 0;
 
   // ---- contacts (leads repeat the edge slabs with their diagonal Sigma^R)
   wg_ew(n, H00, 0, zero, Hb(0), one, sR(0), one, nullptr, one);
-  const int itL = wg_sancho<T, NMAX>(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, H00, Cb(0), 1, Gs, stmp, lds, red,
-                                     hitL, fails);
+  wg_ew(n, W, 0, zero, Hb(N - 1), one, sR(N - 1), one, nullptr, one);
+  Lead left{H00, Cb(0), 1, Gs, stmp, nullptr}, right{W, Cb(N - 1), 0, K1, T0, nullptr};
+  Leads<T, NMAX>::run(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, left, right, lds, red);
+  fails += left.fails + right.fails;
   wg_gemm<T>(n, OP_N, Cb(0), OP_N, Gs, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_C, Cb(0), SL, 0, st, lds);
-  wg_ew(n, H00, 0, zero, Hb(N - 1), one, sR(N - 1), one, nullptr, one);
-  const int itR = wg_sancho<T, NMAX>(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, H00, Cb(N - 1), 0, Gs, stmp, lds,
-                                     red, hitR, fails);
-  wg_gemm<T>(n, OP_C, Cb(N - 1), OP_N, Gs, T0, 0, st, lds);
+  wg_gemm<T>(n, OP_C, Cb(N - 1), OP_N, K1, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_N, Cb(N - 1), SR, 0, st, lds);
   const double fL = ferm_dev((E - a.mu[0]) / (a.boltz * a.temp[0]));
   const double fR = ferm_dev((E - a.mu[1]) / (a.boltz * a.temp[1]));
@@ -231,9 +230,9 @@ __device__ void solve_energy_od(const SweepArgs& a, int e, double2* ws, ldsd* ld
     if (a.tre && lead) a.tre[e] = fL * a1 - (fL - 1.0) * a2;
   }
   if (a.info && lead) {
-    a.info[4 * (size_t)e + 0] = itL;
-    a.info[4 * (size_t)e + 1] = itR;
-    a.info[4 * (size_t)e + 2] = hitL | (hitR << 1);
+    a.info[4 * (size_t)e + 0] = left.it;
+    a.info[4 * (size_t)e + 1] = right.it;
+    a.info[4 * (size_t)e + 2] = left.hit | (right.hit << 1);
     a.info[4 * (size_t)e + 3] = fails;
   }
   __syncthreads();

@@ -165,6 +165,28 @@ __device__ int wg_sancho(typename Dim<T>::type n, double E, double eta, double t
   return it_run;
 }
 
+// A contact's decimation: its input and, after the run, the iterations, whether the limit
+// was hit and the singular inverses.
+struct Lead {
+  const double2 *H00, *C;
+  int left;
+  double2 *G, *tb;
+  const double2* S00;
+  int it, hit, fails;
+};
+
+// The surface functions of both contacts, one after the other (with tb of the first).  A
+// group of workgroups (rgf_group.hpp) runs them at the same time and needs both tb.
+template <int T, int NMAX>
+struct Leads {
+  static __device__ void run(typename Dim<T>::type n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
+                             ldsd* lds, ldsd* red) {
+    L.hit = L.fails = R.hit = R.fails = 0;
+    L.it = wg_sancho<T, NMAX>(n, E, eta, tol, nmax, L.H00, L.C, L.left, L.G, L.tb, lds, red, L.hit, L.fails, L.S00);
+    R.it = wg_sancho<T, NMAX>(n, E, eta, tol, nmax, R.H00, R.C, R.left, R.G, L.tb, lds, red, R.hit, R.fails, R.S00);
+  }
+};
+
 // CMS = true: green_RGF_CMS (src/green_rgf.f90:4167-4383), the compat solve
 // with the overlap blocks Sii: z S_l, Sigma^R_l S_l, Sigma^<_l S_l, the
 // decimation with S00, and pdens / GGi1 from the reference's G^> recursion
@@ -221,7 +243,7 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
   auto gl = [&](int l) { return Gl + gpos(l) * nn; };
   auto gln = [&](int l) { return Gln + gpos(l) * nn; };
   const Epi st = epi_store();
-  int fails = 0, hitL = 0, hitR = 0;
+  int fails = 0;
 
   auto Sb = [&](int l) -> const double2* { return CMS ? a.Sii + (size_t)l * nn : nullptr; };
   // onsite block of slab l: H + Sigma^R (CMS: H + Sigma^R S)
@@ -254,10 +276,15 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
     if (ahp) wg_antiherm(n, T2, gln(l), lds);
   };
 
-  // ---- left contact
+  // ---- the leads' surface functions: left in G, right in Gn until its contact
+  const int L1 = nx - 1;
   onsite(0, H00);
-  const int itL = wg_sancho<T, NMAX>(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, H00, Cb(0), 1, G, stmp,
-                                     lds, red, hitL, fails, Sb(0));
+  onsite(L1, Gp);
+  Lead left{H00, Cb(0), 1, G, stmp, Sb(0)}, right{Gp, Cb(L1), 0, Gn, tb + 7 * nn, Sb(L1)};
+  Leads<T, NMAX>::run(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, left, right, lds, red);
+  fails += left.fails + right.fails;
+
+  // ---- left contact
   wg_gemm<T>(n, OP_N, Cb(0), OP_N, G, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_C, Cb(0), SL, 0, st, lds);
   const double fL = ferm_dev((E - a.mu[0]) / (a.boltz * a.temp[0]));
@@ -296,11 +323,8 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
   for (int l = 1; l < nx - 1; ++l) forward_step(l, true);
 
   // ---- right contact
-  const int L1 = nx - 1;
   onsite(L1, H00);
-  const int itR = wg_sancho<T, NMAX>(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, H00, Cb(L1), 0, G, stmp,
-                                     lds, red, hitR, fails, Sb(L1));
-  wg_gemm<T>(n, OP_C, Cb(L1), OP_N, G, T0, 0, st, lds);
+  wg_gemm<T>(n, OP_C, Cb(L1), OP_N, Gn, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_N, Cb(L1), SR, 0, st, lds);
   wg_gemm<T>(n, OP_N, Cb(L1), OP_N, gl(L1 - 1), T0, 0, st, lds);
   {
@@ -433,9 +457,9 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
     if (a.tre && lead) a.tre[e] = fLt * a1 - (fLt - 1.0) * a2;
   }
   if (a.info && lead) {
-    a.info[4 * (size_t)e + 0] = itL;
-    a.info[4 * (size_t)e + 1] = itR;
-    a.info[4 * (size_t)e + 2] = hitL | (hitR << 1);
+    a.info[4 * (size_t)e + 0] = left.it;
+    a.info[4 * (size_t)e + 1] = right.it;
+    a.info[4 * (size_t)e + 2] = left.hit | (right.hit << 1);
     a.info[4 * (size_t)e + 3] = fails;
   }
   __syncthreads();
