@@ -437,6 +437,12 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
   const bool od = has_offdiag(b) || scba || second;
   long long slot_bytes = pr.slot_elems * 16LL;
   Split sp = group_split(b->nm, b->nE, pr.cus, pr.slots, b->max_slots);
+  const long long pair_extra = (long long)rgf::kPairExtra * b->nm * b->nm;
+  if (!od && !b->Sii && b->max_slots <= 0 && rgf::pair_plan(b->nm, b->nE, pr.cus, &sp.g)) {
+    sp.tail = sp.need = b->nE;
+    pr.a.ws_slot += pair_extra;
+    slot_bytes += pair_extra * 16LL;
+  }
   std::lock_guard<std::mutex> lk(g_ws_mu);
   Buf& ws = g_ws[pr.dev];
   if ((size_t)(sp.need * slot_bytes) + sp.ctl_bytes() > ws.bytes) {
@@ -448,6 +454,9 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
     if (sp.tail && (size_t)(sp.need * slot_bytes) + sp.ctl_bytes() > avail) {
       sp = Split();  // one workgroup per energy, on the slots that fit
       sp.need = pr.slots;
+      pr.a.ws_slot = pr.slot_elems;
+      slot_bytes = pr.slot_elems * 16LL;
+      fit = (long long)(avail / (size_t)slot_bytes);
     }
     // automatic segment recompute: when the full slots leave CUs idle, keep the
     // blocks only at checkpoints every ceil(sqrt(nx)) slabs and one segment, at the

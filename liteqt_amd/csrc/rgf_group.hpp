@@ -421,13 +421,13 @@ __device__ __forceinline__ int wg_inverse(GroupN n, double2* W, double2* out, ld
 // Between the split and the merge a workgroup is a rank of its half, which has a control
 // area of its own.
 template <int NMAX>
-struct Leads<kGrp, NMAX> {
-  static __device__ __noinline__ void run(GroupN n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
+struct Leads<kGrp, NMAX> : LeadsBase {
+  static __device__ __noinline__ bool run(GroupN n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
                                           ldsd* lds, ldsd* red) {
     const int size = group_size(n), rank = group_rank(n), first = (size + 1) / 2;
     if (size == 1) {
       for (int h = 0; h < 2; ++h) one(n, E, eta, tol, nmax, h ? R : L, lds, red);
-      return;
+      return false;
     }
     const int h = rank >= first ? 1 : 0;
     GroupCtx* c = group_ctx();
@@ -463,6 +463,7 @@ struct Leads<kGrp, NMAX> {
       x.hit = uni(agent_load(&ctl->lead[k][1]));
       x.fails = uni(agent_load(&ctl->lead[k][2]));
     }
+    return false;
   }
 
   static __device__ __noinline__ void one(GroupN n, double E, double eta, double tol, int nmax, Lead& m, ldsd* lds,
@@ -472,7 +473,67 @@ struct Leads<kGrp, NMAX> {
   }
 };
 
+// At 32 and 64 orbitals a block operation is too short to share, but the right contact's
+// decimation is not needed before the forward sweep is over: in a group of two, rank 1 runs
+// it and leaves, rank 0 runs the rest of the program.
+constexpr int kPair64 = 66;
+template <>
+struct Cfg<kPair64> : Cfg<2> {};
+
+template <int T, int NMAX>
+struct PairLeads {
+  static constexpr int kRightTemp = kTmpBlocks;
+  static __device__ __forceinline__ bool left() { return uni(group_ctx()->rank) == 0; }
+  static __device__ __forceinline__ bool right() { return uni(group_ctx()->rank) == 1 || uni(group_ctx()->size) == 1; }
+  static __device__ bool run(typename Dim<T>::type n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
+                             ldsd* lds, ldsd* red) {
+    const int rank = uni(group_ctx()->rank), size = uni(group_ctx()->size);
+    for (int h = rank; h < 2; h += size) {
+      Lead& m = h ? R : L;
+      m.hit = m.fails = 0;
+      m.it = wg_sancho<T, NMAX>(n, E, eta, tol, nmax, m.H00, m.C, m.left, m.G, m.tb, lds, red, m.hit, m.fails);
+    }
+    if (rank == 0) return false;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      GroupCtl* ctl = group_ctx()->ctl;
+      agent_store(&ctl->lead[1][0], R.it);
+      agent_store(&ctl->lead[1][1], R.hit);
+      agent_store(&ctl->lead[1][2], R.fails);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      agent_store(&ctl->barrier, 1u);
+    }
+    return true;
+  }
+  static __device__ __forceinline__ void finish(Lead& R) {
+    if (uni(group_ctx()->size) == 1) return;
+    GroupCtl* ctl = uni(group_ctx()->ctl);
+    if (threadIdx.x == 0) {
+      while (agent_load(&ctl->barrier) == 0u) __builtin_amdgcn_s_sleep(1);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    R.it = uni(agent_load(&ctl->lead[1][0]));
+    R.hit = uni(agent_load(&ctl->lead[1][1]));
+    R.fails = uni(agent_load(&ctl->lead[1][2]));
+  }
+};
+template <>
+struct Leads<kPair32, 32> : PairLeads<kPair32, 32> {};
+template <>
+struct Leads<kPair64, 64> : PairLeads<kPair64, 64> {};
+
 // ------------------------------------------------------------------ kernels
+template <int T, int NMAX>
+__global__ __launch_bounds__(256, 1) void rgf_sweep_pair(SweepArgs a, GroupArgs g) {
+  __shared__ __attribute__((aligned(16))) double lds[SweepLds<T, NMAX>::DOUBLES];
+  int grp;
+  if (!group_join(g, grp)) return;
+  solve_energy<T, NMAX>(a, g.e0 + grp, a.ws + (size_t)grp * (size_t)a.ws_slot, (ldsd*)lds, (ldsd*)lds);
+}
+
 template <int NMAX>
 __global__ __launch_bounds__(256, 1) void rgf_sweep_grp(SweepArgs a, GroupArgs g) {
   __shared__ __attribute__((aligned(16))) double lds[SweepLds<kGrp, NMAX>::DOUBLES];

@@ -15,6 +15,7 @@
 namespace rgf {
 
 constexpr int kReg32 = 9;      // variant code: two workgroups per CU
+constexpr int kPair32 = 65;    // the same program with a second workgroup for the right contact
 constexpr int kSmallLd = 33;   // column stride of a block in LDS (elements)
 constexpr int kSmallBlk = 2 * 32 * kSmallLd;  // doubles of an LDS block
 constexpr int kSmallScratch = 1024;           // doubles below the blocks: exchanges and sums
@@ -28,6 +29,10 @@ template <>
 struct Dim<kReg32> {
   typedef SmallN type;
 };
+template <>
+struct Dim<kPair32> {
+  typedef SmallN type;
+};
 __device__ __forceinline__ bool group_leader(SmallN) { return true; }
 
 template <>
@@ -38,11 +43,18 @@ template <>
 struct InvLds<kReg32, 32> {
   static constexpr int DOUBLES = GjLds<1, 4, 2>::DOUBLES + 32 + 8;  // exchange, then piv and its inverse
 };
+template <>
+struct GemmLds<kPair32> : GemmLds<kReg32> {};
+template <>
+struct InvLds<kPair32, 32> : InvLds<kReg32, 32> {};
 static_assert(InvLds<kReg32, 32>::DOUBLES <= kSmallScratch, "scratch below the LDS blocks");
 template <>
 struct SweepLds<kReg32, 32> {
   static constexpr int DOUBLES = kSmallScratch + 4 * kSmallBlk;
 };
+
+template <>
+struct SweepLds<kPair32, 32> : SweepLds<kReg32, 32> {};
 
 // The four LDS blocks by the temporaries' reads and writes per slab: T0 and T1 (6, 5), T2
 // of the forward with X of the backward sweep (3, 4), W with P7 (2, 3); the latter pairs
@@ -61,6 +73,8 @@ struct Temp<kReg32> {
     return (double2*)(lds + kSmallScratch + slot * kSmallBlk);
   }
 };
+template <>
+struct Temp<kPair32> : Temp<kReg32> {};
 
 // A block where it is: element (i, j) at i + j ld.
 struct SmallBlk {
@@ -191,7 +205,7 @@ __device__ __noinline__ double gemm_reg32(const double2* A_, const double2* B_, 
 
 template <int T, int OPA, int OPB, int CRM>
 __device__ __forceinline__ double wg_gemm_k(SmallN, const double2* A, const double2* B, void* C, Epi ep, ldsd* lds) {
-  static_assert(T == kReg32, "32-orbital program");
+  static_assert(T == kReg32 || T == kPair32, "32-orbital program");
   return gemm_reg32<OPA, OPB, CRM>(A, B, C, ep, lds);
 }
 
@@ -316,7 +330,7 @@ __device__ __noinline__ int small_inverse(const double2* W_, double2* out_, ldsd
 
 template <int T, int NMAX>
 __device__ __forceinline__ int wg_inverse(SmallN, double2* W, double2* out, ldsd* lds) {
-  static_assert(T == kReg32 && NMAX == 32, "32-orbital program");
+  static_assert((T == kReg32 || T == kPair32) && NMAX == 32, "32-orbital program");
   return small_inverse(W, out, lds);
 }
 

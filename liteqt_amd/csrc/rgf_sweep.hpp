@@ -28,6 +28,7 @@ struct Dim {
 // Where temporary k of a program is: in the workspace slot, or for some variants in LDS.
 // The decimation's are kTmpSancho + 0 .. 10.
 constexpr int kTmpSancho = 19;
+constexpr int kSanchoBlocks = 11;
 template <int T>
 struct Temp {
   static __device__ __forceinline__ double2* at(double2* tb, size_t nn, int k, ldsd*) { return tb + (size_t)k * nn; }
@@ -177,13 +178,22 @@ struct Lead {
 
 // The surface functions of both contacts, one after the other (with tb of the first).  A
 // group of workgroups (rgf_group.hpp) runs them at the same time and needs both tb.
+// The hooks are for a second workgroup that runs the right contact's alone: which contacts
+// a workgroup has, whether its part ends with run, and the wait for the right one.
+struct LeadsBase {
+  static constexpr int kRightTemp = 7;  // first of the right decimation's temporaries
+  static __device__ __forceinline__ bool left() { return true; }
+  static __device__ __forceinline__ bool right() { return true; }
+  static __device__ __forceinline__ void finish(Lead&) {}
+};
 template <int T, int NMAX>
-struct Leads {
-  static __device__ void run(typename Dim<T>::type n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
+struct Leads : LeadsBase {
+  static __device__ bool run(typename Dim<T>::type n, double E, double eta, double tol, int nmax, Lead& L, Lead& R,
                              ldsd* lds, ldsd* red) {
     L.hit = L.fails = R.hit = R.fails = 0;
     L.it = wg_sancho<T, NMAX>(n, E, eta, tol, nmax, L.H00, L.C, L.left, L.G, L.tb, lds, red, L.hit, L.fails, L.S00);
     R.it = wg_sancho<T, NMAX>(n, E, eta, tol, nmax, R.H00, R.C, R.left, R.G, L.tb, lds, red, R.hit, R.fails, R.S00);
+    return false;
   }
 };
 
@@ -278,11 +288,12 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
 
   // ---- the leads' surface functions: left in G, right in Gn until its contact
   const int L1 = nx - 1;
-  onsite(0, H00);
-  onsite(L1, Gp);
-  Lead left{H00, Cb(0), 1, G, stmp, Sb(0)}, right{Gp, Cb(L1), 0, Gn, tb + 7 * nn, Sb(L1)};
-  Leads<T, NMAX>::run(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, left, right, lds, red);
-  fails += left.fails + right.fails;
+  typedef Leads<T, NMAX> Ls;
+  if (Ls::left()) onsite(0, H00);
+  if (Ls::right()) onsite(L1, Gp);
+  Lead left{H00, Cb(0), 1, G, stmp, Sb(0)}, right{Gp, Cb(L1), 0, Gn, tb + Ls::kRightTemp * nn, Sb(L1)};
+  if (Ls::run(n, E, a.eta_lead, a.dec_tol, a.dec_nmax, left, right, lds, red)) return;
+  fails += left.fails;
 
   // ---- left contact
   wg_gemm<T>(n, OP_N, Cb(0), OP_N, G, T0, 0, st, lds);
@@ -324,6 +335,8 @@ __device__ void solve_energy(const SweepArgs& a, int e, double2* ws, ldsd* lds, 
 
   // ---- right contact
   onsite(L1, H00);
+  Ls::finish(right);
+  fails += right.fails;
   wg_gemm<T>(n, OP_C, Cb(L1), OP_N, Gn, T0, 0, st, lds);
   wg_gemm<T>(n, OP_N, T0, OP_N, Cb(L1), SR, 0, st, lds);
   wg_gemm<T>(n, OP_N, Cb(L1), OP_N, gl(L1 - 1), T0, 0, st, lds);
