@@ -996,165 +996,14 @@ __device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned
 //
 // Panel step (32 columns K, pivot rows P): the panel is swept in registers
 // (gj_sweep), giving F_P = A_PK^-1 and F_R = -A_RK A_PK^-1; the other
-// columns J are updated by one MFMA GEMM W[:,J] += (F - E) W[P,J] with E the pivot
+// columns J are updated on MFMA, W[:,J] += (F - E) W[P,J] with E the pivot
 // incidence (accumulating onto the loaded tiles of W), and columns K take F.
 // out (a separate n x n buffer) receives inv(i, q) = W[piv[i]][pinv[q]] after the
 // last panel.
-template <int T, int NMAX>
-struct InvSmallLds {
-  static constexpr int LDI = NMAX + PAD;
-  static constexpr int KPI = 32;  // columns per panel: the swept panel and the pivot rows fit in LDS
-  static constexpr int DOUBLES = 4 * KPI * LDI + 2 * NMAX + 16;
-};
-
-template <int T, int NMAX>
-__device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, ldsd* lds) {
-  using C = Cfg<T>;
-  constexpr int LDI = NMAX + PAD, KPI = InvSmallLds<T, NMAX>::KPI;
-  constexpr int MR = C::MR, MC = C::MC, NTH = C::NTH, TA = C::TA, TB = C::TB;
-  constexpr int RT = (NMAX + 63) / 64, CT = KPI / 4;
-  gd2* W = gw(W_);
-  gd2* out = gw(out_);
-  ldsd* Mr = lds;
-  ldsd* Mi = Mr + KPI * LDI;
-  ldsd* Br = Mi + KPI * LDI;
-  ldsd* Bi = Br + KPI * LDI;
-  ldsi* piv = (ldsi*)(Bi + KPI * LDI);
-  ldsi* pinv = piv + NMAX;
-  static_assert(NMAX <= NTH && NTH == 256, "four waves, one snapshot column per thread");
-  static_assert(GjLds<RT, CT, 1>::DOUBLES <= KPI * LDI, "the column exchange fits the snapshot area");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int arow = (wave % C::WR) * 16 * TA, bcol = (wave / C::WR) * 16 * TB;
-  int info = 0;
-  const bool own = tid < n;
-  unsigned used = 0;  // bit r: row lane + 64 r has been a pivot
-  for (int k0 = 0; k0 < n && !info; k0 += KPI) {
-    double2 a[RT][CT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        a[r][c] = lane + 64 * r < n ? W[(size_t)(lane + 64 * r) * n + k0 + wave * CT + c] : make_double2(0, 0);
-    // the exchange uses Br, free until the snapshot below
-    info = gj_sweep<RT, CT, 1>(a, n, used, piv + k0, Br);
-    if (info) {
-      info += k0;
-      break;
-    }
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        if (lane + 64 * r < n) {
-          Mr[(wave * CT + c) * LDI + lane + 64 * r] = a[r][c].x;
-          Mi[(wave * CT + c) * LDI + lane + 64 * r] = a[r][c].y;
-        }
-    __syncthreads();
-    // snapshot of the pivot rows before they are updated: thread j copies column j
-    // of the KPI rows, all its loads in flight at once
-    if (own) {
-      double2 v[KPI];
-#pragma unroll
-      for (int c = 0; c < KPI; ++c) v[c] = W[(size_t)piv[k0 + c] * n + tid];
-#pragma unroll
-      for (int c = 0; c < KPI; ++c) {
-        Br[c * LDI + tid] = v[c].x;
-        Bi[c * LDI + tid] = v[c].y;
-      }
-    }
-    __syncthreads();
-    if (tid < KPI) Mr[tid * LDI + piv[k0 + tid]] -= 1.0;  // M = F - E
-    __syncthreads();
-    const int ntr = n / MR, ntc = n / MC;
-    const int m = lane & 15, kq = lane >> 4;
-    // a thread's element (ti, tj, r) of a tile is W[row0 + arow + kq + ti*16 + 4r][col0 + bcol + m + tj*16]
-    const uint32_t t_off = 16u * (uint32_t)((arow + kq) * n + bcol + m);
-    for (int tile = 0; tile < ntr * ntc; ++tile) {
-      const int row0 = (tile % ntr) * MR, col0 = (tile / ntr) * MC;
-      // W += M W[P, :]: the MFMAs accumulate onto the tile's old values, which are
-      // all requested before the first MFMA waits for them
-      d4 cr[TA][TB], ci[TA][TB];
-#pragma unroll
-      for (int ti = 0; ti < TA; ++ti)
-#pragma unroll
-        for (int tj = 0; tj < TB; ++tj)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const double2 o = ldgb(W_ + (size_t)(row0 + ti * 16 + 4 * r) * n + col0 + tj * 16, t_off);
-            cr[ti][tj][r] = o.x;
-            ci[ti][tj][r] = o.y;
-          }
-      mma_steps<TA, TB, 1, KPI / 4>(cr, ci, Mr, Mi, LDI, row0 + arow, Br, Bi, LDI, col0 + bcol);
-      const bool panel = col0 <= k0 && k0 < col0 + MC;  // the panel's columns take F
-      if (!panel) {
-#pragma unroll
-        for (int ti = 0; ti < TA; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < TB; ++tj)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              stgb(W_ + (size_t)(row0 + ti * 16 + 4 * r) * n + col0 + tj * 16, t_off,
-                   make_double2(cr[ti][tj][r], ci[ti][tj][r]));
-      } else {
-#pragma unroll
-        for (int ti = 0; ti < TA; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < TB; ++tj)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int i = row0 + arow + ti * 16 + 4 * r + kq;
-              const int j = col0 + bcol + tj * 16 + m;
-              const bool inp = j >= k0 && j < k0 + KPI;
-              const int c = inp ? j - k0 : 0;
-              double2 f = make_double2(Mr[c * LDI + i], Mi[c * LDI + i]);
-              f.x += (piv[k0 + c] == i) ? 1.0 : 0.0;
-              const double2 v = inp ? f : make_double2(cr[ti][tj][r], ci[ti][tj][r]);
-              stgb(W_ + (size_t)(row0 + ti * 16 + 4 * r) * n + col0 + tj * 16, t_off, v);
-            }
-      }
-    }
-    __syncthreads();
-  }
-  if (info) {
-    for (int idx = tid; idx < n * n; idx += NTH) out[idx] = make_double2(0, 0);
-    __syncthreads();
-    return info;
-  }
-  for (int q = tid; q < n; q += NTH) pinv[piv[q]] = q;  // inverse permutation
-  __syncthreads();
-  // out(i, q) = W[piv[i]][pinv[q]], RB rows of out at a time: the source rows are
-  // read whole into LDS and out is written in column segments of RB elements
-  constexpr int RB = 16;
-  static_assert(2 * RB * (NMAX + 1) <= 4 * KPI * LDI, "row block fits the panel area");
-  const int ldr = n + 1;  // odd stride: the RB rows of one column sit in distinct banks
-  ldsd* Lr = Mr;
-  ldsd* Li = Mr + RB * ldr;
-  for (int i0 = 0; i0 < n; i0 += RB) {
-    if (own) {  // thread c copies column c of the RB source rows, all loads in flight
-      double2 v[RB];
-#pragma unroll
-      for (int rr = 0; rr < RB; ++rr) v[rr] = W[(size_t)piv[i0 + rr] * n + tid];
-#pragma unroll
-      for (int rr = 0; rr < RB; ++rr) {
-        Lr[rr * ldr + tid] = v[rr].x;
-        Li[rr * ldr + tid] = v[rr].y;
-      }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < RB * n; idx += NTH) {
-      const int rr = idx % RB, q = idx / RB;
-      const int c = pinv[q];
-      out[(size_t)(i0 + rr) + (size_t)q * n] = make_double2(Lr[rr * ldr + c], Li[rr * ldr + c]);
-    }
-    __syncthreads();
-  }
-  return 0;
-}
-
-// -------------------------------------------- inverse, 128 < n <= 256
-// The blocked sweep with 32-column panels.  At these sizes the panel updates read and
-// write the whole of W from HBM (256 workgroups hold 256 MB), so the number of passes
-// counts: 32 columns halve those of a 16-column panel.  The swept panel M = F - E (32 x n)
+//
+// 65 to 256 rows.  From 129 on the panel updates read and write the whole of W from HBM
+// (256 workgroups hold 256 MB), so the number of passes counts: 32 columns halve those of
+// a 16-column panel.  The swept panel M = F - E (32 x n)
 // fills the LDS; W is updated in strips of 16 columns, each with its part of the pivot
 // rows staged beside M, and the next strip is loaded while the current one is multiplied
 // (without that overlap the 32-column panels are slower: 1844 us, below).
@@ -1164,7 +1013,10 @@ __device__ __noinline__ int wg_inverse_small(int n, double2* W_, double2* out_, 
 // Strips belong to the ranks of a group in turn (a lone workgroup has all); every rank
 // sweeps the panel for itself.  A panel's own columns take F one step late, after the
 // ranks have all read the panel.  256 blocks, one per CU, 16-column panels -> this: n = 160
-// 587 -> 553 us, 192 767 -> 776, 224 1287 -> 1159, 256 1624 -> 1527.
+// 587 -> 553 us, 192 767 -> 776, 224 1287 -> 1159, 256 1624 -> 1527.  At 96 and 128 against
+// whole tiles with all of the pivot rows beside M: 184 -> 182 and 304 -> 288 us (8 blocks:
+// 153 -> 149, 245 -> 229): the strips' loads run under the MFMAs, and a panel's own columns
+// are not multiplied.
 template <int NMAX>
 struct InvStripLds {
   static constexpr int KPI = 32, SC = 16;
@@ -1658,19 +1510,19 @@ __device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds
 template <int T, int NMAX>
 struct InvLds {
   static constexpr int DOUBLES = NMAX <= 64    ? InvRegLds<T, NMAX>::DOUBLES
-                                 : NMAX <= 128 ? InvSmallLds<T, NMAX>::DOUBLES
+                                 : NMAX <= 128 ? InvStripLds<128>::DOUBLES
                                  : NMAX <= 256 ? InvStripLds<NMAX>::DOUBLES
                                                : InvBigLds<T, NMAX>::DOUBLES;
 };
 
-// Inverse of an n x n block (n <= NMAX): the whole matrix in registers at 32 and 64, panel and pivot rows in LDS up to 128 rows, the panel alone up to 256, the
-// panels staged through `out` above that.
+// Inverse of an n x n block (n <= NMAX): the whole matrix in registers at 32 and 64, the
+// panel in LDS up to 256 rows, the panels staged through `out` above that.
 template <int T, int NMAX>
 __device__ __forceinline__ int wg_inverse(int n, double2* W, double2* out, ldsd* lds) {
   if constexpr (NMAX == 32 || NMAX == 64) {
     return wg_inverse_reg<T, NMAX>(W, out, lds);  // these variants are chosen for n = NMAX only
   } else if constexpr (NMAX <= 128) {
-    return wg_inverse_small<T, NMAX>(n, W, out, lds);
+    return wg_inverse_strip<128>(n, W, out, lds);
   } else if constexpr (NMAX <= 256) {
     if constexpr (NMAX == 256) {
       if (n <= 192) return wg_inverse_strip<192>(n, W, out, lds);  // no wave multiplies rows past 192

@@ -48,7 +48,6 @@ struct GroupCtl {
   unsigned arrivals, pad0[31];  // low half: workgroups arrived; kClosed: no more join
   unsigned members, pad1[31];   // the number of members, written once
   unsigned barrier, pad2[31];   // arrivals at the barriers, all of them
-  int info[2], pad3[30];        // rank 0's result of an operation, by barrier parity
   double part[2][kMaxTiles];    // partial sums of a GEMM's tiles, by barrier parity
   int lead[2][3];               // a contact's iterations, limit flag, singular inverses
 };
@@ -390,29 +389,16 @@ __device__ __forceinline__ double wg_retrace_prod(GroupN n, const double2* X, co
 }
 
 // ------------------------------------------------------------------ inverse
-// Up to 128 orbitals rank 0 inverts (the column steps are serial and the updates between
-// them short); above, the ranks share the panel updates.
+// Every rank sweeps the panels (the column steps are serial) and updates its own strips.
 template <int NMAX>
 struct InvLds<kGrp, NMAX> {
-  static constexpr int A = InvSmallLds<4, 128>::DOUBLES, B = InvStripLds<256>::DOUBLES;
-  static constexpr int DOUBLES = NMAX <= 128 ? A : B;
+  static constexpr int DOUBLES = InvStripLds<NMAX>::DOUBLES;
 };
 
 template <int T, int NMAX>
 __device__ __forceinline__ int wg_inverse(GroupN n, double2* W, double2* out, ldsd* lds) {
   static_assert(T == kGrp && (NMAX == 128 || NMAX == 256), "group program");
-  if constexpr (NMAX == 128) {
-    const int parity = group_parity(n);
-    GroupCtl* ctl = uni(group_ctx()->ctl);
-    if (group_rank(n) == 0) {
-      const int info = (int)n == 128 ? wg_inverse_small<4, 128>(n, W, out, lds) : wg_inverse_small<3, 96>(n, W, out, lds);
-      if (threadIdx.x == 0) agent_store(&ctl->info[parity], info);
-    }
-    group_barrier();
-    return uni(agent_load(&ctl->info[parity]));
-  } else {
-    return wg_inverse_strip<256>(n, W, out, lds);
-  }
+  return wg_inverse_strip<NMAX>(n, W, out, lds);
 }
 
 // ----------------------------------------------------------------- contacts
