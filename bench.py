@@ -715,7 +715,7 @@ def gw_bench(args):
         "full_band_leg": full,
         "roofline": {"bound": "fp64", "unit": "TFLOP/s", "peak": PEAK_FP64_MFMA,
                      "achieved": fp, "frac": fp / PEAK_FP64_MFMA,
-                     "kernel": "k_polarization<2048> (full band nm=32, 5 slabs, nen=2000)",
+                     "kernel": "k_polarization (full band nm=32, 5 slabs, nen=2000)",
                      "selfenergy_achieved": fs, "selfenergy_frac": fs / PEAK_FP64_MFMA, "traffic": None},
     }
     if not args.no_cpu:
