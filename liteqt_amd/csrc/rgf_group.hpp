@@ -26,7 +26,10 @@
 // A group barrier costs 4 us, 7 to 9 us with the write-back and refetch of the blocks
 // (256 workgroups, groups of 2 to 32), against 84 us for a 128-orbital GEMM and 570 us
 // for a 256-orbital one in one workgroup, and 8 to 18 us for the 32- and 64-orbital ones:
-// groups are for blocks of 96 to 256 orbitals.
+// groups are for blocks of 96 to 256 orbitals.  Members on one XCD share its L2, so their
+// barriers leave the write-back out (read from the hardware when the group closes; 128
+// orbitals, 18 slabs, one energy 9.9 -> 8.9 ms, 40 energies 17.7 -> 15.4; 96 orbitals, 120
+// energies 28.0 -> 24.2).
 #pragma once
 #include "rgf_adjoint.hpp"
 #include "rgf_group_api.hpp"
@@ -45,13 +48,16 @@ constexpr int kMaxTiles = (256 / kGrpTile) * (256 / kGrpTile);
 
 // Control words of one group, zero before the launch.
 struct GroupCtl {
-  unsigned arrivals, pad0[31];  // low half: workgroups arrived; kClosed: no more join
-  unsigned members, pad1[31];   // the number of members, written once
+  unsigned arrivals, pad0[31];  // workgroups arrived, their XCDs (kXcdShift), kClosed: no more join
+  unsigned members, pad1[31];   // the number of members and kOneXcd, written once
   unsigned barrier, pad2[31];   // arrivals at the barriers, all of them
   double part[2][kMaxTiles];    // partial sums of a GEMM's tiles, by barrier parity
   int lead[2][3];               // a contact's iterations, limit flag, singular inverses
 };
-constexpr unsigned kClosed = 1u << 16;
+// Arrivals: count in bits 0 .. 6, kClosed, then the sum of the arrivals' XCD numbers and the
+// sum of their squares: the XCDs are equal where count * squares = sum^2.
+constexpr unsigned kCount = 127u, kClosed = 1u << 7, kOneXcd = 1u << 16;
+constexpr int kXcdShift = 8, kXcdSqShift = 17;  // up to 32 members: 9 and 12 bits
 static_assert(sizeof(GroupCtl) <= kCtlBytes, "control area of a group");
 
 struct GroupCtx {  // in LDS, one per workgroup
@@ -59,6 +65,7 @@ struct GroupCtx {  // in LDS, one per workgroup
   int rank, size;
   unsigned epoch;  // barriers passed
   unsigned half_epoch;  // barriers of this workgroup's half
+  int one_xcd;          // the members share an L2
 };
 
 __device__ __forceinline__ GroupCtx* group_ctx() {
@@ -91,9 +98,10 @@ __device__ __forceinline__ int group_size(GroupN) { return uni(group_ctx()->size
 __device__ __forceinline__ bool group_leader(GroupN) { return group_ctx()->rank == 0; }
 __device__ __forceinline__ int group_parity(GroupN) { return uni((int)(group_ctx()->epoch & 1u)); }
 
-// Barrier of the group: every wave's stores are complete before the workgroup barrier,
-// then one thread writes them back (agent release), counts the workgroup in and waits for
-// the others, and drops the stale cache lines (agent acquire) before anyone reads on.
+// Barrier of the group: every wave's stores are complete (in the L2) before the workgroup
+// barrier, then one thread writes them back where the members do not share the L2 (agent
+// release), counts the workgroup in and waits for the others, and drops the stale cache
+// lines (agent acquire) before anyone reads on.
 __device__ __noinline__ void group_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -101,7 +109,7 @@ __device__ __noinline__ void group_barrier() {
   GroupCtx* c = group_ctx();
   if (threadIdx.x == 0) {
     const unsigned target = ++c->epoch * (unsigned)c->size;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (!c->one_xcd) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __hip_atomic_fetch_add(&c->ctl->barrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     while ((int)(agent_load(&c->ctl->barrier) - target) < 0) __builtin_amdgcn_s_sleep(1);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -116,23 +124,29 @@ __device__ __forceinline__ bool group_join(char* area, int size) {
   GroupCtx* c = group_ctx();
   if (threadIdx.x == 0) {
     GroupCtl* ctl = reinterpret_cast<GroupCtl*>(area);
-    const unsigned r = __hip_atomic_fetch_add(&ctl->arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned x = __builtin_amdgcn_s_getreg((31 << 11) | 20) & (kXcds - 1);  // XCC_ID
+    const unsigned a = __hip_atomic_fetch_add(&ctl->arrivals, 1u + (x << kXcdShift) + (x * x << kXcdSqShift),
+                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     c->ctl = ctl;
     c->epoch = c->half_epoch = 0;
-    c->rank = (int)r;
+    c->rank = (int)(a & kCount);
     c->size = 0;
-    if (r == 0) {
+    unsigned m = 0;
+    if (a == 0) {
       const unsigned long long t0 = wall_clock64();
-      while (agent_load(&ctl->arrivals) < (unsigned)size && wall_clock64() - t0 < (unsigned long long)kJoinTicks)
+      while ((agent_load(&ctl->arrivals) & kCount) < (unsigned)size &&
+             wall_clock64() - t0 < (unsigned long long)kJoinTicks)
         __builtin_amdgcn_s_sleep(1);
-      const unsigned m = __hip_atomic_fetch_add(&ctl->arrivals, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned f = __hip_atomic_fetch_add(&ctl->arrivals, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned sum = (f >> kXcdShift) & 511u, sq = f >> kXcdSqShift;
+      m = f & kCount;
+      if (m * sq == sum * sum) m |= kOneXcd;
       agent_store(&ctl->members, m);
-      c->size = (int)m;
-    } else if (r < kClosed) {
-      unsigned m;
+    } else if (!(a & kClosed)) {
       while ((m = agent_load(&ctl->members)) == 0) __builtin_amdgcn_s_sleep(1);
-      c->size = (int)m;
     }
+    c->size = (int)(m & kCount);
+    c->one_xcd = (m & kOneXcd) != 0;
   }
   __syncthreads();
   return uni(c->size) > 0;
