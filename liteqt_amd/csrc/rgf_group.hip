@@ -25,16 +25,17 @@ hipError_t clear(char* ctl, int ngroups, hipStream_t s) {
 // Microseconds of one energy on a group of G workgroups: the measured times of the block
 // operations as functions of the block size, a slab of 16 GEMMs and an inverse, 18
 // decimation iterations of 6 GEMMs and an inverse per contact, each on half of the group.
-// GEMM from 96 orbitals: barrier 5, 1.6 us per 32 x 32 tile and K panel, or 0.33 us per
-// 128 x 64 tile and k; inverse: rank 0 alone up to 128 orbitals, above it the column steps
-// (475 us at 256) and 62 us per round of the strips.  32 and 64 orbitals run on one
-// workgroup.
+// GEMM from 96 orbitals: barrier 4, 1.6 us per 32 x 32 tile and K panel, or 0.33 us per
+// 128 x 64 tile and k; inverse: the column steps (134 us at 128, 475 at 256) and 12 (128)
+// or 62 us (256) per round of the strips.  32 and 64 orbitals run on one workgroup.
 double item_us(int n, int nx, int G) {
   const int t = n / 32;
   auto us = [&](int gemms, int ranks) {
-    double gemm = 5.0 + ((t * t + ranks - 1) / ranks) * 1.6 * t;
-    double inv = n <= 128 ? 1.85 * n : 475.0 * n / 256 + 62.0 * ((n / 16 + ranks - 1) / ranks) * n * n / 65536.0;
-    if (n % 128 == 0) gemm = std::min(gemm, 5.0 + ((t * t / 8 + ranks - 1) / ranks) * 0.33 * n);
+    const double bar = ranks > 1 ? 4.0 : 0.5;
+    double gemm = bar + ((t * t + ranks - 1) / ranks) * 1.6 * t;
+    const double strip = (n <= 128 ? 12.0 / 16384.0 : 62.0 / 65536.0) * n * n;
+    double inv = (n <= 128 ? 1.05 : 1.85) * n + 4 * bar + ((n / 16 + ranks - 1) / ranks) * strip;
+    if (n % 128 == 0) gemm = std::min(gemm, bar + ((t * t / 8 + ranks - 1) / ranks) * 0.33 * n);
     if (n < 96) {
       gemm = n == 64 ? 14.0 : 6.0;
       inv = 1.2 * n;
