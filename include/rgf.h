@@ -271,7 +271,7 @@ int rgf_graph_create_devices(const rgf_params *p, const rgf_batch *devs, int nde
 
 /* Bytes of device workspace rgf_solve_batched uses for `slots` energies in
  * flight at block size nm and nx slabs.  (An energy solved by several workgroups,
- * where a call has few, takes 6 KB besides, and at nm = 32 and 64 11 blocks.) */
+ * where a call has few, takes 6 KB besides, and at nm = 32 11 blocks.) */
 long long rgf_workspace_bytes(int nm, int nx, int slots);
 
 /* Adjoint (reverse-mode) RGF of the physical-mode device with the scattering

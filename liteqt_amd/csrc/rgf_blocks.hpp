@@ -1454,7 +1454,7 @@ __device__ __noinline__ int wg_inverse_big(int n, double2* W_, double2* out_, ld
 // ------------------------------------------------ inverse, n = 32 or 64
 // The whole matrix held in registers and swept by gj_sweep: at N = 64 lane l of wave w
 // holds row l of columns 16 w .. 16 w + 15, at N = 32 each half wave holds the 32 rows
-// of 4 columns.  No global memory between the load of W and the store of the inverse.
+// of 4 columns.  `store` false: only the result's info.  No global memory between the load of W and the store of the inverse.
 template <int T, int N>
 struct InvRegLds {
   static constexpr int HV = N == 32 ? 2 : 1;
@@ -1466,7 +1466,7 @@ struct InvRegLds {
 };
 
 template <int T, int N>
-__device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds) {
+__device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds, bool store = true) {
   using L = InvRegLds<T, N>;
   constexpr int NTH = Cfg<T>::NTH, C = N * N / NTH, LDO = L::LDO;
   static_assert(NTH == 256 && (N == 32 || N == 64), "register inverse: 256 threads, N = 32 or 64");
@@ -1483,7 +1483,7 @@ __device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds
   unsigned used = 0;
   const int info = gj_sweep<1, C, L::HV>(m, N, used, piv, lds);
   if (info) {
-    for (int idx = tid; idx < N * N; idx += NTH) out[idx] = make_double2(0, 0);
+    for (int idx = tid; store && idx < N * N; idx += NTH) out[idx] = make_double2(0, 0);
     __syncthreads();
     return info;
   }
@@ -1498,7 +1498,7 @@ __device__ __noinline__ int wg_inverse_reg(double2* W_, double2* out_, ldsd* lds
   for (int q = tid; q < N; q += NTH) pinv[piv[q]] = q;
   __syncthreads();
   // out(r, q) = W[piv[r]][pinv[q]], r fastest across the lanes: coalesced column-major stores
-  for (int idx = tid; idx < N * N; idx += NTH) {
+  for (int idx = tid; store && idx < N * N; idx += NTH) {
     const int r = idx % N, q = idx / N;
     const int src = piv[r] * LDO + pinv[q];
     out[idx] = make_double2(Lr[src], Li[src]);

@@ -421,6 +421,7 @@ Split group_split(int n, long long nE, int cus, long long slots, int max_slots) 
   Split sp;
   sp.need = slots;
   const long long rem = nE % cus;
+  if (n < 96 && nE > cus) return sp;  // full rounds of these hold two energies per compute unit
   if (max_slots > 0 || rem == 0 || !rgf::group_plan(n, rem, cus, &sp.g)) return sp;
   sp.tail = rem;
   sp.g.e0 = (int)(nE - rem);

@@ -48,7 +48,7 @@ double item_us(int n, int nx, int G) {
 }  // namespace
 
 bool group_plan(int n, long long nE, int cus, GroupArgs* g) {
-  if (n % 32 != 0 || n < 96 || n > 256 || nE < 1 || cus % kXcds != 0) return false;
+  if (n % 32 != 0 || n < 64 || n > 256 || nE < 1 || cus % kXcds != 0) return false;
   const int per = cus / kXcds;                     // compute units of an XCD
   const int rows = (int)((nE + kXcds - 1) / kXcds);  // groups of an XCD
   if (2 * rows > per) return false;                // two workgroups per energy at the least
@@ -63,7 +63,7 @@ bool group_plan(int n, long long nE, int cus, GroupArgs* g) {
 }
 
 bool pair_plan(int n, long long nE, int cus, GroupArgs* g) {
-  if ((n != 32 && n != 64) || nE < 1 || cus % kXcds != 0) return false;
+  if (n != 32 || nE < 1 || cus % kXcds != 0) return false;
   const int rows = (int)((nE + kXcds - 1) / kXcds);
   if (2 * rows > cus / kXcds) return false;  // a compute unit for each workgroup
   *g = GroupArgs{(int)nE, 2, rows, 0, kXcds * rows * 2, nullptr};
@@ -76,8 +76,6 @@ hipError_t launch_sweep_grp(const SweepArgs& a, const GroupArgs& g, bool od, hip
   if (hipError_t e = clear(g.ctl, g.ngroups, s)) return e;
   if (a.n == 32) {
     hipLaunchKernelGGL((rgf_sweep_pair<kPair32, 32>), dim3(g.grid), dim3(256), 0, s, a, g);
-  } else if (a.n == 64) {
-    hipLaunchKernelGGL((rgf_sweep_pair<kPair64, 64>), dim3(g.grid), dim3(256), 0, s, a, g);
   } else if (od) {
     if (a.n <= 128)
       hipLaunchKernelGGL(rgf_sweep_od_grp<128>, dim3(g.grid), dim3(256), 0, s, a, g);

@@ -25,8 +25,10 @@
 //
 // A group barrier costs 4 us, 7 to 9 us with the write-back and refetch of the blocks
 // (256 workgroups, groups of 2 to 32), against 84 us for a 128-orbital GEMM and 570 us
-// for a 256-orbital one in one workgroup, and 8 to 18 us for the 32- and 64-orbital ones:
-// groups are for blocks of 96 to 256 orbitals.  Members on one XCD share its L2, so their
+// for a 256-orbital one in one workgroup, 18 us for a 64-orbital and 8 for a 32-orbital one:
+// groups are for blocks of 64 to 256 orbitals (64 orbitals, 20 slabs against a lone workgroup
+// with a second one for the right contact: one energy 5.6 -> 3.9 ms, 60 energies 7.0 -> 5.5,
+// 100 in groups of two 7.1 either way).  Members on one XCD share its L2, so their
 // barriers leave the write-back out (read from the hardware when the group closes; 128
 // orbitals, 18 slabs, one energy 9.9 -> 8.9 ms, 40 energies 17.7 -> 15.4; 96 orbitals, 120
 // energies 28.0 -> 24.2).
@@ -403,7 +405,8 @@ __device__ __forceinline__ double wg_retrace_prod(GroupN n, const double2* X, co
 }
 
 // ------------------------------------------------------------------ inverse
-// Every rank sweeps the panels (the column steps are serial) and updates its own strips.
+// Every rank sweeps the panels (the column steps are serial) and updates its own strips; at 64
+// orbitals every rank sweeps the whole block in registers and rank 0 stores it.
 template <int NMAX>
 struct InvLds<kGrp, NMAX> {
   static constexpr int DOUBLES = InvStripLds<NMAX>::DOUBLES;
@@ -412,6 +415,11 @@ struct InvLds<kGrp, NMAX> {
 template <int T, int NMAX>
 __device__ __forceinline__ int wg_inverse(GroupN n, double2* W, double2* out, ldsd* lds) {
   static_assert(T == kGrp && (NMAX == 128 || NMAX == 256), "group program");
+  if (NMAX == 128 && (int)n == 64) {
+    const int info = wg_inverse_reg<2, 64>(W, out, lds, group_rank(n) == 0);
+    group_barrier();
+    return info;
+  }
   return wg_inverse_strip<NMAX>(n, W, out, lds);
 }
 
@@ -473,13 +481,9 @@ struct Leads<kGrp, NMAX> : LeadsBase {
   }
 };
 
-// At 32 and 64 orbitals a block operation is too short to share, but the right contact's
+// At 32 orbitals a block operation is too short to share, but the right contact's
 // decimation is not needed before the forward sweep is over: in a group of two, rank 1 runs
 // it and leaves, rank 0 runs the rest of the program.
-constexpr int kPair64 = 66;
-template <>
-struct Cfg<kPair64> : Cfg<2> {};
-
 template <int T, int NMAX>
 struct PairLeads {
   static constexpr int kRightTemp = kTmpBlocks;
@@ -522,8 +526,6 @@ struct PairLeads {
 };
 template <>
 struct Leads<kPair32, 32> : PairLeads<kPair32, 32> {};
-template <>
-struct Leads<kPair64, 64> : PairLeads<kPair64, 64> {};
 
 // ------------------------------------------------------------------ kernels
 template <int T, int NMAX>

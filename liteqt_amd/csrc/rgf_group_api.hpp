@@ -43,7 +43,7 @@ struct MultiGroupPlan {
 // Groups for nE energies of n orbitals on `cus` compute units; false where one workgroup
 // per energy is the faster (or only) form.
 bool group_plan(int n, long long nE, int cus, GroupArgs* g);
-// 32 and 64 orbitals: two workgroups for each of nE energies (launch_sweep_grp, without
+// 32 orbitals: two workgroups for each of nE energies (launch_sweep_grp, without
 // block-tridiagonal Sigma); a slot has kPairExtra more blocks.
 bool pair_plan(int n, long long nE, int cus, GroupArgs* g);
 constexpr int kPairExtra = 11;

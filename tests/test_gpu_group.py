@@ -1,5 +1,5 @@
-"""GPU: an energy solved by a group of workgroups (blocks of 96 to 256 orbitals, few
-energies; at 32 and 64 orbitals a second workgroup for the right contact) against the one-workgroup solve of the same energy, which a caller's slot limit
+"""GPU: an energy solved by a group of workgroups (blocks of 64 to 256 orbitals, few
+energies; at 32 orbitals a second workgroup for the right contact) against the one-workgroup solve of the same energy, which a caller's slot limit
 selects.  Both form every output element from the same products in the same order; the
 bound is the rounding of one reordering, n eps times the conditioning at eta = 1e-3
 (256 * 1.1e-16 * 1e2 < 1e-11), relative per output array."""
@@ -32,8 +32,8 @@ def _close(a, b, name):
 
 
 # one energy takes the largest group, 9 energies two groups an XCD, 40 the smallest tiles
-# per rank with every variant of the inverse; 300 leaves a tail of 44 behind a full round; 32 and
-# 64 orbitals in pairs, 128 energies the most
+# per rank with every variant of the inverse; 300 leaves a tail of 44 behind a full round; 32
+# orbitals in pairs, 128 energies the most
 @pytest.mark.parametrize("nm,nE", [(96, 1), (96, 40), (128, 1), (128, 9), (160, 3), (192, 9), (224, 1), (256, 1), (256, 17),
                                    (96, 300), (32, 1), (32, 128), (64, 1), (64, 9)])
 @pytest.mark.parametrize("mode", ["compat", "physical"])
