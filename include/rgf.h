@@ -178,6 +178,12 @@ typedef struct rgf_batch {
   double *GRi1_lo;
 } rgf_batch;
 
+/* The workspace of the calls on device arrays (this one, rgf_scba_step,
+ * rgf_solve_two_lesser, rgf_solve_devices, rgf_adjoint_batched, rgf_w_solve_batched,
+ * rgf_zinv_batched) is shared per GPU and serves one of them at a time: a call's work
+ * waits on the device for that of the call before it, whatever streams or host threads
+ * they come from.  A call captured into a graph of the caller's is outside of this
+ * order: its replay must not overlap other calls. */
 int rgf_solve_batched(const rgf_params *p, const rgf_batch *b, void *stream);
 
 /* rgf_solve_batched without any allocation: no counterpart in the reference.

@@ -1060,9 +1060,9 @@ __device__ __noinline__ int wg_inverse_strip(N n_, double2* W_, double2* out_, l
       }
     }
   };
-  int info = 0;
+  int info = 0, k0 = 0;
   unsigned used = 0;  // bit r: row lane + 64 r has been a pivot
-  for (int k0 = 0; k0 < n; k0 += KPI) {
+  for (; k0 < n; k0 += KPI) {
     double2 a[RT][CT];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
@@ -1162,6 +1162,8 @@ __device__ __noinline__ int wg_inverse_strip(N n_, double2* W_, double2* out_, l
     }
     group_sync(n_);
   }
+  // a group's barriers do not depend on the block: after a panel without a pivot the rest follow
+  for (; k0 < n; k0 += KPI) group_sync(n_);
   if (!info) {
     late(n - KPI);
     for (int q = tid; q < n; q += NTH) pinv[piv[q]] = q;  // inverse permutation

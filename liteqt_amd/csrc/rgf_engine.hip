@@ -74,6 +74,39 @@ constexpr int kMaxDev = 16;
 Buf g_ws[kMaxDev];
 std::mutex g_ws_mu;
 
+// The shared workspaces (g_ws, g_ctl, g_adj_dh) serve one launch at a time: a launch on any
+// stream waits for the event behind the previous launch that used them, and leaves its own.
+// Held with g_ws_mu from before the first use of the workspace to after the last launch.
+// A stream under capture neither waits nor records (an event of a capture cannot order work
+// outside of it); `capturing` tells, and such a launch stays off g_ctl.
+hipEvent_t g_ws_event[kMaxDev];
+class WsTurn {
+ public:
+  bool capturing = false;
+  int begin(int dev, hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+    capturing = st != hipStreamCaptureStatusNone;
+    if (capturing) return 0;
+    hipEvent_t& ev = g_ws_event[dev];
+    if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    HIPCHK(hipStreamWaitEvent(s, ev, 0));  // (nothing to wait for before its first record)
+    ev_ = ev;
+    s_ = s;
+    return 0;
+  }
+  ~WsTurn() {
+    if (ev_ && hipEventRecord(ev_, s_) != hipSuccess) {
+      (void)hipGetLastError();
+      (void)hipStreamSynchronize(s_);
+    }
+  }
+
+ private:
+  hipEvent_t ev_ = nullptr;
+  hipStream_t s_ = nullptr;
+};
+
 // Copy nblocks n x n blocks into np x np blocks (np >= n): zero padding and
 // `fill` on the padded diagonal, which keeps the padded orbitals decoupled and
 // every padded slab matrix invertible.
@@ -107,6 +140,10 @@ __global__ void unpad_blocks(const V* __restrict__ src, int np, V* __restrict__ 
 Buf g_stage[kMaxDev];
 rgf::PinnedAreas g_pinned[kMaxDev];  // guarded by g_mu, as g_stage
 Buf g_adj_dh[kMaxDev];
+// Control words of the groups (rgf_group.hpp).  Apart from g_ws: a caller's captured launch
+// may run with other calls when it is replayed, and then spoils their slots, but never the
+// counters that a group's members wait on.
+Buf g_ctl[kMaxDev];
 
 typedef void (*AdjLaunch)(const rgf::AdjArgs&, int grid, hipStream_t);
 template <int T, int NMAX>
@@ -411,18 +448,29 @@ void fill_args(const rgf_params* p, const rgf_batch* b, long long se, rgf::Sweep
 // left over when full rounds of one energy per compute unit are taken off, where they
 // leave at least half of the compute units idle.  The rounds run first, then the groups,
 // on the same slots; `need` is the number of slots for both.  A caller that limits the
-// slots keeps one workgroup per energy.
+// slots, or launches under capture (no control areas, ctl null), keeps one workgroup per
+// energy.
 struct Split {
   long long tail = 0, need = 0;
   rgf::GroupArgs g{};
-  size_t ctl_bytes() const { return (size_t)tail * rgf::kGroupCtlBytes; }
 };
-Split group_split(int n, long long nE, int cus, long long slots, int max_slots) {
+
+// The control areas of one launch's groups (at most one group per compute unit); null where
+// they cannot be allocated, and the launch keeps one workgroup per energy.
+char* group_ctl(int dev, int cus) {
+  if (g_ctl[dev].ensure(rgf::kGroupCtlBytes * (size_t)cus)) {
+    (void)hipGetLastError();
+    g_err.clear();
+  }
+  return reinterpret_cast<char*>(g_ctl[dev].p);
+}
+Split group_split(int n, long long nE, int cus, long long slots, int max_slots, char* ctl) {
   Split sp;
   sp.need = slots;
   const long long rem = nE % cus;
   if (n < 96 && nE > cus) return sp;  // full rounds of these hold two energies per compute unit
-  if (max_slots > 0 || rem == 0 || !rgf::group_plan(n, rem, cus, &sp.g)) return sp;
+  if (!ctl || max_slots > 0 || rem == 0 || !rgf::group_plan(n, rem, cus, &sp.g)) return sp;
+  sp.g.ctl = ctl;
   sp.tail = rem;
   sp.g.e0 = (int)(nE - rem);
   sp.need = std::max(rem, std::min<long long>(nE - rem, cus));
@@ -436,23 +484,28 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
   if (int rc = prepare(p, b, scba, &pr, second)) return rc;
   if (pr.nothing) return 0;
   const bool od = has_offdiag(b) || scba || second;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   long long slot_bytes = pr.slot_elems * 16LL;
-  Split sp = group_split(b->nm, b->nE, pr.cus, pr.slots, b->max_slots);
+  std::lock_guard<std::mutex> lk(g_ws_mu);
+  WsTurn turn;
+  if (int rc = turn.begin(pr.dev, s)) return rc;
+  char* ctl = turn.capturing ? nullptr : group_ctl(pr.dev, pr.cus);
+  Split sp = group_split(b->nm, b->nE, pr.cus, pr.slots, b->max_slots, ctl);
   const long long pair_extra = (long long)rgf::kPairExtra * b->nm * b->nm;
-  if (!od && !b->Sii && b->max_slots <= 0 && rgf::pair_plan(b->nm, b->nE, pr.cus, &sp.g)) {
+  if (ctl && !od && !b->Sii && b->max_slots <= 0 && rgf::pair_plan(b->nm, b->nE, pr.cus, &sp.g)) {
+    sp.g.ctl = ctl;
     sp.tail = sp.need = b->nE;
     pr.a.ws_slot += pair_extra;
     slot_bytes += pair_extra * 16LL;
   }
-  std::lock_guard<std::mutex> lk(g_ws_mu);
   Buf& ws = g_ws[pr.dev];
-  if ((size_t)(sp.need * slot_bytes) + sp.ctl_bytes() > ws.bytes) {
+  if ((size_t)(sp.need * slot_bytes) > ws.bytes) {
     // HBM admission: fit the stored left-connected blocks into free memory
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     const size_t avail = (size_t)((double)(fr + ws.bytes) * 0.9);
     long long fit = (long long)(avail / (size_t)slot_bytes);
-    if (sp.tail && (size_t)(sp.need * slot_bytes) + sp.ctl_bytes() > avail) {
+    if (sp.tail && (size_t)(sp.need * slot_bytes) > avail) {
       sp = Split();  // one workgroup per energy, on the slots that fit
       sp.need = pr.slots;
       pr.a.ws_slot = pr.slot_elems;
@@ -476,13 +529,12 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
     }
     if (fit < 1) return fail(RGF_ENOMEM, "not enough device memory for one energy slot");
     sp.need = std::min(sp.need, fit);
-    const size_t bytes = (size_t)(sp.need * slot_bytes) + sp.ctl_bytes();
+    const size_t bytes = (size_t)(sp.need * slot_bytes);
     if (bytes > ws.bytes) {
       ws.release();
       if (int rc = ws.ensure(bytes)) return rc;
     }
   }
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   pr.a.ws = reinterpret_cast<double2*>(ws.p);
   if (sp.tail < b->nE) {
     rgf::SweepArgs a = pr.a;
@@ -491,7 +543,6 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
     HIPCHK(hipGetLastError());
   }
   if (sp.tail) {
-    sp.g.ctl = reinterpret_cast<char*>(ws.p) + (size_t)(sp.need * slot_bytes);
     HIPCHK(rgf::launch_sweep_grp(pr.a, sp.g, od, s));
   }
   return 0;
@@ -926,6 +977,8 @@ int rgf_solve_devices(const rgf_params* p, const rgf_batch* devs, int ndev, int 
   // the descriptor buffer and workspace are reused: let earlier launches finish
   HIPCHK(hipDeviceSynchronize());
   std::lock_guard<std::mutex> lw(g_ws_mu);
+  WsTurn turn;
+  if (int rc = turn.begin(dev, s)) return rc;
   Buf& ws = g_ws[dev];
   MultiPlan pl;
   if (int rc = multi_plan(p, devs, ndev, autotune, 0, s, &pl, ws.bytes)) return rc;
@@ -1448,13 +1501,17 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
   const long long dh_bytes = (long long)b->nx * nn * 16LL;
   long long slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
   if (b->max_slots > 0) slots = std::min<long long>(slots, b->max_slots);
-  Split sp = group_split(b->nm, b->nE, prop.multiProcessorCount, slots, b->max_slots);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  std::lock_guard<std::mutex> lk(g_ws_mu);
+  WsTurn turn;
+  if (int rc = turn.begin(dev, s)) return rc;
+  const int cus = prop.multiProcessorCount;
+  Split sp = group_split(b->nm, b->nE, cus, slots, b->max_slots, turn.capturing ? nullptr : group_ctl(dev, cus));
   slots = sp.need;
   // The larger slot (R, R d and g S kept per slab: 5 fewer GEMMs per slab) is used
   // when every slot still fits; otherwise the small slot, recomputing them.
   const long long keep_bytes = rgf::adj_slot_blocks(b->nx, 1) * nn * 16LL;
   const long long small_bytes = rgf::adj_slot_blocks(b->nx, 0) * nn * 16LL;
-  std::lock_guard<std::mutex> lk(g_ws_mu);
   Buf& ws = g_ws[dev];
   Buf& dh = g_adj_dh[dev];
   // LITEQT_ADJ_RECOMPUTE=1 forces the small slot (the path taken under memory pressure)
@@ -1465,11 +1522,11 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
   int K = b->ckpt > 0 ? b->ckpt : 0;
   if (K) keep = 0;
   long long slot_bytes = K ? rgf::adj_slot_blocks(b->nx, 0, K) * nn * 16LL : keep ? keep_bytes : small_bytes;
-  if ((size_t)(slots * slot_bytes) + sp.ctl_bytes() > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
+  if ((size_t)(slots * slot_bytes) > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     const size_t avail = (size_t)((double)(fr + ws.bytes + dh.bytes) * 0.9);
-    if (sp.tail && (size_t)(slots * ((K ? slot_bytes : small_bytes) + dh_bytes)) + sp.ctl_bytes() > avail) {
+    if (sp.tail && (size_t)(slots * ((K ? slot_bytes : small_bytes) + dh_bytes)) > avail) {
       slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
       sp = Split();  // one workgroup per energy, on the slots that fit
     }
@@ -1490,14 +1547,13 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
     }
     if (fit < 1) return fail(RGF_ENOMEM, "not enough device memory for one adjoint slot");
     slots = std::min(slots, fit);
-    if ((size_t)(slots * slot_bytes) + sp.ctl_bytes() > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
+    if ((size_t)(slots * slot_bytes) > ws.bytes || (size_t)(slots * dh_bytes) > dh.bytes) {
       ws.release();
       dh.release();
-      if (int rc = ws.ensure((size_t)(slots * slot_bytes) + sp.ctl_bytes())) return rc;
+      if (int rc = ws.ensure((size_t)(slots * slot_bytes))) return rc;
       if (int rc = dh.ensure((size_t)(slots * dh_bytes))) return rc;
     }
   }
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   HIPCHK(hipMemsetAsync(dh.p, 0, (size_t)(slots * dh_bytes), s));
   rgf::AdjArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -1527,7 +1583,6 @@ int rgf_adjoint_batched(const rgf_params* p, const rgf_batch* b, const double* w
   }
   if (sp.tail) {
     a.nE = b->nE;
-    sp.g.ctl = reinterpret_cast<char*>(ws.p) + (size_t)(slots * slot_bytes);
     HIPCHK(rgf::launch_adjoint_grp(a, sp.g, s));
   }
   if (dH1i) {
@@ -1571,10 +1626,13 @@ int rgf_zinv_batched(int n, int nbatch, const double* A, double* Ainv, int* info
   const int grid = std::min(nbatch, 1024);
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDev) return fail(RGF_EINVAL, "device index out of range");
   std::lock_guard<std::mutex> lk(g_ws_mu);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  WsTurn turn;
+  if (int rc = turn.begin(dev, s)) return rc;
   // the row-major work buffers live in the engine workspace
   if (int rc = g_ws[dev].ensure((size_t)grid * n * n * 16)) return rc;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const double2* a = reinterpret_cast<const double2*>(A);
   double2* o = reinterpret_cast<double2*>(Ainv);
   double2* w = reinterpret_cast<double2*>(g_ws[dev].p);
@@ -1628,6 +1686,8 @@ int rgf_w_solve_batched(const rgf_w_batch* b, void* stream) {
   const size_t pad_el = pad ? nn * (2 * (size_t)nx + (b->WRi1 ? 7 : 6) * (size_t)nblk) : 0;
   const long long slot_el = (long long)rgf::kWTmpBlocks * (long long)nn;
   std::lock_guard<std::mutex> lk(g_ws_mu);
+  WsTurn turn;
+  if (int rc = turn.begin(dev, s)) return rc;
   Buf& ws = g_ws[dev];
   size_t fr = 0, tot = 0;
   HIPCHK(hipMemGetInfo(&fr, &tot));
@@ -1635,14 +1695,15 @@ int rgf_w_solve_batched(const rgf_w_batch* b, void* stream) {
   const size_t avail = (size_t)((double)(fr + ws.bytes) * 0.9);
   if (avail <= fixed) return fail(RGF_ENOMEM, "rgf_w_solve_batched: not enough device memory for the padded blocks");
   long long slots = std::min<long long>(b->nE, (long long)prop.multiProcessorCount * per_cu);
-  Split sp = group_split(np, b->nE, prop.multiProcessorCount, slots, 0);
-  if (sp.tail && fixed + (size_t)sp.need * slot_el * sizeof(double2) + sp.ctl_bytes() > avail) {
+  const int cus = prop.multiProcessorCount;
+  Split sp = group_split(np, b->nE, cus, slots, 0, turn.capturing ? nullptr : group_ctl(dev, cus));
+  if (sp.tail && fixed + (size_t)sp.need * slot_el * sizeof(double2) > avail) {
     sp = Split();  // one workgroup per energy, on the slots that fit
     sp.need = slots;
   }
   slots = std::min<long long>(sp.need, (long long)((avail - fixed) / (slot_el * sizeof(double2))));
   if (slots < 1) return fail(RGF_ENOMEM, "rgf_w_solve_batched: not enough device memory for one energy slot");
-  if (int rc = ws.ensure(fixed + (size_t)slots * slot_el * sizeof(double2) + sp.ctl_bytes())) return rc;
+  if (int rc = ws.ensure(fixed + (size_t)slots * slot_el * sizeof(double2))) return rc;
   double2* base = reinterpret_cast<double2*>(ws.p);
   rgf::WArgs a{};
   a.n = np;
@@ -1693,7 +1754,6 @@ int rgf_w_solve_batched(const rgf_w_batch* b, void* stream) {
   }
   if (sp.tail) {
     a.nE = b->nE;
-    sp.g.ctl = reinterpret_cast<char*>(a.ws + (size_t)slots * slot_el);
     HIPCHK(rgf::launch_wsweep_grp(a, sp.g, s));
   }
   if (pad) {
@@ -1745,6 +1805,7 @@ void rgf_release(void) {
   g_ws[dev].release();
   g_stage[dev].release();
   g_adj_dh[dev].release();
+  g_ctl[dev].release();
   g_pinned[dev].release();
 }
 

@@ -48,7 +48,7 @@ bool group_plan(int n, long long nE, int cus, GroupArgs* g);
 bool pair_plan(int n, long long nE, int cus, GroupArgs* g);
 constexpr int kPairExtra = 11;
 
-// Clear the control areas (a kernel, so that the launch can be captured) and launch.
+// Clear the control areas and launch.  The areas belong to the launch until it ends.
 hipError_t launch_sweep_grp(const SweepArgs& a, const GroupArgs& g, bool od, hipStream_t s);
 hipError_t launch_adjoint_grp(const AdjArgs& a, const GroupArgs& g, hipStream_t s);
 hipError_t launch_wsweep_grp(const WArgs& a, const GroupArgs& g, hipStream_t s);
