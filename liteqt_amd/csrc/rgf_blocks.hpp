@@ -452,13 +452,21 @@ struct EpiMode {
   static constexpr int value = M;
 };
 
-// The output tiles rank, rank + size, ...; returns this thread's part of sum |C_ij|.
-template <int T, int OPA, int OPB, int CRM>
+// The output tiles rank, rank + size, ...; returns this thread's part of sum |C_ij|.  Given
+// `sums`, each macro tile's parts go there as well: sums(row of the wave's part, its column,
+// in lane ti TB + tj the sum over the part's 16 x 16 tile (ti, tj)).
+struct NoSums {
+  __device__ void operator()(int, int, double) const {}
+};
+__device__ __forceinline__ double cabs_plain(double2 v) { return sqrt(fma(v.y, v.y, v.x * v.x)); }
+
+template <int T, int OPA, int OPB, int CRM, typename Sums = NoSums>
 __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__ A_, const double2* __restrict__ B_,
-                                             void* Cout_, Epi ep_, ldsd* lds, int rank, int size) {
+                                             void* Cout_, Epi ep_, ldsd* lds, int rank, int size,
+                                             const Sums& sums = Sums()) {
   using C = Cfg<T>;
   constexpr int MR = C::MR, MC = C::MC, LDA = C::LDA, LDB = C::LDB, STAGE = C::STAGE, TA = C::TA, TB = C::TB;
-  constexpr bool AKC = (OPA != OP_N), BKC = (OPB == OP_N);
+  constexpr bool AKC = (OPA != OP_N), BKC = (OPB == OP_N), kSums = !__is_same(Sums, NoSums);
   const int n = uni(n_);
   const double2* A = uni(A_);
   const double2* B = uni(B_);
@@ -546,6 +554,7 @@ __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__
           for (int r = 0; r < 4; ++r) d3[r] = ldgb(ep.D3 + tr0 + dj(tj, r) + (size_t)di(ti, r) * n, 16u * t_tr);
         }
       };
+      double part = 0.0;
       double2 n1[4], n2[4], n3[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) n1[r] = n2[r] = n3[r] = make_double2(0, 0);
@@ -553,6 +562,7 @@ __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__
 #pragma unroll
       for (int b = 0; b < TA * TB; ++b) {
         const int ti = b / TB, tj = b % TB;
+        double sum = 0.0;
         double2 c1[4], c2[4], c3[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) { c1[r] = n1[r]; c2[r] = n2[r]; c3[r] = n3[r]; }
@@ -569,7 +579,11 @@ __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__
             if (ep.D1) v = cadd(v, cmul(ep.s1, c1[r]));
             if (ep.D2) v = cadd(v, cmul(ep.s2, c2[r]));
             if (ep.D3) v = cadd(v, cmul(ep.s3, cconj(c3[r])));
-            if (ep.abs_sum) asum += sqrt(v.y * v.y + v.x * v.x);
+            if (ep.abs_sum) {
+              const double m = cabs_plain(v);
+              asum += m;
+              sum += m;
+            }
           }
           const size_t u = CRM ? tr0 + dj(tj, r) + (size_t)di(ti, r) * n : cm0 + di(ti, r) + (size_t)dj(tj, r) * n;
           if (MODE == 2 && ep.real_out)
@@ -577,6 +591,15 @@ __device__ __forceinline__ double gemm_tiles(int n_, const double2* __restrict__
           else
             stgb((double2*)Cout + u, 16u * t_out, v);
         }
+        if constexpr (kSums && MODE == 2) {
+          if (ep.abs_sum) {
+            sum = wave_sum(sum);
+            part = lane == b ? sum : part;
+          }
+        }
+      }
+      if constexpr (kSums && MODE == 2) {
+        if (ep.abs_sum) sums(row0 + arow, col0 + bcol, part);
       }
     };
     if (emode == 0)

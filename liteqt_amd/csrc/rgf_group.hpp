@@ -11,9 +11,11 @@
 //
 // Results do not depend on the number of ranks: an output element is formed by one wave
 // from the same products in the same order as in the one-workgroup kernels, reductions
-// over a block are formed by every rank for itself, and the one sum that is split (the
-// decimation's sum of |C_ij|, which is only compared with the tolerance) is added in the
-// order of its tiles.
+// over a block are formed by every rank for itself, and the one sum that is split (the sum of
+// |C_ij| that the decimation and the contacts' Stein equations compare with their tolerances)
+// is made of the same parts, one per 32 x 32 tile, added in the order of the tiles, whatever
+// the GEMM's tiles are.  (The one-workgroup kernels add it in another order, so that next to
+// the tolerance the two may differ by an iteration.)
 //
 // Membership.  A group is formed by the workgroups that have arrived when its first one
 // closes it, so no workgroup ever waits for one that is not running, whatever else
@@ -192,24 +194,35 @@ __device__ __forceinline__ bool large_tiles(int n, int size) {
   return 13 * ((large + size - 1) / size) < 2 * ((small + size - 1) / size);
 }
 
+// The parts of a sum, one per tile (at most a wave's lanes), added in the order of the tiles.
+__device__ __forceinline__ double tile_sum(const double* part, int ntiles) {
+  static_assert(kMaxTiles <= 64, "a lane for each tile");
+  const int lane = threadIdx.x & 63;
+  const double v = lane < ntiles ? agent_load(part + lane) : 0.0;
+  double s = 0.0;
+  for (int t = 0; t < ntiles; ++t) s += lane_f64(v, t);
+  return s;
+}
+
 template <int OPA, int OPB, int CRM>
 __device__ __noinline__ double grp_gemm_large(GroupN n_, const double2* __restrict__ A, const double2* __restrict__ B,
                                               void* Cout, Epi ep, ldsd* lds) {
   const int rank = group_rank(n_), size = group_size(n_), parity = group_parity(n_);
   GroupCtl* ctl = uni(group_ctx()->ctl);
-  const double asum = gemm_tiles<4, OPA, OPB, CRM>((int)n_, A, B, Cout, ep, lds, rank, size);
-  const int sum = uni(ep.abs_sum);
-  if (sum) {
-    __syncthreads();
-    const double s = block_sum(asum, lds);
-    if (threadIdx.x == 0) agent_store(&ctl->part[parity][rank], s);
-  }
+  const int nt = uni((int)n_) / kGrpTile;
+  // a wave's 64 x 32 part is two of the sum's tiles; each is added as grp_gemm's waves add it
+  auto sums = [&](int row, int col, double part) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const double s = ((lane_f64(part, 4 * a) + lane_f64(part, 4 * a + 2)) + lane_f64(part, 4 * a + 1)) +
+                       lane_f64(part, 4 * a + 3);
+      if ((threadIdx.x & 63) == 0) agent_store(&ctl->part[parity][row / kGrpTile + a + col / kGrpTile * nt], s);
+    }
+  };
+  static_assert(Cfg<4>::TA == 4 && Cfg<4>::TB == 2, "two 32 x 32 tiles per wave");
+  gemm_tiles<4, OPA, OPB, CRM>((int)n_, A, B, Cout, ep, lds, rank, size, sums);
   group_barrier();
-  double s = 0.0;
-  if (sum) {
-    for (int r = 0; r < size; ++r) s += agent_load(&ctl->part[parity][r]);
-  }
-  return s;
+  return uni(ep.abs_sum) ? tile_sum(ctl->part[parity], nt * nt) : 0.0;
 }
 
 template <int OPA, int OPB, int CRM>
@@ -321,7 +334,7 @@ __device__ __noinline__ double grp_gemm(GroupN n_, const double2* __restrict__ A
       if (ep.D1) v = cadd(v, cmul(ep.s1, d1[r]));
       if (ep.D2) v = cadd(v, cmul(ep.s2, d2[r]));
       if (ep.D3) v = cadd(v, cmul(ep.s3, cconj(d3[r])));
-      if (ep.abs_sum) asum += sqrt(v.y * v.y + v.x * v.x);
+      if (ep.abs_sum) asum += cabs_plain(v);
       const uint32_t u = (uint32_t)(CRM ? j + i * n : i + j * n);
       if (ep.real_out)
         stgb_re((double*)Cout, 8u * u, v.x);
@@ -342,11 +355,7 @@ __device__ __noinline__ double grp_gemm(GroupN n_, const double2* __restrict__ A
     if (s + 1 < steps) step(Index<1>(), s + 1);
   }
   group_barrier();
-  double s = 0.0;
-  if (ep.abs_sum) {
-    for (int t = 0; t < ntiles; ++t) s += agent_load(&ctl->part[parity][t]);
-  }
-  return s;
+  return ep.abs_sum ? tile_sum(ctl->part[parity], ntiles) : 0.0;
 }
 
 template <int T, int OPA, int OPB, int CRM>

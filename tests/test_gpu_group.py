@@ -155,3 +155,29 @@ def test_group_devices_equal_one_workgroup(counts):
         assert torch.equal(d["out"]["info"], r["info"])
         _close(d["out"]["tr"], r["tr"], "tr")
         _close(d["out"]["dens_n"], r["dens_n"], "dens_n")
+
+
+def _decimation_sum(nm, nE):
+    """The left contact's sum of |C_ij| after one iteration, to the bit, as each of nE equal
+    energies forms it: the smallest tolerance that it passes."""
+    torch, configs, rgf, H, C, _ = _device(nm, 2, 1, 10 + nm)
+    E = torch.full((nE,), 0.1, dtype=torch.float64, device="cuda")
+    info = torch.zeros(nE, 4, dtype=torch.int32, device="cuda")
+    lo, hi = np.zeros(nE, np.int64), np.full(nE, np.float64(1e30).view(np.int64))  # fails, passes
+    while (hi - lo).max() > 1:
+        mid = lo + (hi - lo) // 2  # (the sum of two such patterns passes 63 bits)
+        e = int((hi - lo).argmax())
+        rgf.solve_batched(rgf.params(rgf.MODE_PHYSICAL, eta_dev=1e-3, dec_nmax=1, dec_tol=float(mid[e:e + 1].view(np.float64)[0])),
+                          E, (300.0, 300.0), (0.1, -0.1), H, C, out={"info": info})
+        passed = (info[:, 2].cpu().numpy() & 1) == 0
+        hi = np.where(passed & (mid[e] < hi), mid[e], hi)
+        lo = np.where(~passed & (mid[e] > lo), mid[e], lo)
+    return hi
+
+
+# groups whose GEMMs take 32 x 32 tiles (one energy, 16 or 32 ranks) and 128 x 64 tiles (many
+# energies, 2 or 4 ranks): the sum that ends the decimation is the same, to the bit
+@pytest.mark.parametrize("nm,many", [(128, 128), (256, 64)])
+def test_decimation_sum_does_not_depend_on_the_group(nm, many):
+    one, sums = _decimation_sum(nm, 1), _decimation_sum(nm, many)
+    assert (sums == one[0]).all(), (one[:1].view(np.float64), sums.view(np.float64))
