@@ -296,13 +296,18 @@ def solve_batched(p, E, temp, mu, Hii, H1i, sigL=None, sigR=None, out=None, max_
     refreshes the given Sigma tensors in place (rgf_scba_step).  ckpt: storage of
     the left-connected blocks (rgf_batch.ckpt: -1 every slab, K > 0 checkpoints every
     K slabs with segment recompute, 0 automatic).  second: dict sigL, sigL_up, ndens of
-    a second lesser source carried along (rgf_solve_two_lesser; physical mode, Sigma per
-    energy as the others).  Asynchronous on `stream` (default: torch's current stream)."""
+    a second lesser source carried along (rgf_solve_two_lesser; physical mode, its Sigma
+    per energy or shared as the others').  Asynchronous on `stream` (default: torch's current stream)."""
     import torch
     out = out or {}
     b = _batch(torch, E, temp, mu, Hii, H1i, sigL, sigR, max_slots, sigR_lo, sigR_up, sigL_up)
     b.ckpt = int(ckpt)
     _out_batch(torch, b, out, E.device)
+    sec = None
+    if second is not None:
+        if plain or scba is not None:
+            raise RgfError(f"second: the {'plain path' if plain else 'SCBA refresh'} takes one lesser source")
+        sec = _second(torch, b, second, any(t is not None for t in (sigL, sigR, sigR_lo, sigR_up, sigL_up)), E.device)
     if stream is None:
         stream = torch.cuda.current_stream()
     if plain:
@@ -310,14 +315,7 @@ def solve_batched(p, E, temp, mu, Hii, H1i, sigL=None, sigR=None, out=None, max_
         if rc != 0:
             raise RgfError(f"plain path error {rc}: {plain_lib().rgf_plain_last_error().decode()}")
         return out
-    if second is not None:
-        if scba is not None:
-            raise RgfError("second: the SCBA refresh takes one lesser source")
-        blk = b.nx * b.nm * b.nm
-        need = blk + b.sig_stride * (b.nE - 1)
-        sec = Lesser(_req(second.get("sigL"), "second sigL", torch.complex128, need, E.device),
-                     _req(second.get("sigL_up"), "second sigL_up", torch.complex128, need, E.device),
-                     _req(second["ndens"], "second ndens", torch.complex128, blk * b.nE, E.device))
+    if sec is not None:
         rc = lib().rgf_solve_two_lesser(ctypes.byref(p), ctypes.byref(b), ctypes.byref(sec),
                                         ctypes.c_void_p(stream.cuda_stream))
     elif scba is not None:
@@ -327,6 +325,20 @@ def solve_batched(p, E, temp, mu, Hii, H1i, sigL=None, sigR=None, out=None, max_
         rc = lib().rgf_solve_batched(ctypes.byref(p), ctypes.byref(b), ctypes.c_void_p(stream.cuda_stream))
     _check(rc)
     return out
+
+
+def _second(torch, b, second, given, dev):
+    """The second lesser source of batch b (`given`: b has Sigma tensors of its own).  Both
+    have one energy stride, so several energies take both per energy or both shared."""
+    blk = b.nx * b.nm * b.nm
+    tensors = {k: second.get(k) for k in ("sigL", "sigL_up")}
+    if any(t is not None and t.dim() == 4 for t in tensors.values()) and b.nE > 1 and not b.sig_stride:
+        if given:
+            raise RgfError("second: its Sigma is per energy (nE, nx, nm, nm), the batch's is shared")
+        b.sig_stride = blk
+    need = blk + b.sig_stride * (b.nE - 1)
+    ptr = {k: _req(t, "second " + k, torch.complex128, need, dev) for k, t in tensors.items()}
+    return Lesser(ptr["sigL"], ptr["sigL_up"], _req(second["ndens"], "second ndens", torch.complex128, blk * b.nE, dev))
 
 
 def _out_batch(torch, b, out, dev):

@@ -31,3 +31,24 @@ def test_second_source_equals_its_own_solve(nm, nE, nx):
     torch.cuda.synchronize()
     for got, ref in ((both["ndens"], one["ndens"]), (both["ldos"], one["ldos"]), (second, two["ndens"])):
         assert (got - ref).norm() <= 1e-11 * ref.norm()
+
+
+def test_second_source_alone_per_energy():
+    """The batch has no Sigma, the second source one per energy: each energy takes its own."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("no HIP device visible")
+    from liteqt_amd import configs, rgf
+    nm, nE, nx = 32, 4, 3
+    Hii, H1i = configs.random_device(nm, nx, nm)
+    H, C = rgf.to_device_blocks(Hii), rgf.to_device_blocks(H1i)
+    E = torch.tensor(np.linspace(-0.6, 0.7, nE), dtype=torch.float64, device="cuda")
+    p = rgf.params(rgf.MODE_PHYSICAL, eta_dev=1e-3)
+    sl, _, _ = configs.scattering_self_energies(nm, nx, 4, E=np.linspace(0.0, 0.4, nE), scale=1e-2)
+    sl = rgf.to_device_blocks(sl)
+    new = lambda: torch.zeros(nE, nx, nm, nm, dtype=torch.complex128, device="cuda")
+    second, own = new(), new()
+    rgf.solve_batched(p, E, (300.0, 300.0), (0.1, -0.1), H, C, out={"ndens": new()}, second={"sigL": sl, "ndens": second})
+    rgf.solve_batched(p, E, (300.0, 300.0), (0.1, -0.1), H, C, sigL=sl, out={"ndens": own})
+    torch.cuda.synchronize()
+    assert (second - own).norm() <= 1e-11 * own.norm()
