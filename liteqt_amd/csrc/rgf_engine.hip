@@ -1228,7 +1228,8 @@ static int rs_core(const rgf_params* p, const double temp[2], int nm, int nx, co
   char* base = (char*)g_stage[dev].p;
   auto D = [&](size_t o) { return (void*)(base + o); };
   hipStream_t s = nullptr;
-  HIPCHK(g_pinned[dev].ensure((size_t)nout * cslab_u * C + (has_cur ? rslab_u * C : 0) + 4096));
+  if (g_pinned[dev].ensure((size_t)nout * cslab_u * C + (has_cur ? rslab_u * C : 0) + 4096) != hipSuccess)
+    (void)hipGetLastError();  // copies without areas
   rgf::HostCopier copier(g_pinned[dev], s);
   const double2 fill = make_double2(1.0e3, 0.0);
   // (count) energies' (nm, nm, nx) complex slabs, energy e0 + i of `a`, into a padded

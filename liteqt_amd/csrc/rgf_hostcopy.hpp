@@ -27,6 +27,7 @@ struct PinnedAreas {
   hipEvent_t done[2] = {nullptr, nullptr};
   bool busy[2] = {false, false};  // a DMA of the area may be under way
   size_t bytes = 0;
+  // Areas for calls of `total` bytes; none (bytes = 0) where they cannot be allocated.
   hipError_t ensure(size_t total) {
     const size_t want = std::min(kMax, std::max(kMin, (total + 4095) / 4096 * 4096));
     if (want <= bytes) return hipSuccess;
@@ -140,12 +141,14 @@ class CopyTeam {
 };
 
 // A stream's copies through the areas: to_device / to_host queue a copy, finish completes
-// the copies to the host (those to the device complete in stream order).
+// the copies to the host (those to the device complete in stream order).  Without areas
+// (pinned memory can run out before the host's does) the copies are the runtime's own.
 class HostCopier {
  public:
   HostCopier(PinnedAreas& areas, hipStream_t s) : a_(areas), s_(s) {}
   ~HostCopier() { (void)close(); }  // after an error: the next user waits for the queued DMA
   hipError_t to_device(void* dst, const void* src, size_t bytes) {
+    if (!a_.bytes) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s_);
     for (size_t o = 0; o < bytes;) {
       if (hipError_t e = open(false)) return e;
       const size_t b = std::min(bytes - o, a_.bytes - used_);
@@ -158,6 +161,7 @@ class HostCopier {
     return hipSuccess;
   }
   hipError_t to_host(void* dst, const void* src, size_t bytes) {
+    if (!a_.bytes) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s_);
     for (size_t o = 0; o < bytes;) {
       if (hipError_t e = open(true)) return e;
       const size_t b = std::min(bytes - o, a_.bytes - used_);
@@ -170,6 +174,7 @@ class HostCopier {
     return hipSuccess;
   }
   hipError_t finish() {
+    if (!a_.bytes) return hipStreamSynchronize(s_);
     if (hipError_t e = close()) return e;
     if (hipError_t e = land(cur_ ^ 1)) return e;
     return land(cur_);
