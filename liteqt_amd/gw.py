@@ -217,22 +217,24 @@ def w_blocks(Vii, V1i, PL, PG, PR, WL=None, WG=None, WR=None, chunk=256):
         del Pr, Mii, Mlo, Mup, A, Lo, Up
         E = torch.zeros(ce, dtype=torch.float64, device=dev)
         shape = (ce, nxp, n2, n2)
+        # (the sources' temporaries are the chunk's largest: before the other arrays)
+        Sd, Su = lesser_source(pad(PL[e0:e1]))
+        Sd2, Su2 = lesser_source(pad(PG[e0:e1]))
         X = torch.empty(shape, dtype=torch.complex128, device=dev)
         Xu = torch.zeros(shape, dtype=torch.complex128, device=dev)
         Xl = torch.zeros(shape, dtype=torch.complex128, device=dev)
-        Sd, Su = lesser_source(pad(PL[e0:e1]))
-        Sd2, Su2 = lesser_source(pad(PG[e0:e1]))
         Gl, Gg = torch.empty(shape, dtype=torch.complex128, device=dev), torch.empty(shape, dtype=torch.complex128, device=dev)
         rgf.solve_batched(p, E, (300.0, 300.0), (0.0, 0.0), zsup, zsup, sigL=Sd, sigR=sig["sigR"],
                           sigR_lo=sig["sigR_lo"], sigR_up=sig["sigR_up"], sigL_up=Su,
                           out={"ndens": Gl, "ldos": X, "GRi1": Xu, "GRi1_lo": Xl},
                           second={"sigL": Sd2, "sigL_up": Su2, "ndens": Gg})
+        del Sd, Su, Sd2, Su2
         for Gn, Wout in ((Gl, WL), (Gg, WG)):
             Gt = tm(Gn)
             Wd = torch.stack([Gt[..., :nm, :nm], Gt[..., nm:, nm:]], dim=2).reshape(ce, nx2, nm, nm)
             Wout[e0:e1] = tm(Wd[:, :nx])
             del Gt, Wd
-        del Sd, Su, Sd2, Su2, Gl, Gg
+        del Gl, Gg, Gn
         Xt, Xut, Xlt = tm(X), tm(Xu), tm(Xl)
         Wr = torch.zeros((ce, nx2, nm, nm), dtype=torch.complex128, device=dev)
         Vu = H_(V1)
