@@ -250,17 +250,21 @@ void rgf_graph_destroy(rgf_graph g);
  * max_slots and the off-diagonal sigma fields must be 0/NULL).  All
  * (device, energy) pairs form one work list ordered by predicted cost,
  * longest first; the workgroups of one launch take items from it
- * dynamically, each with the tile variant of its device's block size.
+ * dynamically, each with the tile variant of its device's block size.  With at
+ * most two pairs per compute unit, and where that is predicted to be faster, the
+ * pairs are laid out on groups of workgroups by their costs instead.
  * autotune != 0: before the first solve at a block size, time its candidate
  * tile variants on the device (results kept per process) and use the fastest
- * and its measured cost for the ordering.  The number of workgroups is
+ * and its measured cost for the ordering (groups do not take the variants: nothing
+ * is timed for them).  The number of workgroups is
  * bounded by the CU count and by free HBM for the largest device's stored
- * blocks.  tile_T (optional, ndev ints) receives the tile parameter chosen
- * per device; rep (optional) the launch shape.  Synchronises the device
+ * blocks.  tile_T (optional, ndev ints) receives the tile parameter that runs
+ * per device (T: 32 T square, 4: 128 x 64; where a device's energies run in groups
+ * of several sizes, one of them); rep (optional) the launch shape.  Synchronises the device
  * before it starts (its descriptor buffer is reused), then runs
  * asynchronously on `stream`.  No counterpart in the reference. */
 typedef struct rgf_multi_report {
-  int slots;          /* workgroups of the persistent launch */
+  int slots;          /* workgroups of the launch */
   int tuned;          /* block sizes timed by the autotuner in this call */
   long long items;    /* (device, energy) pairs */
   long long ws_bytes; /* device workspace of the launch */

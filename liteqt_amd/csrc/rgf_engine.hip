@@ -12,6 +12,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -980,12 +981,35 @@ int rgf_solve_devices(const rgf_params* p, const rgf_batch* devs, int ndev, int 
   WsTurn turn;
   if (int rc = turn.begin(dev, s)) return rc;
   Buf& ws = g_ws[dev];
+  Buf& desc = g_multi_desc[dev];
   MultiPlan pl;
-  if (int rc = multi_plan(p, devs, ndev, autotune, 0, s, &pl, ws.bytes)) return rc;
-  if (tile_T)
+  if (int rc = multi_plan(p, devs, ndev, 0, 0, s, &pl, ws.bytes)) return rc;
+  // few items for the compute units: the longer ones get groups of workgroups, the shorter
+  // ones share a workgroup (with more items the shared counter balances them)
+  rgf::MultiGroupPlan gp;
+  bool groups = false;
+  if (pl.slots == (int)std::min<size_t>(pl.items.size(), (size_t)pl.cus) &&
+      pl.items.size() <= (size_t)rgf::kMultiGroupItems * pl.cus) {
+    std::vector<int> in, inx;
+    for (const int2& it : pl.items) {
+      in.push_back(pl.jobs[it.x].n);
+      inx.push_back(pl.jobs[it.x].nx);
+    }
+    groups = rgf::multi_group_plan(in, inx, pl.cus, &gp);
+  }
+  // the tile variants, which a launch of groups does not take, are only timed for the others
+  if (autotune && !groups)
+    if (int rc = multi_plan(p, devs, ndev, autotune, 0, s, &pl, ws.bytes)) return rc;
+  if (tile_T) {
     for (int j = 0; j < ndev; ++j) tile_T[j] = mv_T(pl.mv[j]);
+    for (size_t g = 0; groups && g < gp.sizes.size(); ++g)
+      for (int i = gp.first[g]; i < gp.first[g + 1]; ++i) {
+        const int j = pl.items[(size_t)gp.order[(size_t)i]].x;
+        tile_T[j] = rgf::group_tile_T(pl.jobs[(size_t)j].n, gp.sizes[g]);
+      }
+  }
   if (rep) {
-    rep->slots = pl.slots;
+    rep->slots = groups ? std::accumulate(gp.sizes.begin(), gp.sizes.end(), 0) : pl.slots;
     rep->items = (long long)pl.items.size();
     rep->ws_bytes = pl.ws_slot * 16LL * pl.slots;
     rep->tuned = pl.ntuned;
@@ -995,19 +1019,7 @@ int rgf_solve_devices(const rgf_params* p, const rgf_batch* devs, int ndev, int 
     ws.release();
     if (int rc = ws.ensure((size_t)(pl.ws_slot * 16LL * pl.slots))) return rc;
   }
-  Buf& desc = g_multi_desc[dev];
-  if (pl.slots == (int)std::min<size_t>(pl.items.size(), (size_t)pl.cus) &&
-      pl.items.size() <= (size_t)rgf::kMultiGroupItems * pl.cus) {
-    // few items for the compute units: the longer ones get groups of workgroups, the
-    // shorter ones share a workgroup (with more items the shared counter balances them)
-    std::vector<int> in, inx;
-    for (const int2& it : pl.items) {
-      in.push_back(pl.jobs[it.x].n);
-      inx.push_back(pl.jobs[it.x].nx);
-    }
-    rgf::MultiGroupPlan gp;
-    if (rgf::multi_group_plan(in, inx, pl.cus, &gp)) return multi_group_launch(pl, gp, &desc, ws.p, s);
-  }
+  if (groups) return multi_group_launch(pl, gp, &desc, ws.p, s);
   const MultiDesc L = multi_layout(ndev, (long long)pl.items.size());
   if (int rc = desc.ensure(L.bytes)) return rc;
   if (int rc = multi_upload(pl.jobs, pl.mv, pl.items, desc.p)) return rc;

@@ -45,7 +45,6 @@
 namespace rgf {
 
 constexpr int kGrp = 64;          // variant code of the group kernels
-constexpr int kGrpTile = 32;      // output tile of a group GEMM: 4 waves of one 16 x 16 MFMA tile
 constexpr int kGrpK = 32;         // its K panel
 constexpr int kJoinTicks = 20000; // 200 us of the 100 MHz clock
 constexpr int kMaxTiles = (256 / kGrpTile) * (256 / kGrpTile);
@@ -183,16 +182,6 @@ template <>
 struct GemmLds<kGrp> {
   static constexpr int DOUBLES = 2 * GrpGemm::STAGE > GemmLds<4>::DOUBLES ? 2 * GrpGemm::STAGE : GemmLds<4>::DOUBLES;
 };
-
-// Where the block is a multiple of 128 and the ranks are few, the 128 x 64 tiles of the
-// one-workgroup GEMM are the better split: they read a third of the operands' panels and
-// run at 80% of the MFMA rate against 54%, so one of them takes as long as 6.5 of the
-// small ones (42 and 6.5 us at K = 128), not 8.
-__device__ __forceinline__ bool large_tiles(int n, int size) {
-  if (n % 128 != 0) return false;
-  const int small = (n / kGrpTile) * (n / kGrpTile), large = small / 8;
-  return 13 * ((large + size - 1) / size) < 2 * ((small + size - 1) / size);
-}
 
 // The parts of a sum, one per tile (at most a wave's lanes), added in the order of the tiles.
 __device__ __forceinline__ double tile_sum(const double* part, int ntiles) {

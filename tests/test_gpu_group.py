@@ -181,3 +181,19 @@ def _decimation_sum(nm, nE):
 def test_decimation_sum_does_not_depend_on_the_group(nm, many):
     one, sums = _decimation_sum(nm, 1), _decimation_sum(nm, many)
     assert (sums == one[0]).all(), (one[:1].view(np.float64), sums.view(np.float64))
+
+
+# one item takes a group of up to 16 workgroups (32 x 32 tiles), 128 of them one of two each
+# (128 x 64), 257 energies of 32 orbitals the work list with its variants
+@pytest.mark.parametrize("nm,nE,groups,tile", [(128, 1, True, 1), (128, 128, True, 4), (32, 257, False, 1)])
+def test_devices_report_what_runs(nm, nE, groups, tile):
+    torch, configs, rgf, H, C, E = _device(nm, 4, nE, 10 + nm)
+    dev = {"E": E, "temp": (300.0, 300.0), "mu": (0.1, -0.1), "Hii": H, "H1i": C,
+           "out": {"tr": torch.zeros(nE, dtype=torch.float64, device="cuda")}}
+    tiles, rep = rgf.solve_devices(rgf.params(rgf.MODE_PHYSICAL, eta_dev=1e-3), [dev], autotune=groups)
+    torch.cuda.synchronize()
+    assert tiles == [tile] and rep["items"] == nE
+    if groups:
+        assert rep["slots"] > nE and rep["tuned"] == 0
+    else:
+        assert rep["slots"] <= nE
