@@ -490,10 +490,11 @@ int solve_impl(const rgf_params* p, const rgf_batch* b, const rgf_scba* scba, vo
   std::lock_guard<std::mutex> lk(g_ws_mu);
   WsTurn turn;
   if (int rc = turn.begin(pr.dev, s)) return rc;
-  char* ctl = turn.capturing ? nullptr : group_ctl(pr.dev, pr.cus);
+  // (the group kernels have no overlap form)
+  char* ctl = turn.capturing || b->Sii ? nullptr : group_ctl(pr.dev, pr.cus);
   Split sp = group_split(b->nm, b->nE, pr.cus, pr.slots, b->max_slots, ctl);
   const long long pair_extra = (long long)rgf::kPairExtra * b->nm * b->nm;
-  if (ctl && !od && !b->Sii && b->max_slots <= 0 && rgf::pair_plan(b->nm, b->nE, pr.cus, &sp.g)) {
+  if (ctl && !od && b->max_slots <= 0 && rgf::pair_plan(b->nm, b->nE, pr.cus, &sp.g)) {
     sp.g.ctl = ctl;
     sp.tail = sp.need = b->nE;
     pr.a.ws_slot += pair_extra;
