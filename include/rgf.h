@@ -134,8 +134,9 @@ int rgf_rs_energies(const rgf_params *p, const double temp[2], int nm, int nx,
  * blocks, real for cur).  dens_n / dens_p (nx per energy) receive
  * Im Tr G^<_ll and -Im Tr G^>_ll, the integrands of the electron and hole
  * densities of src/green_rgf.f90:3919-3945.  max_slots > 0 caps the number of
- * energies in flight (each holds 2*nx stored left-connected blocks in HBM);
- * 0 lets the engine size it from free memory and the CU count. */
+ * energies in flight (each holds 2*nx stored left-connected blocks in HBM) and
+ * keeps one workgroup per energy; 0 lets the engine size it from free memory and
+ * the CU count, and give an energy several workgroups where there are few. */
 typedef struct rgf_batch {
   int nm, nx, nE;
   int max_slots;
@@ -231,7 +232,8 @@ int rgf_solve_two_lesser(const rgf_params *p, const rgf_batch *b, const rgf_less
 
 /* HIP-graph form of rgf_solve_batched / rgf_scba_step: rgf_graph_create
  * captures one launch on `stream` (a created stream, not NULL) into an
- * executable graph that owns its workspace; rgf_graph_launch replays it
+ * executable graph that owns its workspace (one workgroup per energy, however few
+ * there are); rgf_graph_launch replays it
  * `replays` times on `stream` (with scba given, each replay is one SCBA
  * iteration on the same device arrays).  The graph keeps the pointers of b.
  * No counterpart in the reference; for drivers that repeat the solve on
