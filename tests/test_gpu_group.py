@@ -197,3 +197,49 @@ def test_devices_report_what_runs(nm, nE, groups, tile):
         assert rep["slots"] > nE and rep["tuned"] == 0
     else:
         assert rep["slots"] <= nE
+
+
+# full rounds of one energy per workgroup, then groups on the same slots (256 + 4 energies), and
+# 64 orbitals, where every rank sweeps the whole block
+@pytest.mark.parametrize("nm,nE", [(96, 260), (64, 9)])
+def test_group_adjoint_behind_full_rounds(nm, nE):
+    test_group_adjoint_equals_one_workgroup(nm, nE, 0)
+
+
+@pytest.mark.parametrize("nm,nE", [(96, 260), (64, 9)])
+def test_group_offdiag_refresh_behind_full_rounds(nm, nE):
+    test_group_offdiag_refresh_equals_one_workgroup(nm, nE)
+
+
+# (the W solve's one-workgroup form: as the first of 256 energies)
+@pytest.mark.parametrize("nm,nE", [(96, 260), (64, 3)])
+def test_group_w_behind_full_rounds(nm, nE):
+    torch, configs, rgf = _env()
+    nx = 3
+    g = torch.Generator(device="cuda").manual_seed(nm)
+    cn = lambda *s: torch.randn(*s, dtype=torch.complex128, device="cuda", generator=g) / nm ** 0.5
+    V, V1, P = cn(nx, nm, nm), cn(nx, nm, nm) * 0.3, [cn(nE, nx, nm, nm) * 0.2 for _ in range(3)]
+    got = rgf.w_solve_batched(V, V1, *P)
+    tail = nE % 256
+    lone = rgf.w_solve_batched(V, V1, *[torch.cat([x[nE - tail:], x[:1].expand(256 - tail, -1, -1, -1)]).contiguous() for x in P])
+    rest = rgf.w_solve_batched(V, V1, *[x[:256].contiguous() for x in P]) if nE > 256 else None
+    torch.cuda.synchronize()
+    for k in ("WL", "WG", "WR"):
+        _close(got[k][nE - tail:], lone[k][:tail], k)
+        if rest:
+            assert torch.equal(got[k][:256], rest[k]), k
+    assert int(got["info"].sum()) == 0
+
+
+def test_group_singular_slab_at_64_orbitals():
+    nm, nx, nE = 64, 3, 2
+    torch, configs, rgf, H, C, E = _device(nm, nx, nE, 40 + nm)
+    H, C, E = torch.zeros_like(H), torch.zeros_like(C), torch.zeros_like(E)
+    p = rgf.params(rgf.MODE_PHYSICAL, eta_dev=0.0)
+    for slots in (0, nE):
+        out = {"ldos": torch.full((nE, nx, nm, nm), 7.0, dtype=torch.complex128, device="cuda"),
+               "info": torch.zeros(nE, 4, dtype=torch.int32, device="cuda")}
+        rgf.solve_batched(p, E, (300.0, 300.0), (0.0, 0.0), H, C, out=out, max_slots=slots)
+        torch.cuda.synchronize()
+        assert int(out["info"][:, 3].min()) == int(out["info"][:, 3].max()) == nx
+        assert float(out["ldos"].abs().max()) == 0.0
