@@ -970,7 +970,10 @@ __device__ __forceinline__ int gj_sweep(double2 (&a)[RT][CT], int nrow, unsigned
           prow_mine[c] = v;
         }
       }
+      // (the fences emit nothing: they keep the compiler from moving the reads up)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
         const dvec2 v = prow_mine[c];
