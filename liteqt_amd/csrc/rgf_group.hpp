@@ -193,23 +193,38 @@ __device__ __forceinline__ double tile_sum(const double* part, int ntiles) {
   return s;
 }
 
+__device__ __forceinline__ double group_abs(double2 v) { return sqrt(fma(v.y, v.y, v.x * v.x)); }
+
+// Those parts from the 128 x 64 tiles: a wave's 64 x 32 part is two of the sum's tiles, each
+// added as grp_gemm's four waves add it.
+struct GroupSums {
+  double* parts;
+  int nt;
+  double sum = 0.0, part = 0.0;  // of the 16 x 16 tile at work; lane b: of tile b
+  __device__ __forceinline__ void add(double2 v) { sum += group_abs(v); }
+  __device__ __forceinline__ void tile(int b) {
+    sum = wave_sum(sum);
+    part = (int)(threadIdx.x & 63) == b ? sum : part;
+    sum = 0.0;
+  }
+  __device__ __forceinline__ void done(int row, int col) {
+    static_assert(Cfg<4>::TA == 4 && Cfg<4>::TB == 2, "two 32 x 32 tiles per wave");
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const double s = ((lane_f64(part, 4 * a) + lane_f64(part, 4 * a + 2)) + lane_f64(part, 4 * a + 1)) +
+                       lane_f64(part, 4 * a + 3);
+      if ((threadIdx.x & 63) == 0) agent_store(parts + row / kGrpTile + a + col / kGrpTile * nt, s);
+    }
+  }
+};
+
 template <int OPA, int OPB, int CRM>
 __device__ __noinline__ double grp_gemm_large(GroupN n_, const double2* __restrict__ A, const double2* __restrict__ B,
                                               void* Cout, Epi ep, ldsd* lds) {
   const int rank = group_rank(n_), size = group_size(n_), parity = group_parity(n_);
   GroupCtl* ctl = uni(group_ctx()->ctl);
   const int nt = uni((int)n_) / kGrpTile;
-  // a wave's 64 x 32 part is two of the sum's tiles; each is added as grp_gemm's waves add it
-  auto sums = [&](int row, int col, double part) {
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const double s = ((lane_f64(part, 4 * a) + lane_f64(part, 4 * a + 2)) + lane_f64(part, 4 * a + 1)) +
-                       lane_f64(part, 4 * a + 3);
-      if ((threadIdx.x & 63) == 0) agent_store(&ctl->part[parity][row / kGrpTile + a + col / kGrpTile * nt], s);
-    }
-  };
-  static_assert(Cfg<4>::TA == 4 && Cfg<4>::TB == 2, "two 32 x 32 tiles per wave");
-  gemm_tiles<4, OPA, OPB, CRM>((int)n_, A, B, Cout, ep, lds, rank, size, sums);
+  gemm_tiles<4, OPA, OPB, CRM>((int)n_, A, B, Cout, ep, lds, rank, size, GroupSums{ctl->part[parity], nt});
   group_barrier();
   return uni(ep.abs_sum) ? tile_sum(ctl->part[parity], nt * nt) : 0.0;
 }
@@ -323,7 +338,7 @@ __device__ __noinline__ double grp_gemm(GroupN n_, const double2* __restrict__ A
       if (ep.D1) v = cadd(v, cmul(ep.s1, d1[r]));
       if (ep.D2) v = cadd(v, cmul(ep.s2, d2[r]));
       if (ep.D3) v = cadd(v, cmul(ep.s3, cconj(d3[r])));
-      if (ep.abs_sum) asum += cabs_plain(v);
+      if (ep.abs_sum) asum += group_abs(v);
       const uint32_t u = (uint32_t)(CRM ? j + i * n : i + j * n);
       if (ep.real_out)
         stgb_re((double*)Cout, 8u * u, v.x);
