@@ -282,8 +282,9 @@ int rgf_graph_create_devices(const rgf_params *p, const rgf_batch *devs, int nde
                              void *stream, rgf_graph *out);
 
 /* Bytes of device workspace rgf_solve_batched uses for `slots` energies in
- * flight at block size nm and nx slabs.  (An energy solved by several workgroups,
- * where a call has few, takes 6 KB besides, and at nm = 32 11 blocks.) */
+ * flight at block size nm and nx slabs.  (An energy solved by two workgroups, where a
+ * call has few of nm = 32, takes 11 blocks more; the control words of groups of
+ * workgroups are 6 KB per compute unit besides.) */
 long long rgf_workspace_bytes(int nm, int nx, int slots);
 
 /* Adjoint (reverse-mode) RGF of the physical-mode device with the scattering
